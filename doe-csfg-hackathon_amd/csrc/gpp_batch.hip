@@ -65,17 +65,21 @@ __global__ __launch_bounds__(kRedThreads) void k_batch_achstemp(const BInst *__r
     }
 }
 
-template <int WJN, int WIN>
-__global__ __launch_bounds__(64 * WJN * WIN, WJN * WIN >= 4 ? 8 / (WJN * WIN) : 2) void k_batch_gram(const BInst *__restrict__ insts,
-                                                               const GramItem *__restrict__ items, int nitems)
+// Tiles of gram_ring_tile; the last G' tile of an instance runs as many
+// sub-tiles per wave as its columns need.
+template <class C>
+__global__ __launch_bounds__(C::NT) __attribute__((amdgpu_waves_per_eu(C::OCC))) void k_batch_gram(
+    const BInst *__restrict__ insts, const GramItem *__restrict__ items, int nitems)
 {
-    typedef GramCfg<WJN, WIN> C;
-    __shared__ cplx sB[2][C::KS][C::TJ];
-    __shared__ cplx sA[2][C::KS][C::TI];
+    __shared__ cplx lds[C::LDS];
     for (int w = blockIdx.x; w < nitems; w += gridDim.x) {
         const GramItem it = items[w];
         const BInst &b = insts[it.inst];
-        gram_f64_tile<WJN, WIN>(b.bg, b.aqsn, b.ngpown, b.ncouls, b.nv, b.nb, it.j0, it.i0, sB, sA, b.mu);
+        if (C::SJ == 2 && b.ngpown - it.j0 <= 16 * C::WJN)
+            gram_ring_tile<C, 1>(b.bg, b.aqsn, b.ngpown, b.ncouls, b.nv, b.nb, it.j0, it.i0, lds, true, b.mu);
+        else
+            gram_ring_tile<C, C::SJ>(b.bg, b.aqsn, b.ngpown, b.ncouls, b.nv, b.nb, it.j0, it.i0, lds, true, b.mu);
+        __syncthreads();  // every wave is done with lds
     }
 }
 
@@ -181,8 +185,9 @@ __global__ __launch_bounds__(kRedThreads) void k_batch_final(const BInst *__rest
 
 __host__ inline size_t align256(size_t x) { return (x + 255) & ~(size_t)255; }
 
-constexpr int gram_tj(int tile) { return tile == 0 || tile == 2 ? 128 : 64; }
-constexpr int gram_ti(int tile) { return tile == 0 || tile == 1 ? 128 : 64; }
+// Gram tiles of a batch: 0 and 1 64 x 128, 2 128 x 64, 3 64 x 64.
+constexpr int gram_tj(int tile) { return tile == 2 ? GramLt::TJ : tile == 3 ? GramM::TJ : GramL::TJ; }
+constexpr int gram_ti(int tile) { return tile == 2 ? GramLt::TI : tile == 3 ? GramM::TI : GramL::TI; }
 
 }  // namespace
 
@@ -458,10 +463,9 @@ hipError_t launch_batch(const BatchPlan &pl, void *work, int persistent_blocks, 
         const int ng = (int)pl.gram_items.size();
         const dim3 grid(std::max(1, std::min(G, ng)));
         switch (pl.kind.tile) {
-        case 0: hipLaunchKernelGGL((k_batch_gram<2, 4>), grid, dim3(512), 0, s, insts, gi, ng); break;
-        case 1: hipLaunchKernelGGL((k_batch_gram<1, 4>), grid, dim3(256), 0, s, insts, gi, ng); break;
-        case 2: hipLaunchKernelGGL((k_batch_gram<2, 2>), grid, dim3(256), 0, s, insts, gi, ng); break;
-        default: hipLaunchKernelGGL((k_batch_gram<1, 2>), grid, dim3(128), 0, s, insts, gi, ng); break;
+        case 2: hipLaunchKernelGGL((k_batch_gram<GramLt>), grid, dim3(GramLt::NT), 0, s, insts, gi, ng); break;
+        case 3: hipLaunchKernelGGL((k_batch_gram<GramM>), grid, dim3(GramM::NT), 0, s, insts, gi, ng); break;
+        default: hipLaunchKernelGGL((k_batch_gram<GramL>), grid, dim3(GramL::NT), 0, s, insts, gi, ng); break;
         }
     }
     if (which & 4) {

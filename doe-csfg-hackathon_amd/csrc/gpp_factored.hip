@@ -21,6 +21,7 @@
 //                      counts k_acht_occ streams the masked P2 (stage 3
 //                      writes the branch mask) against the occupied aqsn rows
 //   6. k_acht_final    fixed-order sum of the per-band partials.
+#include <math.h>
 #include <string.h>
 
 #include <algorithm>
@@ -60,14 +61,18 @@ AchtSplit acht_split(const DevProblem &p)
 
 // The fused Gram + pole reduce (k_gram_pole) serves at most three
 // frequencies, none negative, at most kFuseNv occupied bands, without
-// acht_n1_loc, on the 128 x 128 FP64 tile.
-typedef GramCfg<2, 4> FuseCfg;
-
+// acht_n1_loc, on its own 128 x 128 FP64 tile.
 bool fused_reduce(const DevProblem &p, const GramKind &k)
 {
     return k.fuse && k.ozaki_slices == 0 && k.tile == 0 && !k.acht && p.nfreq <= 3 && !p.wx_neg &&
            p.nv <= kFuseNv;
 }
+
+// Mu is stored past the caches when it is larger than them (256 MB): it is
+// written once and read back once, by the pole reduce (C1, 859 MB: reduce
+// 0.486-0.502 -> 0.469 ms); a smaller one is read back from them.
+bool mu_streams(const DevProblem &p) { return sizeof(cplx) * (size_t)p.ngpown * p.ncouls > ((size_t)256 << 20); }
+constexpr double kGramCus = 256;  // compute units of an MI355X
 
 struct FactLayout {
     size_t bg, m, col_ach, col_asx, col2_ach, col2_asx, part_achs, p2, br1, acht_part, acht_occ, total;
@@ -109,34 +114,82 @@ FactLayout fact_layout(const DevProblem &p, const GramKind &k)
 
 // 1-D grid over the ceil(ngpown/TJ) x ceil(ncouls/TI) tiles, G' tiles
 // fastest in tile order and tiles spread over the XCDs by xcd_tile, so the
-// blocks sharing one aqsn tile run on one XCD.  Every tile runs two waves per
-// SIMD (at most 256 registers per lane).
-template <int WJN, int WIN>
-__global__ __launch_bounds__(64 * WJN * WIN, WJN * WIN >= 4 ? 8 / (WJN * WIN) : 2) void k_gram_f64(const cplx *__restrict__ bg,
-                                                                    const cplx *__restrict__ aqsn, int ngpown,
-                                                                    int ncouls, int k_begin, int k_end,
-                                                                    cplx *__restrict__ mout)
+// blocks sharing one aqsn tile run on one XCD.  The last G' tile runs SJR <= SJ
+// sub-tiles per wave, as many as its columns need (the launcher picks SJR).
+template <class C, int SJR>
+__global__ __launch_bounds__(C::NT) __attribute__((amdgpu_waves_per_eu(C::OCC))) void k_gram_f64(
+    const cplx *__restrict__ bg, const cplx *__restrict__ aqsn, int ngpown, int ncouls, int k_begin, int k_end,
+    bool nts, cplx *__restrict__ mout)
 {
-    typedef GramCfg<WJN, WIN> C;
-    __shared__ cplx sB[2][C::KS][C::TJ];
-    __shared__ cplx sA[2][C::KS][C::TI];
-    const int nj = (ngpown + C::TJ - 1) / C::TJ;
-    const int ni = (ncouls + C::TI - 1) / C::TI;
+    __shared__ cplx lds[C::LDS];
+    const int nj = (ngpown + C::TJ - 1) / C::TJ, ni = (ncouls + C::TI - 1) / C::TI;
+    if constexpr (SJR == C::SJ) {
+        const int t = xcd_tile(blockIdx.x, nj * ni);
+        gram_ring_tile<C, C::SJ>(bg, aqsn, ngpown, ncouls, k_begin, k_end, (t % nj) * C::TJ, (t / nj) * C::TI, lds,
+                                 nts, mout);
+    } else {
+        // the shorter tiles come last, so that they fill the last round
+        const int full = (nj - 1) * ni, b = blockIdx.x;
+        if (b < full) {
+            const int t = xcd_tile(b, full);
+            gram_ring_tile<C, C::SJ>(bg, aqsn, ngpown, ncouls, k_begin, k_end, (t % (nj - 1)) * C::TJ,
+                                     (t / (nj - 1)) * C::TI, lds, nts, mout);
+        } else {
+            const int t = xcd_tile(b - full, ni);
+            gram_ring_tile<C, SJR>(bg, aqsn, ngpown, ncouls, k_begin, k_end, (nj - 1) * C::TJ, t * C::TI, lds, nts,
+                                   mout);
+        }
+    }
+}
+
+// 16 x 16 tiles, three waves each (gram_small_product); same tile order.
+__global__ __launch_bounds__(kSmThreads) void k_gram_small(const cplx *__restrict__ bg, const cplx *__restrict__ aqsn,
+                                                           int ngpown, int ncouls, int k_begin, int k_end,
+                                                           cplx *__restrict__ mout)
+{
+    // one array (with a second one the compiler waits for every outstanding
+    // load before each fragment read): the stages, then P2 and P3
+    __shared__ cplx lds[kSmBuf * kSmStage];
+    auto *prod = reinterpret_cast<double(*)[4][kWave]>(lds);
+    const int nj = (ngpown + 15) / 16, ni = (ncouls + 15) / 16;
     const int t = xcd_tile(blockIdx.x, nj * ni);
-    gram_f64_tile<WJN, WIN>(bg, aqsn, ngpown, ncouls, k_begin, k_end, (t % nj) * C::TJ, (t / nj) * C::TI, sB, sA,
-                            mout);
+    const int j0 = (t % nj) * 16, i0 = (t / nj) * 16;
+    const int lane = threadIdx.x % kWave;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+    v4d p;
+    if (wave == 0)
+        p = gram_small_product<0>(bg, aqsn, ngpown, ncouls, k_begin, k_end, j0, i0, lds);
+    else if (wave == 1)
+        p = gram_small_product<1>(bg, aqsn, ngpown, ncouls, k_begin, k_end, j0, i0, lds);
+    else
+        p = gram_small_product<2>(bg, aqsn, ngpown, ncouls, k_begin, k_end, j0, i0, lds);
+    __syncthreads();  // every wave is done with the stages
+    if (wave > 0) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) prod[wave - 1][r][lane] = p[r];
+    }
+    __syncthreads();
+    if (wave == 0) {
+        const int ig = i0 + lane % 16;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const int j = j0 + 4 * r + lane / 16;
+            const double p2 = prod[0][r][lane], p3 = prod[1][r][lane];
+            if (j < ngpown && ig < ncouls) mout[(size_t)j * ncouls + ig] = cplx{p[r] + p2, (p3 - p[r]) + p2};
+        }
+    }
 }
 
 // Stages 2 and 3 fused (at most three frequencies, none negative,
 // acht_n1_loc not requested): the Gram tile of k_gram_f64 in the transposed
 // orientation, then the pole terms of its elements summed per column in the
-// epilogue (gram_pole_epilogue), so Mu never reaches HBM.  Same grid and tile
-// order as k_gram_f64; col_ach/col_asx get one sum per (column, G-vector
+// epilogue (gram_pole_epilogue), so Mu never reaches HBM.  Same tile order as
+// k_gram_f64; col_ach/col_asx get one sum per (column, G-vector
 // tile, frequency).
 template <int F>
 __global__ __launch_bounds__(512, 1) void k_gram_pole(PoleTileArgs a)
 {
-    typedef GramCfg<2, 4> C;
+    typedef FuseCfg C;
     __shared__ cplx lds[FuseLds<F>::kLds];
     auto *sB = reinterpret_cast<cplx(*)[C::KS][C::TJ]>(lds);
     auto *sA = reinterpret_cast<cplx(*)[C::KS][C::TI]>(lds + 2 * C::KS * C::TJ);
@@ -145,7 +198,7 @@ __global__ __launch_bounds__(512, 1) void k_gram_pole(PoleTileArgs a)
     const int t = xcd_tile(blockIdx.x, nj * ni);
     const int j0 = (t % nj) * C::TJ, itile = t / nj, i0 = itile * C::TI;
     v4d acc1[4][2], acc2[4][2], acc3[4][2];
-    gram_f64_acc<2, 4, true>(a.bg, a.aqsn, a.ngpown, a.ncouls, a.nv, a.nb, j0, i0, sB, sA, acc1, acc2, acc3);
+    gram_f64_acc(a.bg, a.aqsn, a.ngpown, a.ncouls, a.nv, a.nb, j0, i0, sB, sA, acc1, acc2, acc3);
     gram_pole_epilogue<F>(a, j0, i0, itile, acc1, acc2, acc3, lds);
 }
 
@@ -266,13 +319,18 @@ __global__ __launch_bounds__(256) void k_acht_final(const cplx *__restrict__ par
     }
 }
 
-template <int WJN, int WIN>
-void launch_gram_cfg(const DevProblem &p, const cplx *bg, cplx *mu, hipStream_t s)
+template <class C>
+void launch_gram_ring(const DevProblem &p, const cplx *bg, cplx *mu, hipStream_t s)
 {
-    typedef GramCfg<WJN, WIN> C;
     const unsigned tiles = (unsigned)((p.ngpown + C::TJ - 1) / C::TJ) * (unsigned)((p.ncouls + C::TI - 1) / C::TI);
-    hipLaunchKernelGGL((k_gram_f64<WJN, WIN>), dim3(tiles), dim3(C::NT), 0, s, bg, p.aqsn, p.ngpown, p.ncouls, p.nv,
-                       p.nb, mu);
+    const bool nts = mu_streams(p);
+    const int rem = p.ngpown % C::TJ;
+    if (C::SJ == 2 && rem > 0 && rem <= 16 * C::WJN)
+        hipLaunchKernelGGL((k_gram_f64<C, 1>), dim3(tiles), dim3(C::NT), 0, s, bg, p.aqsn, p.ngpown, p.ncouls, p.nv,
+                           p.nb, nts, mu);
+    else
+        hipLaunchKernelGGL((k_gram_f64<C, C::SJ>), dim3(tiles), dim3(C::NT), 0, s, bg, p.aqsn, p.ngpown, p.ncouls,
+                           p.nv, p.nb, nts, mu);
 }
 
 // P2: also store the pole factor of frequency acht_iw and either sum the
@@ -328,14 +386,65 @@ size_t factored_workspace_bytes(const DevProblem &p, GramKind kind)
     return n;
 }
 
+// The Gram tile of a problem by size (GPP_OPT_GRAM_TILE 0): the least
+// estimated time, the sub-tiles a CU works through (its rounds of whole tiles;
+// the shorter last-row tiles fill the last round as far as they fit) times the
+// time per 16 x 16 sub-tile and k-step of 4 bands.  A CU with one block runs
+// its MFMAs with fewer waves beside them than one with two.  The times are
+// fitted to 17 shapes from 24/2/1000/50 to 1536/8/32768/1638 (us measured /
+// estimated: 512/2/4096/409 64 x 64 102 / 101, 128 x 64 111 / 106, 32 x 64
+// 114 / 115, 16 x 16 154 / 170; 512/2/32768/205 64 x 128 347 / 340, 64 x 64
+// 358 / 354; 512/2/800/40 16 x 16 9.6 / 9.7, 32 x 64 35 / 38).  Larger tiles
+// re-read less and turn stages over less often; smaller ones leave fewer CUs
+// idle, and the 16 x 16 tile has the shortest chain of MFMAs per wave.
+enum GramTile { kTileL = 0, kTileLt, kTileM, kTileS, kTileX };
+int gram_tile_for(const DevProblem &p)
+{
+    struct Kind {
+        int tile, tj, ti, short_j;  // short_j: rows of a short last tile (0: none)
+        double one, many;           // us per sub-tile and k-step: one block per CU, more
+    };
+    static const Kind kinds[] = {{kTileLt, GramLt::TJ, GramLt::TI, GramLt::TJ / 2, 0.0258, 0.0235},
+                                 {kTileL, GramL::TJ, GramL::TI, GramL::TJ / 2, 0.0258, 0.0237},
+                                 {kTileM, GramM::TJ, GramM::TI, GramM::TJ / 2, 0.0287, 0.0247},
+                                 {kTileS, GramS::TJ, GramS::TI, 0, 0.0344, 0.0273},
+                                 {kTileX, 16, 16, 0, 0.0547, 0.0469}};
+    const double ksteps = (p.nb - p.nv + 3) / 4;
+    double best = 1e300;
+    int tile = kTileL;
+    for (const Kind &k : kinds) {
+        const int rem = p.ngpown % k.tj;
+        const bool cut = rem > 0 && rem <= k.short_j;
+        const double ni = (p.ncouls + k.ti - 1) / k.ti, sub = k.tj / 16 * (k.ti / 16);
+        const double whole = ni * ((p.ngpown + k.tj - 1) / k.tj - (cut ? 1 : 0));
+        double rounds = ceil(whole / kGramCus);
+        if (cut) {  // two short tiles take the time of a whole one
+            const double over = ni / 2 - (rounds * kGramCus - whole);
+            if (over > 0) rounds += ceil(2 * over / kGramCus) / 2;
+        }
+        double us = rounds * sub * ksteps * (rounds <= 1 ? k.one : k.many);
+        if (k.tile == kTileX) us += 1.2 * ceil(rounds / 2);  // the first loads of its ring, two blocks at a time
+        if (us < best) best = us, tile = k.tile;
+    }
+    return tile;
+}
+
 hipError_t launch_gram_f64(const DevProblem &p, int tile, const cplx *bg, cplx *mu, hipStream_t s)
 {
-    switch (tile) {
-    case 0: launch_gram_cfg<2, 4>(p, bg, mu, s); break;  // 128 x 128, 8 waves
-    case 1: launch_gram_cfg<1, 4>(p, bg, mu, s); break;  // 64 x 128, 4 waves
-    case 2: launch_gram_cfg<2, 2>(p, bg, mu, s); break;  // 128 x 64, 4 waves
-    case 3: launch_gram_cfg<1, 2>(p, bg, mu, s); break;  // 64 x 64, 2 waves
-    default: return hipErrorInvalidValue;
+    // GPP_OPT_GRAM_TILE: 0 by size, then the ring tiles
+    static const int kinds[kGramTiles] = {-1, kTileL, kTileLt, kTileM};
+    if (tile < 0 || tile >= kGramTiles) return hipErrorInvalidValue;
+    switch (tile == 0 ? gram_tile_for(p) : kinds[tile]) {
+    case kTileL: launch_gram_ring<GramL>(p, bg, mu, s); break;
+    case kTileLt: launch_gram_ring<GramLt>(p, bg, mu, s); break;
+    case kTileM: launch_gram_ring<GramM>(p, bg, mu, s); break;
+    case kTileS: launch_gram_ring<GramS>(p, bg, mu, s); break;
+    default: {
+        const unsigned tiles = (unsigned)((p.ngpown + 15) / 16) * (unsigned)((p.ncouls + 15) / 16);
+        hipLaunchKernelGGL(k_gram_small, dim3(tiles), dim3(kSmThreads), 0, s, bg, p.aqsn, p.ngpown, p.ncouls, p.nv,
+                           p.nb, mu);
+        break;
+    }
     }
     return hipGetLastError();
 }

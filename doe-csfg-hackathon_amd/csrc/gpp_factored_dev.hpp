@@ -20,47 +20,387 @@ namespace fact {
 
 typedef double v4d __attribute__((ext_vector_type(4)));
 
-constexpr int kKS = 8;             // bands per LDS stage of the smaller FP64 Gram tiles (two MFMA k-steps)
-constexpr int kWJ = 64, kWI = 32;  // FP64 Gram wave tile: 64 G' columns x 32 G-vectors
+constexpr int kWJ = 64, kWI = 32;  // wave tile of the fused Gram and the acht product: 64 rows x 32 columns
 constexpr int kRedThreads = 256;   // pole-reduce and final-reduce blocks
 
-// FP64 Gram block tile made of WJN x WIN waves; KS bands per LDS stage,
-// staged through registers in NH pieces.  The 128 x 128 tile stages 16 bands
-// (four k-steps per barrier) in two pieces of 8, each stored to the other
-// buffer after its k-steps, so its staging registers fit two waves per SIMD;
-// the smaller tiles stage 8 in one piece (more would spill).
-template <int WJN, int WIN> struct GramCfg {
-    static constexpr int TJ = kWJ * WJN, TI = kWI * WIN, NT = 64 * WJN * WIN;
-    static constexpr int KS = WJN * WIN == 8 ? 16 : kKS;
-    static constexpr int NH = WJN * WIN == 8 ? 2 : 1;
-};
+// s_waitcnt vmcnt(N) lgkmcnt(0) (N < 64): at most N of the wave's loads from
+// memory are in flight, and none of its LDS reads.
+template <int N> __device__ __forceinline__ void wait_vm_lds()
+{
+    static_assert(N >= 0 && N < 64, "vmcnt has six bits");
+    __builtin_amdgcn_s_waitcnt((N & 15) | ((N >> 4) << 14) | (7 << 4));
+}
 
-// Stage 2: one TJ x TI tile of Mu = conj(Bg)^T * aqsn over bands [k_begin, k_end)
-// on v_mfma_f64_16x16x4f64.  Lane layout (measured on gfx950): A[l%16][l/16],
+// Barrier of waves that order their memory with wait_vm_lds (no fence, which
+// would wait for the loads of the stages ahead); the empty asm keeps the
+// compiler from moving memory accesses across it.
+__device__ __forceinline__ void ring_barrier()
+{
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+}
+// 16 bytes per lane from memory straight into LDS, in lane order from `dst`.
+__device__ __forceinline__ void ring_load(const cplx *src, cplx *dst)
+{
+    __builtin_amdgcn_global_load_lds(src, (__attribute__((address_space(3))) void *)dst, 16, 0, 0);
+}
+
+// Stage 2: Mu = conj(Bg)^T * aqsn over bands [k_begin, k_end) on
+// v_mfma_f64_16x16x4f64.  Lane layout (measured on gfx950): A[l%16][l/16],
 // B[l/16][l%16], result r of lane l = C[4r + l/16][l%16]; MFMA rows are G'
 // columns j and MFMA columns are G-vectors ig, so each result row is
-// contiguous in ig.  sB/sA are the block's double-buffered LDS stages.
-// Three real products per complex product (3M): with b = Bg, a = aqsn,
+// contiguous in ig.  Three real products per complex product (3M): with
+// b = Bg, a = aqsn,
 //   P1 = sum br ar,  P2 = sum bi ai,  P3 = sum (br - bi)(ar + ai),
 //   Re Mu = P1 + P2,  Im Mu = (P3 - P1) + P2  (= sum br ai - bi ar),
 // three accumulators fed by one MFMA each per k-step instead of two fed by
 // two.  Rounding: |P3| <= 2 sum |b||a|, so the error stays of order
-// 1e-16 sum |b||a| (normwise), as with four products.
+// 1e-16 sum |b||a| (normwise), as with four products.  Every element is the
+// same sum of the same products in the same order in every tile below.
 //
-// TRANS swaps the MFMA operands: rows are then G-vectors and columns G'
-// columns, result r of lane l of sub-tile (s, t) is element
-// (ig = wi + 16t + 4r + l/16, j = wj + 16s + l%16) -- each lane holds four
-// G' columns and eight G-vectors of each, the layout the fused pole
-// epilogue sums over G-vectors in.  Every element is the same sum of the
-// same products in either orientation.
-template <int WJN, int WIN, bool TRANS = false>
+// A tile of WJN x WIN waves, each owning SJ x SI sub-tiles of 16 G' columns x
+// 16 G-vectors (TJ x TI in all).  Stages of KS bands go straight from memory
+// into a ring of NB LDS buffers, NB - 1 stages ahead, with one barrier per
+// stage.  Columns past the edge load the last column (their results are
+// dropped); bands past the end load the last band and count as zero.
+//
+// What bounds them: the FP64 MFMA pipe (64 cycles per MFMA and SIMD), kept
+// busy by the waves that do not wait for a stage's barrier and fragments.
+// The tiles take at most 80 KB of LDS, so two blocks share a CU and one's
+// stage turnover runs under the other's MFMAs; staging without registers
+// leaves the 64 x 128 tile four waves per SIMD.  Measured (one launch, the
+// 128 x 128 tile of eight waves staged through registers, one block per CU,
+// against 64 x 128 here): 512/2/32768/1638 2587 -> 2530 us (65 TFLOP/s on the
+// three products; a large FP64 library product reaches 70 on this chip),
+// 1536/8/32768/1638 7564 -> 7451 us, 512/2/16384/819 794 -> 669 us (64 x 64).
+template <int WJN_, int WIN_, int SJ_, int SI_, int KS_, int NB_, int OCC_> struct GramRing {
+    static constexpr int WJN = WJN_, WIN = WIN_, SJ = SJ_, SI = SI_, KS = KS_, NB = NB_;
+    static constexpr int OCC = OCC_;  // waves per SIMD
+    static constexpr int NW = WJN * WIN, TJ = 16 * SJ * WJN, TI = 16 * SI * WIN, NT = 64 * NW;
+    static constexpr int STAGE = KS * (TJ + TI);  // entries
+    static constexpr int LDS = NB * STAGE;
+};
+typedef GramRing<2, 4, 2, 2, 8, 3, 4> GramL;   // 64 x 128
+typedef GramRing<4, 2, 2, 2, 8, 3, 4> GramLt;  // 128 x 64
+typedef GramRing<2, 2, 2, 2, 8, 4, 2> GramM;   // 64 x 64
+typedef GramRing<2, 4, 1, 1, 16, 3, 4> GramS;  // 32 x 64
+
+// One tile with SJC <= SJ sub-tile rows per wave: the first 16 SJC WJN columns
+// from j0, for a last tile whose columns need no more.  nts: non-temporal
+// stores of Mu.  The block's waves must be done with lds before the call.
+template <class C, int SJC>
+__device__ __forceinline__ void gram_ring_tile(const cplx *__restrict__ bg, const cplx *__restrict__ aqsn, int ngpown,
+                                               int ncouls, int k_begin, int k_end, int j0, int i0, cplx *lds,
+                                               bool nts, cplx *__restrict__ mout)
+{
+    constexpr int KS = C::KS, NB = C::NB, TJ = C::TJ, TI = C::TI, SI = C::SI, NW = C::NW;
+    constexpr int QB = KS * TJ / 64 / NW, QA = KS * TI / 64 / NW, LD = QB + QA;  // loads per wave and stage
+    static_assert(QB * 64 * NW == KS * TJ && QA * 64 * NW == KS * TI && NB >= 3, "loads split evenly over the waves");
+    static_assert(SJC >= 1 && SJC <= C::SJ && KS % 4 == 0, "sub-tiles of the tile, whole k-steps");
+    const int lane = threadIdx.x % kWave;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+    const int wj = (wave / C::WIN) * (16 * SJC), wi = (wave % C::WIN) * (16 * SI);
+    const int nst = (k_end - k_begin + KS - 1) / KS;
+
+    // Load q of a side fills elements [64 (q NW + wave), +64) of its rows of a
+    // stage: this lane's source element of each, advanced from stage to stage.
+    const cplx *pb[QB], *pa[QA];
+#pragma unroll
+    for (int q = 0; q < QB; ++q) {
+        const int e = 64 * (q * NW + wave) + lane;
+        pb[q] = bg + (size_t)(k_begin + e / TJ) * ngpown + min(j0 + e % TJ, ngpown - 1);
+    }
+#pragma unroll
+    for (int q = 0; q < QA; ++q) {
+        const int e = 64 * (q * NW + wave) + lane;
+        pa[q] = aqsn + (size_t)(k_begin + e / TI) * ncouls + min(i0 + e % TI, ncouls - 1);
+    }
+    const size_t stepb = (size_t)KS * ngpown, stepa = (size_t)KS * ncouls;
+    int ibuf = 0, rbuf = 0;  // next buffer to fill, to read
+    auto issue = [&]() {
+        cplx *buf = lds + ibuf * C::STAGE + 64 * wave;
+        ibuf = ibuf + 1 == NB ? 0 : ibuf + 1;
+#pragma unroll
+        for (int q = 0; q < QB; ++q) {
+            ring_load(pb[q], buf + 64 * NW * q);
+            pb[q] += stepb;
+        }
+#pragma unroll
+        for (int q = 0; q < QA; ++q) {
+            ring_load(pa[q], buf + KS * TJ + 64 * NW * q);
+            pa[q] += stepa;
+        }
+    };
+    auto issue_last = [&]() {  // stage nst - 1: rows past the end load the last band
+        cplx *buf = lds + ibuf * C::STAGE + 64 * wave;
+        const int over0 = k_begin + (nst - 1) * KS - (k_end - 1);
+#pragma unroll
+        for (int q = 0; q < QB; ++q) {
+            const int over = max(0, over0 + (64 * (q * NW + wave) + lane) / TJ);
+            ring_load(pb[q] - (size_t)over * ngpown, buf + 64 * NW * q);
+        }
+#pragma unroll
+        for (int q = 0; q < QA; ++q) {
+            const int over = max(0, over0 + (64 * (q * NW + wave) + lane) / TI);
+            ring_load(pa[q] - (size_t)over * ncouls, buf + KS * TJ + 64 * NW * q);
+        }
+    };
+
+    v4d acc1[SJC][SI], acc2[SJC][SI], acc3[SJC][SI];  // P1, P2, P3
+#pragma unroll
+    for (int s = 0; s < SJC; ++s)
+#pragma unroll
+        for (int t = 0; t < SI; ++t) acc1[s][t] = acc2[s][t] = acc3[s][t] = v4d{0, 0, 0, 0};
+    auto multiply = [&](auto last) {
+        const cplx *sB = lds + rbuf * C::STAGE, *sA = sB + KS * TJ;
+        rbuf = rbuf + 1 == NB ? 0 : rbuf + 1;
+        __builtin_amdgcn_s_setprio(1);  // the wave with ready operands issues its MFMAs first
+#pragma unroll
+        for (int kk = 0; kk < KS; kk += 4) {
+            const int kr = kk + lane / 16;
+            const bool out = last && k_begin + (nst - 1) * KS + kr >= k_end;
+            double are[SI], aim[SI], asum[SI];
+#pragma unroll
+            for (int t = 0; t < SI; ++t) {
+                cplx a = sA[kr * TI + wi + 16 * t + lane % 16];
+                if (out) a = czero();
+                are[t] = a.re;
+                aim[t] = a.im;
+                asum[t] = a.re + a.im;
+            }
+#pragma unroll
+            for (int s = 0; s < SJC; ++s) {
+                cplx b = sB[kr * TJ + wj + 16 * s + lane % 16];
+                if (out) b = czero();
+                const double bdiff = b.re - b.im;
+#pragma unroll
+                for (int t = 0; t < SI; ++t) {
+                    acc1[s][t] = __builtin_amdgcn_mfma_f64_16x16x4f64(b.re, are[t], acc1[s][t], 0, 0, 0);
+                    acc2[s][t] = __builtin_amdgcn_mfma_f64_16x16x4f64(b.im, aim[t], acc2[s][t], 0, 0, 0);
+                    acc3[s][t] = __builtin_amdgcn_mfma_f64_16x16x4f64(bdiff, asum[t], acc3[s][t], 0, 0, 0);
+                }
+            }
+        }
+        __builtin_amdgcn_s_setprio(0);
+    };
+
+    // At the top of stage st, stages st .. st + NB - 2 have been issued: wait
+    // for this wave's loads of stage st and its fragment reads of stage
+    // st - 1, then (barrier) for every wave's; stage st + NB - 1 then takes the
+    // buffer of stage st - 1.
+    for (int st = 0; st < NB - 1 && st < nst; ++st) {
+        if (st < nst - 1)
+            issue();
+        else
+            issue_last();
+    }
+    int st = 0;
+    for (; st < nst - NB; ++st) {  // the stages that issue a whole stage
+        wait_vm_lds<(NB - 2) * LD>();
+        ring_barrier();
+        issue();
+        multiply(std::integral_constant<bool, false>());
+    }
+    if (nst >= NB) {  // st = nst - NB: issues the last stage
+        wait_vm_lds<(NB - 2) * LD>();
+        ring_barrier();
+        issue_last();
+        multiply(std::integral_constant<bool, false>());
+        ++st;
+    }
+    for (; st < nst - 1; ++st) {
+        wait_vm_lds<0>();
+        ring_barrier();
+        multiply(std::integral_constant<bool, false>());
+    }
+    if (nst > 0) {
+        wait_vm_lds<0>();
+        ring_barrier();
+        multiply(std::integral_constant<bool, true>());
+    }
+#pragma unroll
+    for (int s = 0; s < SJC; ++s)
+#pragma unroll
+        for (int t = 0; t < SI; ++t)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const int j = j0 + wj + 16 * s + 4 * r + lane / 16;
+                const int ig = i0 + wi + 16 * t + lane % 16;
+                if (j < ngpown && ig < ncouls) {
+                    const cplx v = {acc1[s][t][r] + acc2[s][t][r], (acc3[s][t][r] - acc1[s][t][r]) + acc2[s][t][r]};
+                    cplx *o = &mout[(size_t)j * ncouls + ig];
+                    if (nts) {
+                        __builtin_nontemporal_store(v.re, &o->re);
+                        __builtin_nontemporal_store(v.im, &o->im);
+                    } else {
+                        *o = v;
+                    }
+                }
+            }
+}
+
+// One 16 x 16 tile of Mu by three waves, one per real product of the 3M form
+// (P1, P2, P3 of gram_f64_acc, combined as there), for products with fewer
+// tiles than the chip has SIMDs: the chain of dependent MFMAs over the bands
+// bounds those, and a wave with one product per tile has a third of the chain
+// of a wave with all three.  Stages of kSmK bands go straight from memory into
+// a ring of kSmBuf LDS buffers, kSmBuf - 1 stages ahead (about 0.8 us of MFMA
+// time); the fragments of stage st + 1 are read while stage st is multiplied.
+// Columns past the edge load the last column (their results are dropped);
+// bands past the end load the last band and count as zero.
+constexpr int kSmK = 24, kSmBuf = 6, kSmThreads = 192;
+constexpr int kSmStage = 2 * kSmK * 16;  // entries of a stage: Bg rows, then aqsn rows
+template <int P>
+__device__ __forceinline__ v4d gram_small_product(const cplx *__restrict__ bg, const cplx *__restrict__ aqsn,
+                                                  int ngpown, int ncouls, int k_begin, int k_end, int j0, int i0,
+                                                  cplx *lds)
+{
+    constexpr int STEPS = kSmK / 4;
+    constexpr int ROWS = kSmK / 3;  // rows of a stage each wave loads, four per instruction
+    static_assert(ROWS % 4 == 0, "a wave loads whole groups of four rows");
+    constexpr int Q = ROWS / 4, LD = 2 * Q;  // loads per wave and stage: Q of each operand
+    const int lane = threadIdx.x % kWave;
+    const int nst = (k_end - k_begin + kSmK - 1) / kSmK;
+    // This lane's element of the wave's rows (the wave of product P loads rows
+    // [P ROWS, (P + 1) ROWS) of a stage), advanced from stage to stage.
+    const int r0 = P * ROWS + lane / 16;
+    const cplx *pb = bg + (size_t)(k_begin + r0) * ngpown + min(j0 + lane % 16, ngpown - 1);
+    const cplx *pa = aqsn + (size_t)(k_begin + r0) * ncouls + min(i0 + lane % 16, ncouls - 1);
+    const size_t rb = 4 * (size_t)ngpown, ra = 4 * (size_t)ncouls;
+    int issued = 0, ibuf = 0;  // next stage to load and its buffer
+    auto issue = [&]() {
+        cplx *buf = lds + ibuf * kSmStage + P * ROWS * 16;
+        if (issued < nst - 1) {
+#pragma unroll
+            for (int q = 0; q < Q; ++q) {
+                __builtin_amdgcn_global_load_lds(pb + q * rb, (__attribute__((address_space(3))) void *)(buf + q * 64),
+                                                 16, 0, 0);
+                __builtin_amdgcn_global_load_lds(
+                    pa + q * ra, (__attribute__((address_space(3))) void *)(buf + kSmK * 16 + q * 64), 16, 0, 0);
+            }
+            pb += (kSmK / 4) * rb;
+            pa += (kSmK / 4) * ra;
+        } else {  // the last stage: rows past the end load the last band
+#pragma unroll
+            for (int q = 0; q < Q; ++q) {
+                const long long over = max(0, k_begin + issued * kSmK + r0 + 4 * q - (k_end - 1));
+                __builtin_amdgcn_global_load_lds(pb + q * rb - over * ngpown,
+                                                 (__attribute__((address_space(3))) void *)(buf + q * 64), 16, 0, 0);
+                __builtin_amdgcn_global_load_lds(
+                    pa + q * ra - over * ncouls,
+                    (__attribute__((address_space(3))) void *)(buf + kSmK * 16 + q * 64), 16, 0, 0);
+            }
+        }
+        ++issued;
+        ibuf = ibuf + 1 == kSmBuf ? 0 : ibuf + 1;
+    };
+    // Operands of a stage: the wave's part of the fragments (P1 real, P2
+    // imaginary parts; P3 both, summed after they have arrived).
+    struct Frag {
+        double b[STEPS], a[STEPS], bi[P == 2 ? STEPS : 1], ai[P == 2 ? STEPS : 1];
+    };
+    Frag f0, f1;
+    int rbuf = 0;  // buffer of the next stage to read
+    auto read = [&](Frag &f, const cplx *buf, int s) {
+        const cplx &b = buf[s * 64 + lane], &a = buf[kSmK * 16 + s * 64 + lane];
+        f.b[s] = P == 1 ? b.im : b.re;
+        f.a[s] = P == 1 ? a.im : a.re;
+        if constexpr (P == 2) {
+            f.bi[s] = b.im;
+            f.ai[s] = a.im;
+        }
+    };
+    auto finish = [&](Frag &f) {
+        if constexpr (P == 2) {
+#pragma unroll
+            for (int s = 0; s < STEPS; ++s) {
+                f.b[s] -= f.bi[s];
+                f.a[s] += f.ai[s];
+            }
+        }
+    };
+    v4d acc = {0, 0, 0, 0};
+    // All of a wave's loads of stage st have landed (of the kSmBuf - 2 stages
+    // st .. st + kSmBuf - 3 issued by now, those after it may be in flight)
+    // and its fragment reads are done, then every wave's.  The empty asm keeps
+    // the LDS reads below the barrier.
+    auto arrive = [&](int st) {
+        if (st + kSmBuf - 3 < nst)
+            wait_vm_lds<(kSmBuf - 3) * LD>();
+        else
+            wait_vm_lds<0>();
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+    };
+    // Round st of all but the last: stage st + 1 lands; the buffer that stage
+    // st + kSmBuf - 1 takes is that of stage st - 1, whose fragments every wave
+    // has read.  The fragment reads of stage st + 1 go between the products of
+    // stage st.
+    auto round = [&](int st, Frag &cur, Frag &nxt) {
+        finish(cur);
+        arrive(st + 1);
+        if (issued < nst) issue();
+        const cplx *buf = lds + rbuf * kSmStage;
+        rbuf = rbuf + 1 == kSmBuf ? 0 : rbuf + 1;
+#pragma unroll
+        for (int s = 0; s < STEPS; ++s) {
+            acc = __builtin_amdgcn_mfma_f64_16x16x4f64(cur.b[s], cur.a[s], acc, 0, 0, 0);
+            read(nxt, buf, s);
+            __builtin_amdgcn_sched_group_barrier(8, 1, 0);      // one MFMA
+            __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);  // two LDS reads
+        }
+    };
+    auto last_round = [&](Frag &f) {
+        finish(f);
+#pragma unroll
+        for (int s = 0; s < STEPS; ++s) {
+            const bool out = k_begin + (nst - 1) * kSmK + 4 * s + lane / 16 >= k_end;
+            acc = __builtin_amdgcn_mfma_f64_16x16x4f64(out ? 0.0 : f.b[s], out ? 0.0 : f.a[s], acc, 0, 0, 0);
+        }
+    };
+    if (nst == 0) return acc;
+    for (int st = 0; st < kSmBuf - 1 && st < nst; ++st) issue();
+    arrive(0);
+#pragma unroll
+    for (int s = 0; s < STEPS; ++s) read(f0, lds, s);
+    rbuf = 1;
+    int st = 0;
+    for (; st + 2 < nst; st += 2) {
+        round(st, f0, f1);
+        round(st + 1, f1, f0);
+    }
+    if (st + 1 < nst) {
+        round(st, f0, f1);
+        last_round(f1);
+    } else {
+        last_round(f0);
+    }
+    return acc;
+}
+
+// The Gram tile of the fused Gram + pole reduce: 128 x 128 by 2 x 4 waves of
+// 64 x 32, 16 bands per LDS stage staged through registers in two pieces of 8,
+// each stored to the other buffer after its k-steps, so that its staging
+// registers fit two waves per SIMD.
+struct FuseCfg {
+    static constexpr int WIN = 4, TJ = 2 * kWJ, TI = 4 * kWI, NT = 512;
+    static constexpr int KS = 16, NH = 2;
+};
+
+// The sums of gram_ring_tile with the MFMA operands swapped: rows are
+// G-vectors and columns G' columns, result r of lane l of sub-tile (s, t) is
+// element (ig = wi + 16t + 4r + l/16, j = wj + 16s + l%16) -- each lane holds
+// four G' columns and eight G-vectors of each, the layout the fused pole
+// epilogue sums over G-vectors in.
 __device__ __forceinline__ void gram_f64_acc(const cplx *__restrict__ bg, const cplx *__restrict__ aqsn, int ngpown,
                                              int ncouls, int k_begin, int k_end, int j0, int i0,
-                                             cplx (*sB)[GramCfg<WJN, WIN>::KS][GramCfg<WJN, WIN>::TJ],
-                                             cplx (*sA)[GramCfg<WJN, WIN>::KS][GramCfg<WJN, WIN>::TI], v4d (&acc1)[4][2],
+                                             cplx (*sB)[FuseCfg::KS][FuseCfg::TJ],
+                                             cplx (*sA)[FuseCfg::KS][FuseCfg::TI], v4d (&acc1)[4][2],
                                              v4d (&acc2)[4][2], v4d (&acc3)[4][2])
 {
-    typedef GramCfg<WJN, WIN> C;
+    typedef FuseCfg C;
     constexpr int TJ = C::TJ, TI = C::TI, NT = C::NT, KS = C::KS, NH = C::NH;
     constexpr int PB = KS * TJ / NT / NH, PA = KS * TI / NT / NH;  // staged elements per thread and piece
     static_assert(PB * NT * NH == KS * TJ && PA * NT * NH == KS * TI, "stage must split evenly");
@@ -68,8 +408,8 @@ __device__ __forceinline__ void gram_f64_acc(const cplx *__restrict__ bg, const 
                   "a piece is whole band rows and whole k-steps");
     const int lane = threadIdx.x % kWave;
     const int wave = threadIdx.x / kWave;
-    const int wj = (wave / WIN) * kWJ;
-    const int wi = (wave % WIN) * kWI;
+    const int wj = (wave / C::WIN) * kWJ;
+    const int wi = (wave % C::WIN) * kWI;
 
 #pragma unroll
     for (int s = 0; s < 4; ++s)
@@ -140,15 +480,9 @@ __device__ __forceinline__ void gram_f64_acc(const cplx *__restrict__ bg, const 
                 const double bdiff = b.re - b.im;
 #pragma unroll
                 for (int t = 0; t < 2; ++t) {
-                    if constexpr (TRANS) {
-                        acc1[s][t] = __builtin_amdgcn_mfma_f64_16x16x4f64(are[t], b.re, acc1[s][t], 0, 0, 0);
-                        acc2[s][t] = __builtin_amdgcn_mfma_f64_16x16x4f64(aim[t], b.im, acc2[s][t], 0, 0, 0);
-                        acc3[s][t] = __builtin_amdgcn_mfma_f64_16x16x4f64(asum[t], bdiff, acc3[s][t], 0, 0, 0);
-                    } else {
-                        acc1[s][t] = __builtin_amdgcn_mfma_f64_16x16x4f64(b.re, are[t], acc1[s][t], 0, 0, 0);
-                        acc2[s][t] = __builtin_amdgcn_mfma_f64_16x16x4f64(b.im, aim[t], acc2[s][t], 0, 0, 0);
-                        acc3[s][t] = __builtin_amdgcn_mfma_f64_16x16x4f64(bdiff, asum[t], acc3[s][t], 0, 0, 0);
-                    }
+                    acc1[s][t] = __builtin_amdgcn_mfma_f64_16x16x4f64(are[t], b.re, acc1[s][t], 0, 0, 0);
+                    acc2[s][t] = __builtin_amdgcn_mfma_f64_16x16x4f64(aim[t], b.im, acc2[s][t], 0, 0, 0);
+                    acc3[s][t] = __builtin_amdgcn_mfma_f64_16x16x4f64(asum[t], bdiff, acc3[s][t], 0, 0, 0);
                 }
             }
         }
@@ -157,38 +491,6 @@ __device__ __forceinline__ void gram_f64_acc(const cplx *__restrict__ bg, const 
         }
         __syncthreads();
     }
-}
-
-// Stage 2 with Mu written to HBM ([ngpown][ncouls], rows contiguous in ig).
-template <int WJN, int WIN>
-__device__ __forceinline__ void gram_f64_tile(const cplx *__restrict__ bg, const cplx *__restrict__ aqsn, int ngpown,
-                                              int ncouls, int k_begin, int k_end, int j0, int i0,
-                                              cplx (*sB)[GramCfg<WJN, WIN>::KS][GramCfg<WJN, WIN>::TJ],
-                                              cplx (*sA)[GramCfg<WJN, WIN>::KS][GramCfg<WJN, WIN>::TI],
-                                              cplx *__restrict__ mout)
-{
-    const int lane = threadIdx.x % kWave;
-    const int wave = threadIdx.x / kWave;
-    const int wj = (wave / WIN) * kWJ;
-    const int wi = (wave % WIN) * kWI;
-    v4d acc1[4][2], acc2[4][2], acc3[4][2];  // P1, P2, P3
-    gram_f64_acc<WJN, WIN>(bg, aqsn, ngpown, ncouls, k_begin, k_end, j0, i0, sB, sA, acc1, acc2, acc3);
-#pragma unroll
-    for (int s = 0; s < 4; ++s)
-#pragma unroll
-        for (int t = 0; t < 2; ++t)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const int j = j0 + wj + 16 * s + 4 * r + lane / 16;
-                const int ig = i0 + wi + 16 * t + lane % 16;
-                if (j < ngpown && ig < ncouls) {
-                    // non-temporal: Mu is written once and read back once, by
-                    // the pole reduce (C1 reduce 0.486-0.502 -> 0.469 ms)
-                    __builtin_nontemporal_store(acc1[s][t][r] + acc2[s][t][r], &mout[(size_t)j * ncouls + ig].re);
-                    __builtin_nontemporal_store((acc3[s][t][r] - acc1[s][t][r]) + acc2[s][t][r],
-                                                &mout[(size_t)j * ncouls + ig].im);
-                }
-            }
 }
 
 // 2^-40 band around a threshold inside which a decision made on an estimate
@@ -631,7 +933,7 @@ struct PoleTileArgs {
 // per-wave column sums of one column round.
 constexpr int kFuseNv = 4;
 template <int F> struct FuseLds {
-    typedef GramCfg<2, 4> C;
+    typedef FuseCfg C;
     static constexpr int kCols = 32, kRows = 64;   // columns x G-vectors per round
     static constexpr int kPitch = kRows + 1;       // entries per staged row
     static constexpr int kWt = 0, kIe = kCols * kPitch, kMu = 2 * kCols * kPitch;
@@ -664,7 +966,7 @@ __device__ __forceinline__ void gram_pole_epilogue(const PoleTileArgs &a, int j0
 {
 #pragma clang fp contract(off)
     typedef FuseLds<F> L;
-    typedef GramCfg<2, 4> C;
+    typedef FuseCfg C;
     const int lane = threadIdx.x % kWave;
     const int wave = threadIdx.x / kWave;
     const int wjn = wave / 4, wv = wave % 4;  // 64-column half, 32-G-vector quarter

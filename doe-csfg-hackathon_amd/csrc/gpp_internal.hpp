@@ -125,7 +125,7 @@ struct GramKind {
     int layout = 4;        // Ozaki block layout (0, 1: 64x64 staged in registers; 2: 64x32; 3: 64x64 on 32x32 MFMAs;
                            // 4: layout 3 in persistent blocks; 2-4 load straight into LDS)
     int group = 0;         // Ozaki G' tiles per tile group (0: sized for the L2)
-    int tile = 0;          // FP64 Gram tile: 0 128x128, 1 64x128, 2 128x64, 3 64x64 (G' x G)
+    int tile = 0;          // FP64 Gram tile: 0 by size (batches 64x128), 1 64x128, 2 128x64, 3 64x64 (G' x G)
     int red_chunk = 8192;  // G-vectors per pole-reduce block
     int red_fc = 0;        // frequencies per pole-reduce pass when nfreq > 4 (4, 8, 16; 0: 16 from 16 up, else 8;
                            // the batched form: 4, else 8)

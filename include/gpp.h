@@ -118,8 +118,9 @@ typedef enum {
      * layout 3 in persistent blocks, one per compute unit, whose tiles form
      * one stream of band steps (default). */
     GPP_OPT_OZAKI_LAYOUT = 2,
-    /* FP64-MFMA Gram tile (G' columns x G-vectors): 0 = 128x128 (default),
-     * 1 = 64x128, 2 = 128x64, 3 = 64x64. */
+    /* FP64-MFMA Gram tile (G' columns x G-vectors): 0 = chosen by the
+     * problem's size (default; a batch runs 64x128), 1 = 64x128, 2 = 128x64,
+     * 3 = 64x64.  Every tile gives the same bits. */
     GPP_OPT_GRAM_TILE = 3,
     /* G-vectors per pole-reduce block: a power of two in [256, 2^20]
      * (default 8192). */
@@ -147,7 +148,7 @@ typedef enum {
      * digit planes once per group.  0 = sized for the L2 (default). */
     GPP_OPT_OZAKI_GROUP = 8,
     /* GPP_FORM_FACTORED_F64 with at most 3 frequencies, none negative, at
-     * most 4 occupied bands, the 128x128 Gram tile and acht_n1_loc not
+     * most 4 occupied bands, GPP_OPT_GRAM_TILE 0 and acht_n1_loc not
      * requested: 1 = evaluate the pole factors in the epilogue of the Gram
      * product, so the G'xG product Mu (ngpown * ncouls * 16 bytes of
      * workspace) is never stored -- for problems whose Mu does not fit in
