@@ -35,27 +35,54 @@ using namespace fact;
 
 __host__ inline size_t align256(size_t x) { return (x + 255) & ~(size_t)255; }
 
-// acht product tiles: rows j in 128s for both band ranges; unoccupied bands
-// in columns of 128, occupied bands (few) in columns of 32.
-typedef AchtCfg<2, 4> AchtU;
+constexpr double kGramCus = 256;  // compute units of an MI355X
 
+// Rounds of blocks over the CUs for `whole` tiles and then `halves` tiles of
+// half their work, which fill the last round as far as they fit.
+double tile_rounds(double whole, double halves)
+{
+    const double rounds = ceil(whole / kGramCus), over = halves / 2 - (rounds * kGramCus - whole);
+    return over > 0 ? rounds + ceil(2 * over / kGramCus) / 2 : rounds;
+}
+
+// acht product tiles (rows j x bands): 64 x 128, or 64 x 64 (narrow).
 struct AchtSplit {
-    int jtiles, nks, chunk;
+    int jtiles, ntiles, nks, chunk;
+    bool narrow;
+    bool cut;  // the last j tile has at most 32 rows: one sub-tile row per wave
 };
 
-// Split of the G-vector sum so that the unoccupied launch has ~4096 blocks
-// (C1: 3.9 % faster than ~2048, 7 % faster than ~1024).
+// Tile and split of the G-vector sum of the acht product: the least estimated
+// time over splits that give each CU a whole number of blocks.  A block's
+// k-steps run at the Gram product's rates (gram_tile_for); kBlock covers its
+// first loads and its epilogue, kPart the fixed-order sum of the partials.
+// acht stage, us, against one 128 x 128 tile staged through registers and at
+// least 512 G-vectors a block: 24/2/1000/50 389 -> 14, 512/2/4096/409
+// 227 -> 110, 512/2/32768/1638 2805 -> 2550.
 AchtSplit acht_split(const DevProblem &p)
 {
     AchtSplit a;
-    a.jtiles = (p.ngpown + AchtU::TJ - 1) / AchtU::TJ;
-    const int ntiles = (p.nb - p.nv + AchtU::TN - 1) / AchtU::TN;
-    const int tiles = a.jtiles * (ntiles > 0 ? ntiles : 1);
-    int nks = (4096 + tiles - 1) / tiles;
-    const int max_nks = p.ncouls / 512 > 1 ? p.ncouls / 512 : 1;
-    if (nks > max_nks) nks = max_nks;
-    a.chunk = ((p.ncouls + nks - 1) / nks + kAKS - 1) / kAKS * kAKS;
-    a.nks = (p.ncouls + a.chunk - 1) / a.chunk;
+    const int nu = p.nb - p.nv, rem = p.ngpown % GramL::TJ;
+    a.jtiles = (p.ngpown + GramL::TJ - 1) / GramL::TJ;
+    a.cut = rem > 0 && rem <= GramL::TJ / 2;
+    const double kBlock = 3.0, kPart = 0.01;  // us
+    double best = 1e300;
+    for (int narrow = 0; narrow < 2; ++narrow) {
+        const int tn = narrow ? GramM::TI : GramL::TI;
+        const int ntiles = std::max(1, (nu + tn - 1) / tn);
+        const double tiles = (a.jtiles - (a.cut ? 0.5 : 0.0)) * ntiles, sub = GramL::TJ / 16 * (tn / 16);
+        const double whole = (a.jtiles - (a.cut ? 1 : 0)) * ntiles, halves = a.cut ? ntiles : 0;
+        for (int r = 1; r <= 32; ++r) {
+            int nks = (int)(r * kGramCus / tiles);
+            nks = std::max(1, std::min(nks, (p.ncouls + 31) / 32));
+            const int chunk = ((p.ncouls + nks - 1) / nks + GramL::KS - 1) / GramL::KS * GramL::KS;
+            nks = (p.ncouls + chunk - 1) / chunk;
+            const double rounds = tile_rounds(whole * nks, halves * nks);
+            const double rate = rounds <= 1 ? (narrow ? 0.0287 : 0.0258) : narrow ? 0.0247 : 0.0237;
+            const double us = rounds * (sub * (chunk / 4) * rate + kBlock) + kPart * a.jtiles * nks;
+            if (us < best) best = us, a.nks = nks, a.chunk = chunk, a.ntiles = ntiles, a.narrow = narrow != 0;
+        }
+    }
     return a;
 }
 
@@ -72,11 +99,21 @@ bool fused_reduce(const DevProblem &p, const GramKind &k)
 // written once and read back once, by the pole reduce (C1, 859 MB: reduce
 // 0.486-0.502 -> 0.469 ms); a smaller one is read back from them.
 bool mu_streams(const DevProblem &p) { return sizeof(cplx) * (size_t)p.ngpown * p.ncouls > ((size_t)256 << 20); }
-constexpr double kGramCus = 256;  // compute units of an MI355X
+
+// G-vectors per block of k_acht_occ: the reduce's range, halved while the
+// launch has fewer than 2048 blocks (each thread waits on its own loads:
+// 100/8/3000/200/5 33 -> 21 us).
+int acht_occ_chunk(const DevProblem &p, int red_chunk)
+{
+    int chunk = red_chunk;
+    while (chunk > 512 && (long long)p.ngpown * ((p.ncouls + chunk - 1) / chunk) < 2048) chunk /= 2;
+    return chunk;
+}
 
 struct FactLayout {
     size_t bg, m, col_ach, col_asx, col2_ach, col2_asx, part_achs, p2, br1, acht_part, acht_occ, total;
     int nsplit;  // G-vector ranges of the pole-reduce partials (the fused form: G-vector tiles)
+    int occ_chunk = 0, occ_nsplit = 0;  // G-vector ranges of the occupied bands' acht_n1_loc partials
     bool fused;
     AchtSplit as;
 };
@@ -98,7 +135,7 @@ FactLayout fact_layout(const DevProblem &p, const GramKind &k)
     }
     L.part_achs = off; off += align256(sizeof(cplx) * ach_region_entries(p.nb, p.ngpown));
     L.p2 = L.br1 = L.acht_part = L.acht_occ = off;
-    L.as = AchtSplit{0, 0, 0};
+    L.as = AchtSplit{};
     if (k.acht) {
         L.as = acht_split(p);
         L.p2 = off;        off += align256(sizeof(cplx) * (size_t)p.ngpown * p.ncouls);
@@ -106,7 +143,9 @@ FactLayout fact_layout(const DevProblem &p, const GramKind &k)
         // occupied bands itself
         L.br1 = off;       off += p.nv > 0 && !reduce_sums_acht_occ(p.nv, p.wx_neg) ? align256((size_t)p.ngpown * p.ncouls) : 0;
         L.acht_part = off; off += align256(sizeof(cplx) * (size_t)L.as.jtiles * L.as.nks * p.nb);
-        L.acht_occ = off;  off += align256(sizeof(cplx) * (size_t)p.ngpown * L.nsplit * (p.nv > 0 ? p.nv : 1));
+        L.occ_chunk = acht_occ_chunk(p, k.red_chunk);
+        L.occ_nsplit = reduce_sums_acht_occ(p.nv, p.wx_neg) ? L.nsplit : (p.ncouls + L.occ_chunk - 1) / L.occ_chunk;
+        L.acht_occ = off;  off += align256(sizeof(cplx) * (size_t)p.ngpown * L.occ_nsplit * (p.nv > 0 ? p.nv : 1));
     }
     L.total = off;
     return L;
@@ -241,31 +280,32 @@ __global__ __launch_bounds__(kRedThreads) void k_fact_final(const cplx *col_ach,
     final_block(col_ach, col_asx, part_achs, ncols, nfreq, nb, nv, out, scratch, blockIdx.x);
 }
 
-// 1-D grid over (column tiles, j tiles, G-vector splits), column tiles
-// fastest in tile order and spread over the XCDs by xcd_tile, so the blocks
-// that share one R tile run on one XCD.  part: [jtiles * nks][nb].
-template <int WJN, int WIN>
-__global__ __launch_bounds__(64 * WJN * WIN) void k_acht_f64(const cplx *__restrict__ p2,
-                                                                    const cplx *__restrict__ aqsn,
-                                                                    const cplx *__restrict__ bg,
-                                                                    const int32_t *__restrict__ idx,
-                                                                    const double *__restrict__ vcoul, int ngpown,
-                                                                    int ncouls, int nb, int n1_begin, int n1_end,
-                                                                    int chunk, int nks, int jtiles,
-                                                                    cplx *__restrict__ part)
+// 1-D grid over (band tiles, j tiles, G-vector splits), band tiles fastest in
+// tile order and spread over the XCDs by xcd_tile, so the blocks that share one
+// R tile run on one XCD.  part: [jtiles * nks][nb].  CUT: the last j tile runs
+// one sub-tile row per wave.
+template <class C, bool CUT>
+__global__ __launch_bounds__(C::NT) __attribute__((amdgpu_waves_per_eu(C::OCC))) void k_acht_f64(
+    const cplx *__restrict__ p2, const cplx *__restrict__ aqsn, const cplx *__restrict__ bg,
+    const int32_t *__restrict__ idx, const double *__restrict__ vcoul, int ngpown, int ncouls, int nb, int n1_begin,
+    int n1_end, int chunk, int nks, int jtiles, cplx *__restrict__ part)
 {
-    typedef AchtCfg<WJN, WIN> C;
-    __shared__ cplx sR[2][2][C::TJ][kAK];
-    __shared__ cplx sA[2][2][C::TN][kAK];
-    __shared__ cplx red[WJN][C::TN];
-    const int nn = (n1_end - n1_begin + C::TN - 1) / C::TN;
-    const int t = xcd_tile(blockIdx.x, nn * jtiles * nks);
-    const int ct = t % nn, jt = (t / nn) % jtiles, ks = t / (nn * jtiles);
+    __shared__ cplx lds[C::LDS];
+    const int nn = (n1_end - n1_begin + C::TI - 1) / C::TI;
+    // CUT: the last j tile's blocks come after the others, filling the last round
+    const int nj = CUT ? jtiles - 1 : jtiles, full = nn * nj * nks, b = blockIdx.x;
+    const bool last = CUT && b >= full;
+    const int t = last ? xcd_tile(b - full, nn * nks) : xcd_tile(b, full);
+    const int ct = t % nn, jt = last ? nj : (t / nn) % nj, ks = last ? t / nn : t / (nn * nj);
     const int k_begin = ks * chunk;
     const int k_end = k_begin + chunk < ncouls ? k_begin + chunk : ncouls;
-    acht_f64_tile<WJN, WIN>(p2, aqsn, bg, idx, vcoul, ngpown, ncouls, n1_end, k_begin, k_end,
-                                  jt * C::TJ, n1_begin + ct * C::TN, sR, sA, red,
-                                  part + ((size_t)jt * nks + ks) * nb);
+    cplx *const out = part + ((size_t)jt * nks + ks) * nb;
+    if (last)
+        acht_ring_tile<C, 1>(p2, aqsn, bg, idx, vcoul, ngpown, ncouls, n1_end, k_begin, k_end, jt * C::TJ,
+                             n1_begin + ct * C::TI, lds, out);
+    else
+        acht_ring_tile<C, C::SJ>(p2, aqsn, bg, idx, vcoul, ngpown, ncouls, n1_end, k_begin, k_end, jt * C::TJ,
+                                 n1_begin + ct * C::TI, lds, out);
 }
 
 // Grid (ngpown, nsplit): the occupied bands' acht_n1_loc partials (where the
@@ -331,6 +371,14 @@ void launch_gram_ring(const DevProblem &p, const cplx *bg, cplx *mu, hipStream_t
     else
         hipLaunchKernelGGL((k_gram_f64<C, C::SJ>), dim3(tiles), dim3(C::NT), 0, s, bg, p.aqsn, p.ngpown, p.ncouls,
                            p.nv, p.nb, nts, mu);
+}
+
+template <class C, bool CUT>
+void launch_acht(const DevProblem &p, const AchtSplit &as, const cplx *p2, const cplx *bg, cplx *part, hipStream_t s)
+{
+    hipLaunchKernelGGL((k_acht_f64<C, CUT>), dim3((unsigned)as.ntiles * as.jtiles * as.nks), dim3(C::NT), 0, s, p2,
+                       p.aqsn, bg, p.idx, p.vcoul, p.ngpown, p.ncouls, p.nb, p.nv, p.nb, as.chunk, as.nks, as.jtiles,
+                       part);
 }
 
 // P2: also store the pole factor of frequency acht_iw and either sum the
@@ -417,11 +465,7 @@ int gram_tile_for(const DevProblem &p)
         const bool cut = rem > 0 && rem <= k.short_j;
         const double ni = (p.ncouls + k.ti - 1) / k.ti, sub = k.tj / 16 * (k.ti / 16);
         const double whole = ni * ((p.ngpown + k.tj - 1) / k.tj - (cut ? 1 : 0));
-        double rounds = ceil(whole / kGramCus);
-        if (cut) {  // two short tiles take the time of a whole one
-            const double over = ni / 2 - (rounds * kGramCus - whole);
-            if (over > 0) rounds += ceil(2 * over / kGramCus) / 2;
-        }
+        const double rounds = tile_rounds(whole, cut ? ni : 0);
         double us = rounds * sub * ksteps * (rounds <= 1 ? k.one : k.many);
         if (k.tile == kTileX) us += 1.2 * ceil(rounds / 2);  // the first loads of its ring, two blocks at a time
         if (us < best) best = us, tile = k.tile;
@@ -536,19 +580,23 @@ hipError_t run_factored(const DevProblem &p, GramKind kind, void *work, const De
         cplx *part = reinterpret_cast<cplx *>(w + L.acht_part);
         cplx *part_occ = reinterpret_cast<cplx *>(w + L.acht_occ);
         if (p.nb > p.nv) {
-            const unsigned n = (unsigned)((p.nb - p.nv + AchtU::TN - 1) / AchtU::TN) * as.jtiles * as.nks;
-            hipLaunchKernelGGL((k_acht_f64<2, 4>), dim3(n), dim3(AchtU::NT), 0, s, ra.p2, p.aqsn, bg, p.idx,
-                               p.vcoul, p.ngpown, p.ncouls, p.nb, p.nv, p.nb, as.chunk, as.nks, as.jtiles, part);
+            if (as.narrow)
+                as.cut ? launch_acht<GramM, true>(p, as, ra.p2, bg, part, s)
+                       : launch_acht<GramM, false>(p, as, ra.p2, bg, part, s);
+            else
+                as.cut ? launch_acht<GramL, true>(p, as, ra.p2, bg, part, s)
+                       : launch_acht<GramL, false>(p, as, ra.p2, bg, part, s);
             GPP_TRY(hipGetLastError());
         }
         if (p.nv > 0 && !occ_in_reduce) {  // else summed by the reduce
-            hipLaunchKernelGGL(k_acht_occ, dim3(p.ngpown, L.nsplit), dim3(kRedThreads), 0, s, ra.p2, ra.br1, p.aqsn,
-                               bg, p.idx, p.vcoul, p.ngpown, p.ncouls, p.nv, kind.red_chunk, L.nsplit, part_occ);
+            hipLaunchKernelGGL(k_acht_occ, dim3(p.ngpown, L.occ_nsplit), dim3(kRedThreads), 0, s, ra.p2, ra.br1,
+                               p.aqsn, bg, p.idx, p.vcoul, p.ngpown, p.ncouls, p.nv, L.occ_chunk, L.occ_nsplit,
+                               part_occ);
             GPP_TRY(hipGetLastError());
         }
         hipLaunchKernelGGL(k_acht_final, dim3((p.nb + kAchtFinalBands - 1) / kAchtFinalBands + p.nv), dim3(256), 0,
                            s, part, as.jtiles * as.nks, part_occ,
-                           p.ngpown * L.nsplit, p.nb, p.nv, res.acht_n1_loc());
+                           p.ngpown * L.occ_nsplit, p.nb, p.nv, res.acht_n1_loc());
         GPP_TRY(hipGetLastError());
         if (timer) timer->mark(s, "factored_acht");
     }

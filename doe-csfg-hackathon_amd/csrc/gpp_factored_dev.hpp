@@ -1118,108 +1118,89 @@ __device__ __forceinline__ void pole_cols_wave(const cplx *col_ach, const cplx *
 // P1 = sum rr ar, P2 = sum ri ai, P3 = sum (rr + ri)(ar + ai), Re Y = P1 - P2,
 // Im Y = (P3 - P1) - P2) and reduces it at once to the column sums
 // sum_j w_j conj(bg[n1][j]) Y[j][n1], written to part[n1] (one entry per
-// column of the tile).  Operand tiles are staged K-fastest in 128-byte rows
-// of 8 complex, element (row, k) at slot k ^ (row & 7): the stores (8 lanes
-// per row) and the MFMA reads (16 rows per 16 lanes) are then free of LDS
-// bank conflicts on gfx950 (measured with SQ_LDS_BANK_CONFLICT; a padded
-// pitch of 9 complex is not).  A stage is two such pieces of 8 G-vectors
-// (one barrier per 16), each loaded through registers during the previous
-// piece's MFMAs and stored to the other buffer right after them.
-constexpr int kAK = 8;          // G-vectors per LDS piece of the acht product
-constexpr int kAKS = 2 * kAK;   // per stage
-
-template <int WJN, int WIN> struct AchtCfg {
-    static constexpr int TJ = kWJ * WJN, TN = kWI * WIN, NT = 64 * WJN * WIN;
-};
-
-template <int WJN, int WIN>
-__device__ __forceinline__ void acht_f64_tile(const cplx *__restrict__ p2,
-                                              const cplx *__restrict__ aqsn, const cplx *__restrict__ bg,
-                                              const int32_t *__restrict__ idx, const double *__restrict__ vcoul,
-                                              int ngpown, int ncouls, int n1_end, int k_begin, int k_end, int j0,
-                                              int c0, cplx (*sR)[2][AchtCfg<WJN, WIN>::TJ][kAK],
-                                              cplx (*sA)[2][AchtCfg<WJN, WIN>::TN][kAK],
-                                              cplx (*red)[AchtCfg<WJN, WIN>::TN], cplx *__restrict__ part)
+// column of the tile).  The tile runs through the same ring of LDS stages as
+// gram_ring_tile (C::KS = 8 G-vectors a stage), both operands K-fastest: rows
+// of 8 complex (128 bytes), element (row, k) at slot k ^ (row & 7), which makes
+// the MFMA reads (16 rows per 16 lanes) free of LDS bank conflicts on gfx950
+// (a padded pitch of 9 complex is not); each lane of a stage's loads takes the
+// element its slot holds.  Bounded by the FP64 MFMA pipe, as the Gram product.
+// Rows and bands past the edge load the last one (their results are dropped),
+// G-vectors past the end the last one, counted as zero.  SJ <= C::SJ: sub-tile
+// rows per wave, fewer for a last tile with fewer rows.
+template <class C, int SJ>
+__device__ __forceinline__ void acht_ring_tile(const cplx *__restrict__ p2, const cplx *__restrict__ aqsn,
+                                               const cplx *__restrict__ bg, const int32_t *__restrict__ idx,
+                                               const double *__restrict__ vcoul, int ngpown, int ncouls, int n1_end,
+                                               int k_begin, int k_end, int j0, int c0, cplx *lds,
+                                               cplx *__restrict__ part)
 {
-    typedef AchtCfg<WJN, WIN> C;
-    constexpr int TJ = C::TJ, TN = C::TN, NT = C::NT;
-    constexpr int PR = kAK * TJ / NT, PA = kAK * TN / NT;
-    static_assert(PR * NT == kAK * TJ && PA * NT == kAK * TN, "stage must split evenly");
+    constexpr int KS = C::KS, NB = C::NB, TJ = C::TJ, TN = C::TI, SI = C::SI, NW = C::NW;
+    constexpr int QR = KS * TJ / 64 / NW, QA = KS * TN / 64 / NW, LD = QR + QA;  // loads per wave and stage
+    static_assert(KS == 8 && QR * 64 * NW == KS * TJ && QA * 64 * NW == KS * TN && NB >= 3,
+                  "rows of 8, loads split evenly over the waves");
     const int lane = threadIdx.x % kWave;
-    const int wave = threadIdx.x / kWave;
-    const int wjn = wave / WIN;
-    const int wj = wjn * kWJ;
-    const int wi = (wave % WIN) * kWI;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+    const int wjn = wave / C::WIN;
+    const int wj = wjn * (16 * SJ), wi = (wave % C::WIN) * (16 * SI);
+    const int nst = (k_end - k_begin + KS - 1) / KS;  // >= 1: a split is never empty
 
-    v4d acc1[4][2], acc2[4][2], acc3[4][2];  // P1, P2, P3
+    // Load q of a side fills rows [8 (q NW + wave), +8): lane l row l / 8,
+    // slot l % 8, so G-vector (l % 8) ^ (l / 8) of the stage.
+    const int lk = (lane % 8) ^ (lane / 8);
+    const cplx *pr[QR], *pa[QA];
 #pragma unroll
-    for (int s = 0; s < 4; ++s)
+    for (int q = 0; q < QR; ++q)
+        pr[q] = p2 + (size_t)min(j0 + 8 * (q * NW + wave) + lane / 8, ngpown - 1) * ncouls + k_begin + lk;
 #pragma unroll
-        for (int t = 0; t < 2; ++t) acc1[s][t] = acc2[s][t] = acc3[s][t] = v4d{0, 0, 0, 0};
-
-    cplx stR[PR], stA[PA];
-    auto load_piece = [&](int k0) {
+    for (int q = 0; q < QA; ++q)
+        pa[q] = aqsn + (size_t)min(c0 + 8 * (q * NW + wave) + lane / 8, n1_end - 1) * ncouls + k_begin + lk;
+    int ibuf = 0, rbuf = 0;  // next buffer to fill, to read
+    // over: how far this lane's G-vector lies past the end (last stage only)
+    auto issue = [&](int over) {
+        cplx *buf = lds + ibuf * C::STAGE + 64 * wave;
+        ibuf = ibuf + 1 == NB ? 0 : ibuf + 1;
 #pragma unroll
-        for (int q = 0; q < PR; ++q) {
-            const int e = threadIdx.x + q * NT;
-            const int r = e / kAK, k = k0 + e % kAK, j = j0 + r;
-            stR[q] = (k < k_end && j < ngpown) ? p2[(size_t)j * ncouls + k] : czero();
+        for (int q = 0; q < QR; ++q) {
+            ring_load(pr[q] - over, buf + 64 * NW * q);
+            pr[q] += KS;
         }
 #pragma unroll
-        for (int q = 0; q < PA; ++q) {
-            const int e = threadIdx.x + q * NT;
-            const int r = e / kAK, k = k0 + e % kAK, n1 = c0 + r;
-            stA[q] = (k < k_end && n1 < n1_end) ? aqsn[(size_t)n1 * ncouls + k] : czero();
+        for (int q = 0; q < QA; ++q) {
+            ring_load(pa[q] - over, buf + KS * TJ + 64 * NW * q);
+            pa[q] += KS;
         }
     };
-    auto store_piece = [&](int buf, int h) {
-#pragma unroll
-        for (int q = 0; q < PR; ++q) {
-            const int e = threadIdx.x + q * NT;
-            const int r = e / kAK;
-            sR[buf][h][r][(e % kAK) ^ (r & 7)] = stR[q];
-        }
-#pragma unroll
-        for (int q = 0; q < PA; ++q) {
-            const int e = threadIdx.x + q * NT;
-            const int r = e / kAK;
-            sA[buf][h][r][(e % kAK) ^ (r & 7)] = stA[q];
-        }
-    };
+    const int over_last = max(0, k_begin + (nst - 1) * KS + lk - (k_end - 1));
 
-    const int nst = (k_end - k_begin + kAKS - 1) / kAKS;
+    v4d acc1[SJ][SI], acc2[SJ][SI], acc3[SJ][SI];  // P1, P2, P3
 #pragma unroll
-    for (int h = 0; h < 2; ++h) {
-        load_piece(k_begin + h * kAK);
-        store_piece(0, h);
-    }
-    __syncthreads();
-    for (int st = 0; st < nst; ++st) {
-        const int buf = st & 1;
+    for (int s = 0; s < SJ; ++s)
 #pragma unroll
-        for (int h = 0; h < 2; ++h) {
-        if (st + 1 < nst) load_piece(k_begin + (st + 1) * kAKS + h * kAK);
-        // as in the Gram product: MFMA section first, fragment reads
-        // interleaved with the MFMAs (C1 2.823 -> 2.799 ms, C3 33.96 -> 33.66)
+        for (int t = 0; t < SI; ++t) acc1[s][t] = acc2[s][t] = acc3[s][t] = v4d{0, 0, 0, 0};
+    auto multiply = [&](auto last) {
+        const cplx *sR = lds + rbuf * C::STAGE, *sA = sR + KS * TJ;
+        rbuf = rbuf + 1 == NB ? 0 : rbuf + 1;
         __builtin_amdgcn_s_setprio(1);
-        __builtin_amdgcn_iglp_opt(1);
 #pragma unroll
-        for (int kk = 0; kk < kAK; kk += 4) {
+        for (int kk = 0; kk < KS; kk += 4) {
             const int kr = (kk + lane / 16) ^ (lane & 7);  // every row read below is = lane (mod 8)
-            double are[2], aim[2], asum[2];
+            const bool out = last && k_begin + (nst - 1) * KS + kk + lane / 16 >= k_end;
+            double are[SI], aim[SI], asum[SI];
 #pragma unroll
-            for (int t = 0; t < 2; ++t) {
-                const cplx a = sA[buf][h][wi + 16 * t + lane % 16][kr];
+            for (int t = 0; t < SI; ++t) {
+                cplx a = sA[(wi + 16 * t + lane % 16) * KS + kr];
+                if (out) a = czero();
                 are[t] = a.re;
                 aim[t] = a.im;
                 asum[t] = a.re + a.im;
             }
 #pragma unroll
-            for (int s = 0; s < 4; ++s) {
-                const cplx r = sR[buf][h][wj + 16 * s + lane % 16][kr];
+            for (int s = 0; s < SJ; ++s) {
+                cplx r = sR[(wj + 16 * s + lane % 16) * KS + kr];
+                if (out) r = czero();
                 const double rsum = r.re + r.im;
 #pragma unroll
-                for (int t = 0; t < 2; ++t) {
+                for (int t = 0; t < SI; ++t) {
                     acc1[s][t] = __builtin_amdgcn_mfma_f64_16x16x4f64(r.re, are[t], acc1[s][t], 0, 0, 0);
                     acc2[s][t] = __builtin_amdgcn_mfma_f64_16x16x4f64(r.im, aim[t], acc2[s][t], 0, 0, 0);
                     acc3[s][t] = __builtin_amdgcn_mfma_f64_16x16x4f64(rsum, asum[t], acc3[s][t], 0, 0, 0);
@@ -1227,43 +1208,70 @@ __device__ __forceinline__ void acht_f64_tile(const cplx *__restrict__ p2,
             }
         }
         __builtin_amdgcn_s_setprio(0);
-        if (st + 1 < nst) store_piece(buf ^ 1, h);
-        }
-        __syncthreads();
+    };
+    // the schedule of gram_ring_tile
+    for (int st = 0; st < NB - 1 && st < nst; ++st) issue(st < nst - 1 ? 0 : over_last);
+    int st = 0;
+    for (; st < nst - NB; ++st) {
+        wait_vm_lds<(NB - 2) * LD>();
+        ring_barrier();
+        issue(0);
+        multiply(std::integral_constant<bool, false>());
     }
+    if (nst >= NB) {
+        wait_vm_lds<(NB - 2) * LD>();
+        ring_barrier();
+        issue(over_last);
+        multiply(std::integral_constant<bool, false>());
+        ++st;
+    }
+    for (; st < nst - 1; ++st) {
+        wait_vm_lds<0>();
+        ring_barrier();
+        multiply(std::integral_constant<bool, false>());
+    }
+    wait_vm_lds<0>();
+    ring_barrier();
+    multiply(std::integral_constant<bool, true>());
 
     // Epilogue: result r of lane l is Y[j][n1] with j = 4r + l/16 + 16s + wj,
     // n1 = l%16 + 16t + wi.  Weight by 0.5 vcoul[igp(j)] conj(bg[n1][j]), sum
-    // the wave's 64 rows (fixed order: s, r, then the xor butterfly over
+    // the wave's 16 SJ rows (fixed order: s, r, then the xor butterfly over
     // l/16), then the WJN waves of one column range in wave order.
+    __syncthreads();  // every wave is done with the stages
+    auto *red = reinterpret_cast<cplx(*)[TN]>(lds);
+    cplx sum[SI];
 #pragma unroll
-    for (int t = 0; t < 2; ++t) {
-        const int col = wi + 16 * t + lane % 16;
-        const int n1 = c0 + col;
-        cplx sum = czero();
+    for (int t = 0; t < SI; ++t) sum[t] = czero();
 #pragma unroll
-        for (int s = 0; s < 4; ++s)
+    for (int s = 0; s < SJ; ++s)
 #pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const int j = j0 + wj + 16 * s + 4 * r + lane / 16;
-                if (j < ngpown && n1 < n1_end) {
-                    const double w = 0.5 * vcoul[igp_of(idx, j, ncouls)];
+        for (int r = 0; r < 4; ++r) {
+            const int j = j0 + wj + 16 * s + 4 * r + lane / 16;
+            if (j < ngpown) {
+                const double w = 0.5 * vcoul[igp_of(idx, j, ncouls)];
+#pragma unroll
+                for (int t = 0; t < SI; ++t) {
+                    const int n1 = min(c0 + wi + 16 * t + lane % 16, n1_end - 1);
                     const cplx b = bg[(size_t)n1 * ngpown + j];
                     const cplx y = cplx{acc1[s][t][r] - acc2[s][t][r], (acc3[s][t][r] - acc1[s][t][r]) - acc2[s][t][r]};
-                    sum = cadd(sum, cscale(cmul_fast(cconj(b), y), w));
+                    sum[t] = cadd(sum[t], cscale(cmul_fast(cconj(b), y), w));
                 }
             }
-        sum.re += __shfl_xor(sum.re, 16);
-        sum.im += __shfl_xor(sum.im, 16);
-        sum.re += __shfl_xor(sum.re, 32);
-        sum.im += __shfl_xor(sum.im, 32);
-        if (lane < 16) red[wjn][col] = sum;
+        }
+#pragma unroll
+    for (int t = 0; t < SI; ++t) {
+        sum[t].re += __shfl_xor(sum[t].re, 16);
+        sum[t].im += __shfl_xor(sum[t].im, 16);
+        sum[t].re += __shfl_xor(sum[t].re, 32);
+        sum[t].im += __shfl_xor(sum[t].im, 32);
+        if (lane < 16) red[wjn][wi + 16 * t + lane] = sum[t];
     }
     __syncthreads();
-    for (int col = threadIdx.x; col < TN; col += NT) {
+    for (int col = threadIdx.x; col < TN; col += C::NT) {
         cplx s = czero();
 #pragma unroll
-        for (int w = 0; w < WJN; ++w) s = cadd(s, red[w][col]);
+        for (int w2 = 0; w2 < C::WJN; ++w2) s = cadd(s, red[w2][col]);
         if (c0 + col < n1_end) part[c0 + col] = s;
     }
 }

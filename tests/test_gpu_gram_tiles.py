@@ -1,4 +1,4 @@
-"""The FP64 Gram tiles at the edges of their stages and tiles: every tile gives
+"""The FP64 Gram and acht products at the edges of their stages and tiles.  Every Gram tile gives
 the same bits (each Mu entry is the same sum in the same order), within 1e-10
 of the oracle.  Option 0 picks by size: the 16 x 16 tile for the first list, the
 32 x 64 one for the second."""
@@ -51,3 +51,29 @@ def test_gram_tiles_at_their_edges(ctx, oracle, shape):
     for tile in range(1, 4):
         for k in KEYS:
             np.testing.assert_array_equal(out[tile][k], out[0][k], err_msg=f"tile {tile} {k}")
+
+
+# nb, nv, ncouls, ngpown: G-vector stages of 8 against splits of at least 32,
+# tiles of 64 rows (a last one of at most 32 runs half) by 128 or 64 bands
+ACHT = [
+    (4, 2, 7, 5),        # one partial stage
+    (20, 3, 8, 8),
+    (67, 2, 33, 32),     # 65 bands: the wider tile's edge
+    (66, 2, 64, 33),     # 64 bands, 33 rows
+    (131, 3, 257, 65),   # 128 bands, a last tile of one row
+    (60, 0, 1000, 96),
+    (200, 8, 2100, 97),  # occupied bands by their own launch
+    (300, 3, 4100, 130),
+]
+
+
+@pytest.mark.parametrize("shape", ACHT, ids=lambda s: "x".join(map(str, s)))
+def test_acht_product_at_its_edges(ctx, oracle, shape):
+    """acht_n1_loc of the factored form against the oracle, bitwise repeatable."""
+    nb, nv, ncouls, ngpown = shape
+    arrs = gpp_inputs.seeded_inputs(nb, ncouls, min(ngpown, ncouls), seed=sum(shape) + 1)
+    ctx.upload(problem_of(arrs, nv), arrs)
+    out = ctx.sigma("factored-f64", acht_n1_loc=True)
+    assert_close(out, oracle.sigma(arrs, nvband=nv, threads=8), TOL_FACTORED, KEYS + ("acht_n1_loc",))
+    again = ctx.sigma("factored-f64", acht_n1_loc=True)
+    np.testing.assert_array_equal(out["acht_n1_loc"], again["acht_n1_loc"])
