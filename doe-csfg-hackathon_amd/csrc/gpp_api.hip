@@ -132,40 +132,46 @@ void Workspace::release()
     bytes = 0;
 }
 
-hipError_t StageTimer::init()
+hipError_t StageTimer::init(int device)
 {
-    for (int k = 0; k < kRing; ++k)
-        for (int i = 0; i <= kMax; ++i) {
-            hipError_t e = hipEventCreate(&slot[k].ev[i]);
-            if (e != hipSuccess) return e;
-        }
-    ready = true;
-    return hipSuccess;
+    hipError_t e = hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, device);
+    if (e != hipSuccess) return e;
+    if (khz <= 0) return hipErrorInvalidValue;
+    return hipMalloc(reinterpret_cast<void **>(&dev), sizeof(unsigned long long) * kRing * (kMax + 1));
 }
 
 void StageTimer::destroy()
 {
-    for (int k = 0; k < kRing; ++k)
-        for (int i = 0; i <= kMax; ++i)
-            if (slot[k].ev[i]) (void)hipEventDestroy(slot[k].ev[i]);
-    ready = false;
+    if (dev) (void)hipFree(dev);
+    dev = nullptr;
 }
 
-void StageTimer::begin(hipStream_t s)
+void StageTimer::begin()
 {
     if (filled > 0) cur = (cur + 1) % kRing;
     if (filled < kRing) ++filled;
     slot[cur].n = 0;
-    if (ready) (void)hipEventRecord(slot[cur].ev[0], s);
 }
 
-void StageTimer::mark(hipStream_t s, const char *nm)
+Stamp StageTimer::stage(const char *nm)
 {
     Slot &sl = slot[cur];
-    if (!ready || sl.n >= kMax) return;
+    if (!dev || sl.n >= kMax) return Stamp{};
     sl.name[sl.n] = nm;
-    (void)hipEventRecord(sl.ev[sl.n + 1], s);
+    const Stamp st{dev + cur * (kMax + 1) + sl.n, sl.n == 0 ? kMax : 0};
     ++sl.n;
+    return st;
+}
+
+hipError_t StageTimer::read(int k, double *total, double (&stage_ms)[kMax]) const
+{
+    const int i = (cur - k + kRing) % kRing, n = slot[i].n;
+    unsigned long long t[kMax + 1];
+    hipError_t e = hipMemcpy(t, dev + i * (kMax + 1), sizeof(unsigned long long) * (n + 1), hipMemcpyDeviceToHost);
+    if (e != hipSuccess) return e;
+    for (int q = 0; q < n; ++q) stage_ms[q] = (double)(t[q + 1] - t[q]) / khz;
+    *total = (double)(t[n] - t[0]) / khz;
+    return hipSuccess;
 }
 
 }  // namespace gpp
@@ -181,6 +187,8 @@ struct gpp_ctx {
     gpp::DevProblem dp;
     DevBuf idx, wx, vcoul, aqsm, aqsn, ieps, wtilde;  // owned inputs
     DevBuf results, flag;
+    cplx *host_results = nullptr;  // pinned, grow-only: a copy into pageable memory stages through the runtime
+    size_t host_results_cap = 0;
     gpp::Workspace work;
     gpp::StageTimer timer;
     bool timed = false;
@@ -314,7 +322,7 @@ gpp_status gpp_ctx_create(gpp_ctx **out, int device)
     e = hipSetDevice(device);
     if (e == hipSuccess) e = hipStreamCreateWithFlags(&ctx->own_stream, hipStreamNonBlocking);
     ctx->stream = ctx->own_stream;
-    if (e == hipSuccess) e = ctx->timer.init();
+    if (e == hipSuccess) e = ctx->timer.init(device);
     if (e != hipSuccess) {
         gpp_ctx_destroy(ctx);
         return fail_hip(e, "context setup");
@@ -332,6 +340,7 @@ gpp_status gpp_ctx_destroy(gpp_ctx *ctx)
     ctx->aqsm.release(); ctx->aqsn.release(); ctx->ieps.release(); ctx->wtilde.release();
     ctx->results.release(); ctx->flag.release(); ctx->wxb.release();
     ctx->work.release();
+    if (ctx->host_results) (void)hipHostFree(ctx->host_results);
     ctx->timer.destroy();
     if (ctx->own_stream) (void)hipStreamDestroy(ctx->own_stream);
     delete ctx;
@@ -805,15 +814,24 @@ gpp_status gpp_ctx_wait(gpp_ctx *ctx, const gpp_outputs *out)
         HIP_OR_FAIL(hipStreamSynchronize(ctx->stream), "sigma synchronize");
         return GPP_OK;
     }
-    std::vector<cplx> host(count);
-    HIP_OR_FAIL(hipMemcpyAsync(host.data(), ctx->results.ptr, sizeof(cplx) * count, hipMemcpyDeviceToHost,
+    if (count > ctx->host_results_cap) {
+        if (ctx->host_results) (void)hipHostFree(ctx->host_results);
+        ctx->host_results = nullptr;
+        ctx->host_results_cap = 0;
+        HIP_OR_FAIL(hipHostMalloc(reinterpret_cast<void **>(&ctx->host_results), sizeof(cplx) * count,
+                                  hipHostMallocDefault),
+                    "pinned results allocation");
+        ctx->host_results_cap = count;
+    }
+    const cplx *host = ctx->host_results;
+    HIP_OR_FAIL(hipMemcpyAsync(ctx->host_results, ctx->results.ptr, sizeof(cplx) * count, hipMemcpyDeviceToHost,
                                ctx->stream),
                 "D2H results");
     HIP_OR_FAIL(hipStreamSynchronize(ctx->stream), "sigma synchronize");
-    if (out->achtemp) memcpy(out->achtemp, host.data(), sizeof(cplx) * nf);
-    if (out->asxtemp) memcpy(out->asxtemp, host.data() + nf, sizeof(cplx) * nf);
-    if (out->acht_n1_loc) memcpy(out->acht_n1_loc, host.data() + 2 * nf, sizeof(cplx) * nb);
-    if (out->achstemp) memcpy(out->achstemp, host.data() + 2 * nf + nb, sizeof(cplx));
+    if (out->achtemp) memcpy(out->achtemp, host, sizeof(cplx) * nf);
+    if (out->asxtemp) memcpy(out->asxtemp, host + nf, sizeof(cplx) * nf);
+    if (out->acht_n1_loc) memcpy(out->acht_n1_loc, host + 2 * nf, sizeof(cplx) * nb);
+    if (out->achstemp) memcpy(out->achstemp, host + 2 * nf + nb, sizeof(cplx));
     return GPP_OK;
 }
 
@@ -927,14 +945,13 @@ gpp_status gpp_ctx_autotune(gpp_ctx *ctx, gpp_form form)
             HIP_OR_FAIL(gpp::run_factored(dp, k, ctx->work.ptr, res, ctx->stream, &ctx->timer), "autotune launch");
             HIP_OR_FAIL(hipStreamSynchronize(ctx->stream), "autotune synchronize");
             if (rep == 0) continue;  // warm-up
-            float ms = 0.f;
-            double g_ms = 0.0, r_ms = 0.0;
+            double g_ms = 0.0, r_ms = 0.0, total = 0.0, ms[gpp::StageTimer::kMax];
+            HIP_OR_FAIL(ctx->timer.read(0, &total, ms), "autotune stage times");
             const gpp::StageTimer::Slot &t = ctx->timer.last();
             for (int i = 0; i < t.n; ++i) {
-                HIP_OR_FAIL(hipEventElapsedTime(&ms, t.ev[i], t.ev[i + 1]), "hipEventElapsedTime");
-                if (strncmp(t.name[i], "factored_gram", 13) == 0) g_ms = ms;
+                if (strncmp(t.name[i], "factored_gram", 13) == 0) g_ms = ms[i];
                 if (strcmp(t.name[i], "factored_pole_reduce") == 0 || strcmp(t.name[i], "factored_pole_cols") == 0)
-                    r_ms = ms;
+                    r_ms = ms[i];
             }
             best_g = std::min(best_g, g_ms);
             best_r = std::min(best_r, r_ms);
@@ -978,14 +995,13 @@ gpp_status gpp_ctx_last_timing(const gpp_ctx *ctx, double *total_ms, double *sta
         if (nstages) *nstages = 0;
         return GPP_OK;
     }
-    HIP_OR_FAIL(hipEventSynchronize(t.ev[t.n]), "hipEventSynchronize");
-    float ms = 0.f;
-    HIP_OR_FAIL(hipEventElapsedTime(&ms, t.ev[0], t.ev[t.n]), "hipEventElapsedTime");
-    if (total_ms) *total_ms = ms;
-    for (int i = 0; i < t.n && stage_ms && i < max_stages; ++i) {
-        HIP_OR_FAIL(hipEventElapsedTime(&ms, t.ev[i], t.ev[i + 1]), "hipEventElapsedTime");
-        stage_ms[i] = ms;
-    }
+    gpp_status st = set_device(ctx);
+    if (st) return st;
+    HIP_OR_FAIL(hipStreamSynchronize(ctx->stream), "hipStreamSynchronize");
+    double total = 0.0, ms[gpp::StageTimer::kMax];
+    HIP_OR_FAIL(ctx->timer.read(0, &total, ms), "stage times");
+    if (total_ms) *total_ms = total;
+    for (int i = 0; i < t.n && stage_ms && i < max_stages; ++i) stage_ms[i] = ms[i];
     if (nstages) *nstages = t.n;
     return GPP_OK;
 }
@@ -1000,7 +1016,9 @@ gpp_status gpp_ctx_timing_summary(const gpp_ctx *ctx, int last_n, int *nevals, d
     if (avg_total_ms) *avg_total_ms = 0.0;
     if (nstages) *nstages = 0;
     if (!ctx->timed || L.n == 0) return GPP_OK;
-    HIP_OR_FAIL(hipEventSynchronize(L.ev[L.n]), "hipEventSynchronize");
+    gpp_status status = set_device(ctx);
+    if (status) return status;
+    HIP_OR_FAIL(hipStreamSynchronize(ctx->stream), "hipStreamSynchronize");
     const int want = std::min(last_n, tm.filled);
     double tot = 0.0, st[gpp::StageTimer::kMax] = {};
     int m = 0;
@@ -1009,13 +1027,10 @@ gpp_status gpp_ctx_timing_summary(const gpp_ctx *ctx, int last_n, int *nevals, d
         bool same = S.n == L.n;
         for (int i = 0; same && i < L.n; ++i) same = S.name[i] && strcmp(S.name[i], L.name[i]) == 0;
         if (!same) break;  // an evaluation of another kind: stop at it
-        float ms = 0.f;
-        HIP_OR_FAIL(hipEventElapsedTime(&ms, S.ev[0], S.ev[S.n]), "hipEventElapsedTime");
-        tot += ms;
-        for (int i = 0; i < S.n; ++i) {
-            HIP_OR_FAIL(hipEventElapsedTime(&ms, S.ev[i], S.ev[i + 1]), "hipEventElapsedTime");
-            st[i] += ms;
-        }
+        double total = 0.0, ms[gpp::StageTimer::kMax];
+        HIP_OR_FAIL(tm.read(k, &total, ms), "stage times");
+        tot += total;
+        for (int i = 0; i < S.n; ++i) st[i] += ms[i];
         ++m;
     }
     if (nevals) *nevals = m;

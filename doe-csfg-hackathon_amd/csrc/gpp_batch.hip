@@ -47,7 +47,8 @@ __global__ __launch_bounds__(256) void k_batch_ach_cols(const BInst *__restrict_
     const BInst &b = insts[blockIdx.y];
     const int j = blockIdx.x * blockDim.x + threadIdx.x;
     if (j < b.ngpown)
-        ach_col(b.ieps, b.idx, b.vcoul, b.ncouls, j, reinterpret_cast<AchCol *>(b.part_achs + ach_cols_entry(b.nb)));
+        reinterpret_cast<AchCol *>(b.part_achs + ach_cols_entry(b.nb))[j] =
+            ach_col(b.ieps, b.idx, b.vcoul, b.ncouls, j);
 }
 
 // One wave per (instance, band, column group) item.
@@ -59,8 +60,8 @@ __global__ __launch_bounds__(kRedThreads) void k_batch_achstemp(const BInst *__r
         const int2 it = items[w];
         const BInst &b = insts[it.x];  // it.y = band * kAchSplit + column group
         const AchCol *cols = reinterpret_cast<const AchCol *>(b.part_achs + ach_cols_entry(b.nb));
-        const cplx s = achstemp_band(b.aqsm, b.aqsn, cols, b.ncouls, b.ngpown, it.y / kAchSplit, it.y % kAchSplit,
-                                     b.bg);
+        const cplx s = achstemp_band(b.aqsm, b.aqsn, [&](int j) { return cols[j]; }, b.ncouls, b.ngpown,
+                                     it.y / kAchSplit, it.y % kAchSplit, b.bg);
         if (threadIdx.x % kWave == 0) b.part_achs[it.y] = s;
     }
 }

@@ -186,6 +186,50 @@ __device__ __forceinline__ cplx block_sum(cplx v, cplx *scratch)
     return r;
 }
 
+// Where a launch notes that its stage starts: the device's constant-rate clock,
+// written by the launch's first block.  clear: the later entries of the
+// evaluation to zero (the first stage's launch).  Stages run in stream order,
+// so the start of one is the end of the one before.  Events between the
+// launches took 6-10 us each (five stages: 33 of 65 us of an evaluation of
+// empty kernels).
+struct Stamp {
+    unsigned long long *at = nullptr;
+    int clear = 0;
+};
+// Reads the clock at a kernel's start; store() goes after the kernel's loads.
+// `tie`, a wave-uniform value of the kernel, passes through the reading, which
+// thereby happens before the value's uses.  wall_clock64() counts as a memory
+// write to the compiler, and so does a store at the start: either kept every
+// wave-uniform input out of scalar registers (the direct kernel took 146 VGPRs
+// instead of 117, one block less per CU).
+struct StampStart {
+    const Stamp &st;
+    unsigned long long t0;
+    __device__ __forceinline__ StampStart(const Stamp &s, int &tie) : st(s)
+    {
+        asm("s_memrealtime %0\n\ts_waitcnt lgkmcnt(0)" : "=&s"(t0), "+s"(tie));
+    }
+    __device__ __forceinline__ void store() const
+    {
+        if (st.at && threadIdx.x == 0 && blockIdx.x == 0 && blockIdx.y == 0 && blockIdx.z == 0) {
+            st.at[0] = t0;
+            for (int i = 1; i <= st.clear; ++i) st.at[i] = 0;
+        }
+    }
+};
+__device__ __forceinline__ void stamp_start(const Stamp &st)
+{
+    if (st.at && threadIdx.x == 0 && blockIdx.x == 0 && blockIdx.y == 0 && blockIdx.z == 0) {
+        st.at[0] = wall_clock64();
+        for (int i = 1; i <= st.clear; ++i) st.at[i] = 0;
+    }
+}
+// The end of the evaluation: the latest block of its last launch.
+__device__ __forceinline__ void stamp_end(unsigned long long *at)
+{
+    if (at && threadIdx.x == 0) atomicMax(at, wall_clock64());
+}
+
 constexpr double kTo1 = 1e-6;    // to1, gppComplex.cpp:20, :241
 constexpr double kSexcut = 4.0;  // sexcut, gppComplex.cpp:21, :243
 
@@ -275,11 +319,6 @@ __host__ __device__ inline size_t ach_region_entries(int nb, int ngpown)
     return ach_cols_entry(nb) + 2 * (size_t)ngpown;
 }
 
-__device__ __forceinline__ void ach_col(const cplx *ieps, const int32_t *idx, const double *vcoul, int ncouls, int j,
-                                        AchCol *cols);
-__device__ __forceinline__ cplx achstemp_band(const cplx *aqsm, const cplx *aqsn, const AchCol *cols, int ncouls,
-                                               int ngpown, int n1, int q, cplx *bg);
-
 // igp = min(inv_igp_index[j], ncouls-1), gppComplex.cpp:342-344.  Negative
 // entries are rejected before any launch; the max(.,0) only keeps a kernel
 // in bounds should one slip through.
@@ -290,17 +329,18 @@ __device__ __forceinline__ int igp_of(const int32_t *idx, int j, int ncouls)
     return igp < 0 ? 0 : igp;
 }
 
-__device__ __forceinline__ void ach_col(const cplx *ieps, const int32_t *idx, const double *vcoul, int ncouls, int j,
-                                        AchCol *cols)
+__device__ __forceinline__ AchCol ach_col(const cplx *ieps, const int32_t *idx, const double *vcoul, int ncouls, int j)
 {
     const int igp = igp_of(idx, j, ncouls);
     const cplx ie = ieps[(size_t)j * ncouls + igp];
     const cplx schs = cplx{-ie.re, -ie.im};  // :86-88
     const bool keep = cabs_(schs) > kTo1;    // :91
-    cols[j] = AchCol{keep ? schs.re : 0.0, keep ? schs.im : 0.0, vcoul[igp] * 0.5, igp, 0};
+    return AchCol{keep ? schs.re : 0.0, keep ? schs.im : 0.0, vcoul[igp] * 0.5, igp, 0};
 }
 
-__device__ __forceinline__ cplx achstemp_band(const cplx *aqsm, const cplx *aqsn, const AchCol *cols, int ncouls,
+// col(j): column j's AchCol, read from the table or formed.
+template <class Col>
+__device__ __forceinline__ cplx achstemp_band(const cplx *aqsm, const cplx *aqsn, const Col &col, int ncouls,
                                                int ngpown, int n1, int q, cplx *bg)
 {
     cplx s = czero();
@@ -308,7 +348,7 @@ __device__ __forceinline__ cplx achstemp_band(const cplx *aqsm, const cplx *aqsn
     // scattered aqsm / aqsn elements) in flight per lane
 #pragma unroll 4
     for (int j = q * kWave + threadIdx.x % kWave; j < ngpown; j += kAchSplit * kWave) {
-        const AchCol c = cols[j];
+        const AchCol c = col(j);
         const cplx m = aqsm[(size_t)n1 * ncouls + c.igp];
         if (bg) bg[(size_t)n1 * ngpown + j] = m;
         if (c.sre != 0.0 || c.sim != 0.0) {  // |schs| > to1: schs is nonzero

@@ -46,6 +46,8 @@ struct DirectArgs {
     cplx *band_ach;   // [nb][nfreq]
     cplx *band_asx;   // [max(nv,1)][nfreq]
     cplx *bg;         // optional gathered rows of aqsm (factored forms), else null
+    Stamp stamp;      // the launch's stage start
+    unsigned long long *end;  // the evaluation's end (last launch)
 };
 
 struct WorkLayout {
@@ -85,6 +87,7 @@ DirectArgs make_args(const DevProblem &p, void *work)
     a.band_ach = reinterpret_cast<cplx *>(w + L.band_ach);
     a.band_asx = reinterpret_cast<cplx *>(w + L.band_asx);
     a.bg = nullptr;
+    a.end = nullptr;
     return a;
 }
 
@@ -143,6 +146,8 @@ __global__ __launch_bounds__(kNW *kWave) void k_unocc(DirectArgs a)
 {
     constexpr int TILE = kBJ * kWave;  // (column, G-vector) positions per chunk
     static_assert(TILE <= kNW * kWave, "one position per staging thread");
+    int ncouls = a.ncouls;
+    const StampStart stamp(a.stamp, ncouls);
     __shared__ cplx s_wt[2][kBJ][kWave];
     __shared__ cplx s_ie[2][kBJ][kWave];  // I_eps (strict) or wtilde * I_eps (fast)
 
@@ -153,7 +158,6 @@ __global__ __launch_bounds__(kNW *kWave) void k_unocc(DirectArgs a)
     const int jt = blockIdx.y;
     const int j0 = jt * kBJ;
     const int iw0 = blockIdx.z * FC;
-    const int ncouls = a.ncouls;
 
     // conj(aqsm[n1, igp(j)]) per column (mygpvar1, gppComplex.cpp:134).
     cplx cm[kBJ];
@@ -230,6 +234,7 @@ __global__ __launch_bounds__(kNW *kWave) void k_unocc(DirectArgs a)
         }
         if (lane == 0 && iw0 + f < a.nfreq) a.part_ach[((size_t)n1 * a.njt + jt) * a.nfreq + iw0 + f] = s;
     }
+    stamp.store();
 }
 
 // ---------------------------------------------------------------------------
@@ -240,6 +245,8 @@ __global__ __launch_bounds__(kNW *kWave) void k_unocc(DirectArgs a)
 template <int FC>
 __global__ __launch_bounds__(kOccWaves *kWave) void k_occ(DirectArgs a)
 {
+    int ncouls = a.ncouls;
+    const StampStart stamp(a.stamp, ncouls);
     __shared__ cplx s_ach[kBJ][FC];
     __shared__ cplx s_asx[kBJ][FC];
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
@@ -247,7 +254,6 @@ __global__ __launch_bounds__(kOccWaves *kWave) void k_occ(DirectArgs a)
     const int jt = blockIdx.x;
     const int n1 = blockIdx.y;
     const int iw0 = blockIdx.z * FC;
-    const int ncouls = a.ncouls;
 
     double wxv[FC], wx2[FC], rwx4[FC];
 #pragma unroll
@@ -320,35 +326,49 @@ __global__ __launch_bounds__(kOccWaves *kWave) void k_occ(DirectArgs a)
         a.part_ach[o] = sa;
         a.part_asx[o] = sx;
     }
+    stamp.store();
 }
 
 // ---------------------------------------------------------------------------
 // achstemp per band, reduce_achstemp (gppComplex.cpp:66-101): one wave per
 // band and block, so that the few hundred bands spread over every CU.
+// With COLS the columns' entries come from the table k_ach_cols wrote, without
+// it each wave forms them itself (one launch instead of two).
 constexpr int kAchWaves = 1;
+template <bool COLS>
 __global__ __launch_bounds__(kAchWaves * kWave) void k_achstemp(DirectArgs a)
 {
+    if (!COLS) stamp_start(a.stamp);
     const int item = blockIdx.x * kAchWaves + threadIdx.x / kWave;  // band * kAchSplit + column group
     if (item >= a.nb * kAchSplit) return;
     const AchCol *cols = reinterpret_cast<const AchCol *>(a.part_achs + ach_cols_entry(a.nb));
-    const cplx s = achstemp_band(a.aqsm, a.aqsn, cols, a.ncouls, a.ngpown, item / kAchSplit, item % kAchSplit, a.bg);
+    const auto col = [&](int j) { return COLS ? cols[j] : ach_col(a.ieps, a.idx, a.vcoul, a.ncouls, j); };
+    const cplx s = achstemp_band(a.aqsm, a.aqsn, col, a.ncouls, a.ngpown, item / kAchSplit, item % kAchSplit, a.bg);
     if (threadIdx.x % kWave == 0) a.part_achs[item] = s;
 }
 
 __global__ __launch_bounds__(256) void k_ach_cols(DirectArgs a)
 {
+    stamp_start(a.stamp);
     const int j = blockIdx.x * blockDim.x + threadIdx.x;
     if (j < a.ngpown)
-        ach_col(a.ieps, a.idx, a.vcoul, a.ncouls, j, reinterpret_cast<AchCol *>(a.part_achs + ach_cols_entry(a.nb)));
+        reinterpret_cast<AchCol *>(a.part_achs + ach_cols_entry(a.nb))[j] =
+            ach_col(a.ieps, a.idx, a.vcoul, a.ncouls, j);
 }
 
-// The columns' achstemp entries, then the (band, column group) partials (and
-// the Bg gather when a.bg is set).
+// The (band, column group) partials (and the Bg gather when a.bg is set), after
+// the columns' entries where forming them once saves more than their launch
+// costs: at 512 bands x 1638 columns the two launches take 33 us and the one
+// takes 50, at 512 x 40 the one saves a launch of 4-5 us.
 hipError_t launch_ach(const DirectArgs &a, hipStream_t s)
 {
-    if (a.ngpown > 0) hipLaunchKernelGGL(k_ach_cols, dim3((a.ngpown + 255) / 256), dim3(256), 0, s, a);
-    hipLaunchKernelGGL(k_achstemp, dim3((a.nb * kAchSplit + kAchWaves - 1) / kAchWaves), dim3(kAchWaves * kWave), 0, s,
-                       a);
+    const dim3 grid((a.nb * kAchSplit + kAchWaves - 1) / kAchWaves), block(kAchWaves * kWave);
+    if ((long long)a.nb * a.ngpown > (1 << 18)) {
+        hipLaunchKernelGGL(k_ach_cols, dim3((a.ngpown + 255) / 256), dim3(256), 0, s, a);
+        hipLaunchKernelGGL((k_achstemp<true>), grid, block, 0, s, a);
+    } else {
+        hipLaunchKernelGGL((k_achstemp<false>), grid, block, 0, s, a);
+    }
     return hipGetLastError();
 }
 
@@ -402,6 +422,7 @@ __global__ __launch_bounds__(kReduceThreads) void k_reduce_final(DirectArgs a, c
         for (int t = threadIdx.x; t < a.nb * kAchSplit; t += blockDim.x) h = cadd(h, a.part_achs[t]);
     h = block_sum(h, scratch);
     if (threadIdx.x == 0) out[2 * nf + a.nb] = h;
+    stamp_end(a.end);
 }
 
 __global__ void k_zero_ints(int *p, int n)
@@ -495,21 +516,20 @@ size_t direct_workspace_bytes(const DevProblem &p) { return layout_for(p).total;
 hipError_t run_direct(const DevProblem &p, bool strict, void *work, const DevResults &res,
                       hipStream_t s, StageTimer *timer)
 {
-    const DirectArgs a = make_args(p, work);
-    if (timer) timer->begin(s);
+    DirectArgs a = make_args(p, work);
+    const auto stage = [&](const char *nm) { a.stamp = timer ? timer->stage(nm) : Stamp{}; };
+    if (timer) timer->begin();
+    if (p.nv > 0) stage("direct_occupied");
     GPP_TRY(launch_occ(a, s));
-    if (timer) timer->mark(s, "direct_occupied");
+    if (p.nb > p.nv) stage(strict ? "direct_unoccupied_strict" : "direct_unoccupied");
     GPP_TRY(launch_unocc(a, strict, s));
-    if (timer) timer->mark(s, strict ? "direct_unoccupied_strict" : "direct_unoccupied");
-    if (p.nb > 0) {
-        GPP_TRY(launch_ach(a, s));
-        hipLaunchKernelGGL(k_reduce_bands, dim3(p.nb), dim3(kReduceThreads), 0, s, a, 0);
-        GPP_TRY(hipGetLastError());
-    }
-    hipLaunchKernelGGL(k_reduce_final, dim3(1), dim3(kReduceThreads), 0, s, a, res.base, 0, p.nb, 1);
+    stage("direct_reduce");
+    GPP_TRY(launch_ach(a, s));
+    hipLaunchKernelGGL(k_reduce_bands, dim3(p.nb), dim3(kReduceThreads), 0, s, a, 0);
     GPP_TRY(hipGetLastError());
-    if (timer) timer->mark(s, "direct_reduce");
-    return hipSuccess;
+    if (timer) a.end = timer->end();
+    hipLaunchKernelGGL(k_reduce_final, dim3(1), dim3(kReduceThreads), 0, s, a, res.base, 0, p.nb, 1);
+    return hipGetLastError();
 }
 
 hipError_t run_direct_part(const DevProblem &p, int which, void *work, const DevResults &res,
@@ -537,12 +557,12 @@ hipError_t run_direct_part(const DevProblem &p, int which, void *work, const Dev
     return hipGetLastError();
 }
 
-hipError_t launch_achstemp(const DevProblem &p, cplx *part_achs, cplx *bg, hipStream_t s)
+hipError_t launch_achstemp(const DevProblem &p, cplx *part_achs, cplx *bg, Stamp stamp, hipStream_t s)
 {
-    if (p.nb <= 0) return hipSuccess;
     DirectArgs a = make_args(p, nullptr);
     a.part_achs = part_achs;
     a.bg = bg;
+    a.stamp = stamp;
     return launch_ach(a, s);
 }
 

@@ -158,8 +158,9 @@ FactLayout fact_layout(const DevProblem &p, const GramKind &k)
 template <class C, int SJR>
 __global__ __launch_bounds__(C::NT) __attribute__((amdgpu_waves_per_eu(C::OCC))) void k_gram_f64(
     const cplx *__restrict__ bg, const cplx *__restrict__ aqsn, int ngpown, int ncouls, int k_begin, int k_end,
-    bool nts, cplx *__restrict__ mout)
+    bool nts, cplx *__restrict__ mout, Stamp stamp)
 {
+    stamp_start(stamp);
     __shared__ cplx lds[C::LDS];
     const int nj = (ngpown + C::TJ - 1) / C::TJ, ni = (ncouls + C::TI - 1) / C::TI;
     if constexpr (SJR == C::SJ) {
@@ -184,8 +185,9 @@ __global__ __launch_bounds__(C::NT) __attribute__((amdgpu_waves_per_eu(C::OCC)))
 // 16 x 16 tiles, three waves each (gram_small_product); same tile order.
 __global__ __launch_bounds__(kSmThreads) void k_gram_small(const cplx *__restrict__ bg, const cplx *__restrict__ aqsn,
                                                            int ngpown, int ncouls, int k_begin, int k_end,
-                                                           cplx *__restrict__ mout)
+                                                           cplx *__restrict__ mout, Stamp stamp)
 {
+    stamp_start(stamp);
     // one array (with a second one the compiler waits for every outstanding
     // load before each fragment read): the stages, then P2 and P3
     __shared__ cplx lds[kSmBuf * kSmStage];
@@ -228,6 +230,7 @@ __global__ __launch_bounds__(kSmThreads) void k_gram_small(const cplx *__restric
 template <int F>
 __global__ __launch_bounds__(512, 1) void k_gram_pole(PoleTileArgs a)
 {
+    stamp_start(a.stamp);
     typedef FuseCfg C;
     __shared__ cplx lds[FuseLds<F>::kLds];
     auto *sB = reinterpret_cast<cplx(*)[C::KS][C::TJ]>(lds);
@@ -244,8 +247,9 @@ __global__ __launch_bounds__(512, 1) void k_gram_pole(PoleTileArgs a)
 // One wave per column: the fused epilogue's tile sums, summed and scaled.
 __global__ __launch_bounds__(256) void k_pole_cols(const cplx *col_ach, const cplx *col_asx, int nsplit, int nfreq,
                                                    const int32_t *idx, const double *vcoul, int ncouls, int ngpown,
-                                                   double occ, cplx *out_ach, cplx *out_asx)
+                                                   double occ, cplx *out_ach, cplx *out_asx, Stamp stamp)
 {
+    stamp_start(stamp);
     const int j = blockIdx.x * (blockDim.x / kWave) + threadIdx.x / kWave;
     if (j < ngpown) pole_cols_wave(col_ach, col_asx, nsplit, nfreq, idx, vcoul, ncouls, occ, j, out_ach, out_asx);
 }
@@ -266,18 +270,24 @@ __global__ __launch_bounds__(256) void k_pole_cols(const cplx *col_ach, const cp
 template <int FC, int NV, bool P2, bool NEG = false>
 __global__ __launch_bounds__(kRedThreads, (FC <= 3 && !P2 && !NEG) ? 4 : FC > 8 || (NEG && FC > 4) ? 2 : 3) void k_pole_reduce(ReduceArgs a)
 {
+    int fpb = a.fpb;
+    const StampStart stamp(a.stamp, fpb);
     __shared__ cplx scratch[kRedThreads / kWave];
-    const int iw_begin = blockIdx.z * a.fpb;
-    const int iw_end = iw_begin + a.fpb < a.nfreq ? iw_begin + a.fpb : a.nfreq;
+    const int iw_begin = blockIdx.z * fpb;
+    const int iw_end = iw_begin + fpb < a.nfreq ? iw_begin + fpb : a.nfreq;
     pole_reduce_item<FC, NV, P2, (FC > 4 ? 4 : FC), NEG>(a, blockIdx.x, blockIdx.y, iw_begin, iw_end, scratch);
+    stamp.store();
 }
 
 __global__ __launch_bounds__(kRedThreads) void k_fact_final(const cplx *col_ach, const cplx *col_asx,
                                                             const cplx *part_achs, int ncols, int nfreq, int nb,
-                                                            int nv, cplx *out)
+                                                            int nv, cplx *out, Stamp stamp,
+                                                            unsigned long long *end)
 {
+    stamp_start(stamp);
     __shared__ cplx scratch[kRedThreads / kWave];
     final_block(col_ach, col_asx, part_achs, ncols, nfreq, nb, nv, out, scratch, blockIdx.x);
+    stamp_end(end);
 }
 
 // 1-D grid over (band tiles, j tiles, G-vector splits), band tiles fastest in
@@ -288,8 +298,9 @@ template <class C, bool CUT>
 __global__ __launch_bounds__(C::NT) __attribute__((amdgpu_waves_per_eu(C::OCC))) void k_acht_f64(
     const cplx *__restrict__ p2, const cplx *__restrict__ aqsn, const cplx *__restrict__ bg,
     const int32_t *__restrict__ idx, const double *__restrict__ vcoul, int ngpown, int ncouls, int nb, int n1_begin,
-    int n1_end, int chunk, int nks, int jtiles, cplx *__restrict__ part)
+    int n1_end, int chunk, int nks, int jtiles, cplx *__restrict__ part, Stamp stamp)
 {
+    stamp_start(stamp);
     __shared__ cplx lds[C::LDS];
     const int nn = (n1_end - n1_begin + C::TI - 1) / C::TI;
     // CUT: the last j tile's blocks come after the others, filling the last round
@@ -315,8 +326,10 @@ __global__ __launch_bounds__(kRedThreads) void k_acht_occ(const cplx *__restrict
                                                           const cplx *__restrict__ aqsn, const cplx *__restrict__ bg,
                                                           const int32_t *__restrict__ idx,
                                                           const double *__restrict__ vcoul, int ngpown, int ncouls,
-                                                          int nv, int chunk, int nsplit, cplx *__restrict__ part_occ)
+                                                          int nv, int chunk, int nsplit, cplx *__restrict__ part_occ,
+                                                          Stamp stamp)
 {
+    stamp_start(stamp);
     __shared__ cplx scratch[kRedThreads / kWave];
     acht_occ_item(p2, br1, aqsn, bg, idx, vcoul, ngpown, ncouls, nv, chunk, blockIdx.x, blockIdx.y,
                   part_occ + ((size_t)blockIdx.x * nsplit + blockIdx.y) * nv, scratch);
@@ -330,7 +343,7 @@ __global__ __launch_bounds__(kRedThreads) void k_acht_occ(const cplx *__restrict
 constexpr int kAchtFinalBands = 16;
 __global__ __launch_bounds__(256) void k_acht_final(const cplx *__restrict__ part, int nparts,
                                                     const cplx *__restrict__ part_occ, int nparts_occ, int nb,
-                                                    int nv, cplx *__restrict__ out)
+                                                    int nv, cplx *__restrict__ out, unsigned long long *end)
 {
     __shared__ cplx grp[256 / kAchtFinalBands][kAchtFinalBands];
     const int nblk = (nb + kAchtFinalBands - 1) / kAchtFinalBands;
@@ -357,28 +370,30 @@ __global__ __launch_bounds__(256) void k_acht_final(const cplx *__restrict__ par
         s = block_sum(s, &grp[0][0]);
         if (threadIdx.x == 0) out[n1] = s;
     }
+    stamp_end(end);
 }
 
 template <class C>
-void launch_gram_ring(const DevProblem &p, const cplx *bg, cplx *mu, hipStream_t s)
+void launch_gram_ring(const DevProblem &p, const cplx *bg, cplx *mu, Stamp stamp, hipStream_t s)
 {
     const unsigned tiles = (unsigned)((p.ngpown + C::TJ - 1) / C::TJ) * (unsigned)((p.ncouls + C::TI - 1) / C::TI);
     const bool nts = mu_streams(p);
     const int rem = p.ngpown % C::TJ;
     if (C::SJ == 2 && rem > 0 && rem <= 16 * C::WJN)
         hipLaunchKernelGGL((k_gram_f64<C, 1>), dim3(tiles), dim3(C::NT), 0, s, bg, p.aqsn, p.ngpown, p.ncouls, p.nv,
-                           p.nb, nts, mu);
+                           p.nb, nts, mu, stamp);
     else
         hipLaunchKernelGGL((k_gram_f64<C, C::SJ>), dim3(tiles), dim3(C::NT), 0, s, bg, p.aqsn, p.ngpown, p.ncouls,
-                           p.nv, p.nb, nts, mu);
+                           p.nv, p.nb, nts, mu, stamp);
 }
 
 template <class C, bool CUT>
-void launch_acht(const DevProblem &p, const AchtSplit &as, const cplx *p2, const cplx *bg, cplx *part, hipStream_t s)
+void launch_acht(const DevProblem &p, const AchtSplit &as, const cplx *p2, const cplx *bg, cplx *part, Stamp stamp,
+                 hipStream_t s)
 {
     hipLaunchKernelGGL((k_acht_f64<C, CUT>), dim3((unsigned)as.ntiles * as.jtiles * as.nks), dim3(C::NT), 0, s, p2,
                        p.aqsn, bg, p.idx, p.vcoul, p.ngpown, p.ncouls, p.nb, p.nv, p.nb, as.chunk, as.nks, as.jtiles,
-                       part);
+                       part, stamp);
 }
 
 // P2: also store the pole factor of frequency acht_iw and either sum the
@@ -473,20 +488,20 @@ int gram_tile_for(const DevProblem &p)
     return tile;
 }
 
-hipError_t launch_gram_f64(const DevProblem &p, int tile, const cplx *bg, cplx *mu, hipStream_t s)
+hipError_t launch_gram_f64(const DevProblem &p, int tile, const cplx *bg, cplx *mu, Stamp stamp, hipStream_t s)
 {
     // GPP_OPT_GRAM_TILE: 0 by size, then the ring tiles
     static const int kinds[kGramTiles] = {-1, kTileL, kTileLt, kTileM};
     if (tile < 0 || tile >= kGramTiles) return hipErrorInvalidValue;
     switch (tile == 0 ? gram_tile_for(p) : kinds[tile]) {
-    case kTileL: launch_gram_ring<GramL>(p, bg, mu, s); break;
-    case kTileLt: launch_gram_ring<GramLt>(p, bg, mu, s); break;
-    case kTileM: launch_gram_ring<GramM>(p, bg, mu, s); break;
-    case kTileS: launch_gram_ring<GramS>(p, bg, mu, s); break;
+    case kTileL: launch_gram_ring<GramL>(p, bg, mu, stamp, s); break;
+    case kTileLt: launch_gram_ring<GramLt>(p, bg, mu, stamp, s); break;
+    case kTileM: launch_gram_ring<GramM>(p, bg, mu, stamp, s); break;
+    case kTileS: launch_gram_ring<GramS>(p, bg, mu, stamp, s); break;
     default: {
         const unsigned tiles = (unsigned)((p.ngpown + 15) / 16) * (unsigned)((p.ncouls + 15) / 16);
         hipLaunchKernelGGL(k_gram_small, dim3(tiles), dim3(kSmThreads), 0, s, bg, p.aqsn, p.ngpown, p.ncouls, p.nv,
-                           p.nb, mu);
+                           p.nb, mu, stamp);
         break;
     }
     }
@@ -512,7 +527,7 @@ hipError_t launch_pole_reduce(const ReduceArgs &ra, int red_fc, hipStream_t s)
 }
 
 hipError_t run_factored(const DevProblem &p, GramKind kind, void *work, const DevResults &res, hipStream_t s,
-                        StageTimer *timer)
+                        StageTimer *timer, Stamp first)
 {
     if (p.wx_stride != 0) return hipErrorInvalidValue;  // the band sum factors only for a shared wx row
     const FactLayout L = fact_layout(p, kind);
@@ -523,39 +538,38 @@ hipError_t run_factored(const DevProblem &p, GramKind kind, void *work, const De
     cplx *col_asx = reinterpret_cast<cplx *>(w + L.col_asx);
     cplx *part_achs = reinterpret_cast<cplx *>(w + L.part_achs);
 
-    if (timer) timer->begin(s);
-    GPP_TRY(launch_achstemp(p, part_achs, bg, s));  // also gathers Bg
-    if (timer) timer->mark(s, "factored_gather_achstemp");
+    const auto stage = [&](const char *nm) { return timer ? timer->stage(nm) : Stamp{}; };
+    const auto end = [&]() { return timer ? timer->end() : nullptr; };
+    if (timer) timer->begin();
+    // also gathers Bg
+    GPP_TRY(launch_achstemp(p, part_achs, bg, timer ? stage("factored_gather_achstemp") : first, s));
     if (L.fused) {
         PoleTileArgs pa;
         pa.aqsn = p.aqsn; pa.ieps = p.ieps; pa.wtilde = p.wtilde; pa.bg = bg; pa.wx = p.wx;
         pa.nb = p.nb; pa.nv = p.nv; pa.ncouls = p.ncouls; pa.ngpown = p.ngpown; pa.nsplit = L.nsplit;
         pa.col_ach = col_ach; pa.col_asx = col_asx;
+        pa.stamp = stage("factored_gram_pole");
         switch (p.nfreq) {
         case 1: launch_gram_pole_f<1>(p, pa, s); break;
         case 2: launch_gram_pole_f<2>(p, pa, s); break;
         default: launch_gram_pole_f<3>(p, pa, s); break;
         }
         GPP_TRY(hipGetLastError());
-        if (timer) timer->mark(s, "factored_gram_pole");
         cplx *c2a = reinterpret_cast<cplx *>(w + L.col2_ach);
         cplx *c2x = reinterpret_cast<cplx *>(w + L.col2_asx);
         hipLaunchKernelGGL(k_pole_cols, dim3((p.ngpown + 3) / 4), dim3(256), 0, s, col_ach, col_asx, L.nsplit,
-                           p.nfreq, p.idx, p.vcoul, p.ncouls, p.ngpown, p.occ, c2a, c2x);
+                           p.nfreq, p.idx, p.vcoul, p.ncouls, p.ngpown, p.occ, c2a, c2x, stage("factored_pole_cols"));
         GPP_TRY(hipGetLastError());
-        if (timer) timer->mark(s, "factored_pole_cols");
+        const Stamp st = stage("factored_final");
         hipLaunchKernelGGL(k_fact_final, dim3(p.nfreq + 1), dim3(kRedThreads), 0, s, c2a, c2x, part_achs, p.ngpown,
-                           p.nfreq, p.nb, p.nv, res.base);
-        GPP_TRY(hipGetLastError());
-        if (timer) timer->mark(s, "factored_final");
-        return hipSuccess;
+                           p.nfreq, p.nb, p.nv, res.base, st, end());
+        return hipGetLastError();
     }
     if (kind.ozaki_slices) {
-        GPP_TRY(launch_gram_ozaki(p, kind.ozaki_slices, kind.int8, kind.layout, kind.group, bg, w + L.total, mu, s));
-        if (timer) timer->mark(s, kind.int8 ? "factored_gram_ozaki_i8" : "factored_gram_ozaki");
+        GPP_TRY(launch_gram_ozaki(p, kind.ozaki_slices, kind.int8, kind.layout, kind.group, bg, w + L.total, mu,
+                                  stage(kind.int8 ? "factored_gram_ozaki_i8" : "factored_gram_ozaki"), s));
     } else {
-        GPP_TRY(launch_gram_f64(p, kind.tile, bg, mu, s));
-        if (timer) timer->mark(s, "factored_gram_f64");
+        GPP_TRY(launch_gram_f64(p, kind.tile, bg, mu, stage("factored_gram_f64"), s));
     }
     ReduceArgs ra;
     ra.mu = mu; ra.ieps = p.ieps; ra.wtilde = p.wtilde; ra.aqsn = p.aqsn; ra.bg = bg; ra.idx = p.idx;
@@ -569,36 +583,37 @@ hipError_t run_factored(const DevProblem &p, GramKind kind, void *work, const De
     ra.part_occ = occ_in_reduce ? reinterpret_cast<cplx *>(w + L.acht_occ) : nullptr;
     ra.acht_iw = p.nfreq > 2 ? 2 : p.nfreq - 1;  // sch_array[2], gppComplex.cpp:381
     ra.neg = p.wx_neg;
+    ra.stamp = stage("factored_pole_reduce");
     GPP_TRY(launch_pole_reduce(ra, kind.red_fc, s));
-    if (timer) timer->mark(s, "factored_pole_reduce");
+    const Stamp st_final = stage("factored_final");
     hipLaunchKernelGGL(k_fact_final, dim3(p.nfreq + 1), dim3(kRedThreads), 0, s, col_ach, col_asx, part_achs,
-                       p.ngpown * L.nsplit, p.nfreq, p.nb, p.nv, res.base);
+                       p.ngpown * L.nsplit, p.nfreq, p.nb, p.nv, res.base, st_final, kind.acht ? nullptr : end());
     GPP_TRY(hipGetLastError());
-    if (timer) timer->mark(s, "factored_final");
     if (kind.acht) {
+        Stamp st = stage("factored_acht");  // for the first launch of the stage
         const AchtSplit &as = L.as;
         cplx *part = reinterpret_cast<cplx *>(w + L.acht_part);
         cplx *part_occ = reinterpret_cast<cplx *>(w + L.acht_occ);
         if (p.nb > p.nv) {
             if (as.narrow)
-                as.cut ? launch_acht<GramM, true>(p, as, ra.p2, bg, part, s)
-                       : launch_acht<GramM, false>(p, as, ra.p2, bg, part, s);
+                as.cut ? launch_acht<GramM, true>(p, as, ra.p2, bg, part, st, s)
+                       : launch_acht<GramM, false>(p, as, ra.p2, bg, part, st, s);
             else
-                as.cut ? launch_acht<GramL, true>(p, as, ra.p2, bg, part, s)
-                       : launch_acht<GramL, false>(p, as, ra.p2, bg, part, s);
+                as.cut ? launch_acht<GramL, true>(p, as, ra.p2, bg, part, st, s)
+                       : launch_acht<GramL, false>(p, as, ra.p2, bg, part, st, s);
             GPP_TRY(hipGetLastError());
+            st = Stamp{};
         }
         if (p.nv > 0 && !occ_in_reduce) {  // else summed by the reduce
             hipLaunchKernelGGL(k_acht_occ, dim3(p.ngpown, L.occ_nsplit), dim3(kRedThreads), 0, s, ra.p2, ra.br1,
                                p.aqsn, bg, p.idx, p.vcoul, p.ngpown, p.ncouls, p.nv, L.occ_chunk, L.occ_nsplit,
-                               part_occ);
+                               part_occ, st);
             GPP_TRY(hipGetLastError());
         }
         hipLaunchKernelGGL(k_acht_final, dim3((p.nb + kAchtFinalBands - 1) / kAchtFinalBands + p.nv), dim3(256), 0,
                            s, part, as.jtiles * as.nks, part_occ,
-                           p.ngpown * L.occ_nsplit, p.nb, p.nv, res.acht_n1_loc());
+                           p.ngpown * L.occ_nsplit, p.nb, p.nv, res.acht_n1_loc(), end());
         GPP_TRY(hipGetLastError());
-        if (timer) timer->mark(s, "factored_acht");
     }
     return hipSuccess;
 }
@@ -614,8 +629,9 @@ hipError_t run_factored(const DevProblem &p, GramKind kind, void *work, const De
 namespace {
 
 __global__ void k_permute_rows(const cplx *__restrict__ src, const int32_t *__restrict__ perm, int nrows,
-                               int ncols, cplx *__restrict__ dst)
+                               int ncols, cplx *__restrict__ dst, Stamp stamp)
 {
+    stamp_start(stamp);
     const size_t n = (size_t)nrows * ncols;
     for (size_t t = (size_t)blockIdx.x * blockDim.x + threadIdx.x; t < n; t += (size_t)gridDim.x * blockDim.x) {
         const size_t r = t / ncols, c = t % ncols;
@@ -627,8 +643,9 @@ __global__ void k_permute_rows(const cplx *__restrict__ src, const int32_t *__re
 // bucket b; bres holds each bucket's DevResults back to back.
 __global__ void k_bucket_combine(const cplx *__restrict__ bres, const int32_t *__restrict__ tab,
                                  const int32_t *__restrict__ perm, int nbuckets, int nfreq, int nb,
-                                 cplx *__restrict__ out)
+                                 cplx *__restrict__ out, Stamp stamp, unsigned long long *end)
 {
+    stamp_start(stamp);
     for (int iw = threadIdx.x; iw < 2 * nfreq; iw += blockDim.x) {
         cplx s = czero();
         for (int b = 0; b < nbuckets; ++b) s = cadd(s, bres[tab[3 * b] + iw]);
@@ -642,6 +659,7 @@ __global__ void k_bucket_combine(const cplx *__restrict__ bres, const int32_t *_
     for (int b = 0; b < nbuckets; ++b)
         for (int k = threadIdx.x; k < tab[3 * b + 2]; k += blockDim.x)
             out[2 * nfreq + perm[tab[3 * b + 1] + k]] = bres[tab[3 * b] + 2 * nfreq + k];
+    stamp_end(end);
 }
 
 struct BucketLayout {
@@ -742,7 +760,8 @@ hipError_t run_factored_bucketed(const DevProblem &p, GramKind kind, const Bucke
     cplx *bres = reinterpret_cast<cplx *>(w + L.bres);
     const int nbk = (int)bp.size.size();
 
-    if (timer) timer->begin(s);
+    const auto stage = [&](const char *nm) { return timer ? timer->stage(nm) : Stamp{}; };
+    if (timer) timer->begin();
     GPP_TRY(hipMemcpyAsync(perm, bp.perm.data(), sizeof(int32_t) * p.nb, hipMemcpyHostToDevice, s));
     GPP_TRY(hipMemcpyAsync(tab, bp.tab.data(), sizeof(int32_t) * 3 * nbk, hipMemcpyHostToDevice, s));
     {
@@ -750,25 +769,24 @@ hipError_t run_factored_bucketed(const DevProblem &p, GramKind kind, const Bucke
         size_t blocks = (n + 255) / 256;
         if (blocks > 8192) blocks = 8192;
         hipLaunchKernelGGL(k_permute_rows, dim3((unsigned)blocks), dim3(256), 0, s, p.aqsm, perm, p.nb, p.ncouls,
-                           aqsm_p);
+                           aqsm_p, stage("bucket_permute"));
         hipLaunchKernelGGL(k_permute_rows, dim3((unsigned)blocks), dim3(256), 0, s, p.aqsn, perm, p.nb, p.ncouls,
-                           aqsn_p);
+                           aqsn_p, Stamp{});
         GPP_TRY(hipGetLastError());
     }
-    if (timer) timer->mark(s, "bucket_permute");
+    Stamp st = stage("bucket_factored");
     for (int b = 0; b < nbk; ++b) {
         const DevProblem q = bucket_problem(p, bp, b, aqsm_p, aqsn_p);
         DevResults r;
         r.base = bres + bp.tab[3 * b];
         r.nfreq = p.nfreq;
         r.nb = q.nb;
-        GPP_TRY(run_factored(q, kind, w + L.sub, r, s, nullptr));
+        GPP_TRY(run_factored(q, kind, w + L.sub, r, s, nullptr, b == 0 ? st : Stamp{}));
     }
-    if (timer) timer->mark(s, "bucket_factored");
-    hipLaunchKernelGGL(k_bucket_combine, dim3(1), dim3(256), 0, s, bres, tab, perm, nbk, p.nfreq, p.nb, res.base);
-    GPP_TRY(hipGetLastError());
-    if (timer) timer->mark(s, "bucket_combine");
-    return hipSuccess;
+    st = stage("bucket_combine");
+    hipLaunchKernelGGL(k_bucket_combine, dim3(1), dim3(256), 0, s, bres, tab, perm, nbk, p.nfreq, p.nb, res.base, st,
+                       timer ? timer->end() : nullptr);
+    return hipGetLastError();
 }
 
 }  // namespace gpp

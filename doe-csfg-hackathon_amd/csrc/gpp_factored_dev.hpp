@@ -555,6 +555,7 @@ struct ReduceArgs {
     // With p2 and reduce_sums_acht_occ: the occupied bands' acht_n1_loc
     // partials, [ngpown][nsplit][nv], summed in the pass (br1 not written).
     cplx *part_occ;
+    Stamp stamp;
 };
 
 // Whether the p2-storing reduce sums the occupied bands' acht_n1_loc terms
@@ -922,6 +923,7 @@ struct PoleTileArgs {
     const double *wx;
     int nb, nv, ncouls, ngpown, nsplit;  // nsplit = G-vector tiles
     cplx *col_ach, *col_asx;             // [ngpown][nsplit][F], unscaled tile sums
+    Stamp stamp;
 };
 
 // LDS of the fused Gram + pole reduce block (128 x 128 tile, 8 waves), in

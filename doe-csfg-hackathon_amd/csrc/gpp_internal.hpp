@@ -50,27 +50,31 @@ struct Workspace {
     void release();
 };
 
-// Records HIP events between the stages of an evaluation, for the last
-// kRing evaluations (so that evaluations enqueued back to back can be timed
-// after one synchronisation).
+// Stage times of the last kRing evaluations, noted by the stages' own launches
+// in device memory (Stamp), so that evaluations enqueued back to back can be
+// timed after one synchronisation.
 struct StageTimer {
     static constexpr int kMax = 12;
     static constexpr int kRing = 32;
     struct Slot {
-        hipEvent_t ev[kMax + 1] = {};
         const char *name[kMax] = {};
         int n = 0;  // stages recorded
     };
     Slot slot[kRing];
     int cur = 0;     // slot of the current (last) evaluation
     int filled = 0;  // evaluations recorded, at most kRing
-    bool ready = false;
-    hipError_t init();
+    unsigned long long *dev = nullptr;  // [kRing][kMax + 1]: stage starts, then the end
+    int khz = 100000;                   // rate of the device clock
+    hipError_t init(int device);
     void destroy();
-    void begin(hipStream_t s);                 // starts a slot, records ev[0]
-    void mark(hipStream_t s, const char *nm);  // closes one stage
+    void begin();                 // starts a slot
+    Stamp stage(const char *nm);  // for the first launch of the next stage
+    unsigned long long *end() { return dev ? dev + cur * (kMax + 1) + slot[cur].n : nullptr; }  // for the last launch
     const Slot &last() const { return slot[cur]; }
     const Slot &back(int k) const { return slot[(cur - k + kRing) % kRing]; }  // k evaluations before the last
+    // Milliseconds of the evaluation k before the last, total and per stage
+    // (the stream must be idle).
+    hipError_t read(int k, double *total, double (&stage_ms)[kMax]) const;
 };
 
 // 1 if some of the n frequencies is negative (NaN counts as negative, so an
@@ -97,10 +101,9 @@ hipError_t run_direct(const DevProblem &p, bool strict, void *work, const DevRes
 hipError_t run_direct_part(const DevProblem &p, int which, void *work, const DevResults &res,
                            hipStream_t s);
 
-// reduce_achstemp per band into part_achs[nb] (fixed-order sums over j).
-// achstemp per band into part_achs[nb]; with bg non-null also the gathered
+// achstemp per band into part_achs[nb] (fixed-order sums over j); with bg non-null also the gathered
 // rows Bg[n1][j] = aqsm[n1][igp(j)] [nb][ngpown].
-hipError_t launch_achstemp(const DevProblem &p, cplx *part_achs, cplx *bg, hipStream_t s);
+hipError_t launch_achstemp(const DevProblem &p, cplx *part_achs, cplx *bg, Stamp stamp, hipStream_t s);
 
 // Zeroes n ints with a fill kernel (no memset node when a caller captures).
 hipError_t launch_zero_ints(int *d_p, int n, hipStream_t s);
@@ -136,8 +139,9 @@ struct GramKind {
 constexpr int kGramTiles = 4;
 
 size_t factored_workspace_bytes(const DevProblem &p, GramKind kind);
+// first: without a timer, the stamp of the first launch.
 hipError_t run_factored(const DevProblem &p, GramKind kind, void *work, const DevResults &res,
-                        hipStream_t s, StageTimer *timer);
+                        hipStream_t s, StageTimer *timer, Stamp first = Stamp{});
 
 // Band-dependent frequencies (gpp_factored.hip): bands grouped by identical
 // wx rows; bucket b holds bands perm[start[b] .. start[b]+size[b]), its
@@ -160,7 +164,7 @@ hipError_t run_factored_bucketed(const DevProblem &p, GramKind kind, const Bucke
 // [nv, nb), written to mout [ngpown][ncouls].
 size_t ozaki_workspace_bytes(const DevProblem &p, int slices, bool int8);
 hipError_t launch_gram_ozaki(const DevProblem &p, int slices, bool int8, int layout, int group, const cplx *bg,
-                             void *work, cplx *mout, hipStream_t s);
+                             void *work, cplx *mout, Stamp stamp, hipStream_t s);
 
 // ---- batched factored form (gpp_batch.hip) --------------------------------
 struct GramItem {  // one Gram tile of one instance

@@ -78,8 +78,9 @@ template <> struct OzWaves<2> {
 
 // Column exponents: grid ncols_pad / 64.
 __global__ __launch_bounds__(256) void k_oz_colexp(const cplx *__restrict__ src, int ld, int k_begin, int k_end,
-                                                   int ncols, int ncols_pad, int *__restrict__ exps)
+                                                   int ncols, int ncols_pad, int *__restrict__ exps, Stamp stamp)
 {
+    stamp_start(stamp);
     __shared__ double part[4][64];
     colexp_block(src, ld, k_begin, k_end, ncols, ncols_pad, exps, blockIdx.x, part);
 }
@@ -418,7 +419,7 @@ void launch_gram_tiles(const OzLayout &L, const DevProblem &p, const D *bd, cons
 
 template <int S, typename D>
 hipError_t launch_ozaki_s(const DevProblem &p, int layout, int group, const cplx *bg, void *work, cplx *mout,
-                          hipStream_t s)
+                          Stamp stamp, hipStream_t s)
 {
     const OzLayout L = oz_layout(p, S, sizeof(D) == 1);
     char *w = static_cast<char *>(work);
@@ -428,9 +429,9 @@ hipError_t launch_ozaki_s(const DevProblem &p, int layout, int group, const cplx
     D *ad = reinterpret_cast<D *>(w + L.ad);
     constexpr int KP = 16 / (int)sizeof(D);
     hipLaunchKernelGGL(k_oz_colexp, dim3(L.ngp_pad / 64), dim3(256), 0, s, bg, p.ngpown, p.nv, p.nb, p.ngpown,
-                       L.ngp_pad, eb);
+                       L.ngp_pad, eb, stamp);
     hipLaunchKernelGGL(k_oz_colexp, dim3(L.nc_pad / 64), dim3(256), 0, s, p.aqsn, p.ncouls, p.nv, p.nb, p.ncouls,
-                       L.nc_pad, ea);
+                       L.nc_pad, ea, Stamp{});
     hipLaunchKernelGGL((k_oz_split<S, D>), dim3((L.ngp_pad + 255) / 256, L.kpad / KP), dim3(256), 0, s, bg,
                        p.ngpown, p.nv, L.K, p.ngpown, L.ngp_pad, L.kpad, eb, bd);
     hipLaunchKernelGGL((k_oz_split<S, D>), dim3((L.nc_pad + 255) / 256, L.kpad / KP), dim3(256), 0, s, p.aqsn,
@@ -475,13 +476,13 @@ hipError_t launch_ozaki_s(const DevProblem &p, int layout, int group, const cplx
 
 template <typename D>
 hipError_t launch_ozaki_d(const DevProblem &p, int slices, int layout, int group, const cplx *bg, void *work,
-                          cplx *mout, hipStream_t s)
+                          cplx *mout, Stamp stamp, hipStream_t s)
 {
     switch (slices) {
-    case 3: return launch_ozaki_s<3, D>(p, layout, group, bg, work, mout, s);
-    case 4: return launch_ozaki_s<4, D>(p, layout, group, bg, work, mout, s);
-    case 5: return launch_ozaki_s<5, D>(p, layout, group, bg, work, mout, s);
-    case 6: return launch_ozaki_s<6, D>(p, layout, group, bg, work, mout, s);
+    case 3: return launch_ozaki_s<3, D>(p, layout, group, bg, work, mout, stamp, s);
+    case 4: return launch_ozaki_s<4, D>(p, layout, group, bg, work, mout, stamp, s);
+    case 5: return launch_ozaki_s<5, D>(p, layout, group, bg, work, mout, stamp, s);
+    case 6: return launch_ozaki_s<6, D>(p, layout, group, bg, work, mout, stamp, s);
     default: return hipErrorInvalidValue;
     }
 }
@@ -491,10 +492,10 @@ hipError_t launch_ozaki_d(const DevProblem &p, int slices, int layout, int group
 size_t ozaki_workspace_bytes(const DevProblem &p, int slices, bool int8) { return oz_layout(p, slices, int8).total; }
 
 hipError_t launch_gram_ozaki(const DevProblem &p, int slices, bool int8, int layout, int group, const cplx *bg,
-                             void *work, cplx *mout, hipStream_t s)
+                             void *work, cplx *mout, Stamp stamp, hipStream_t s)
 {
-    return int8 ? launch_ozaki_d<int8_t>(p, slices, layout, group, bg, work, mout, s)
-                : launch_ozaki_d<_Float16>(p, slices, layout, group, bg, work, mout, s);
+    return int8 ? launch_ozaki_d<int8_t>(p, slices, layout, group, bg, work, mout, stamp, s)
+                : launch_ozaki_d<_Float16>(p, slices, layout, group, bg, work, mout, stamp, s);
 }
 
 }  // namespace gpp

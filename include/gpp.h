@@ -181,7 +181,7 @@ const char *gpp_last_error(void);
 int gpp_abi_version(void);
 
 /* Creates a context on HIP device `device`: a default-priority stream and
- * timing events.  No input buffers are allocated until gpp_upload. */
+ * a table of stage times.  No input buffers are allocated until gpp_upload. */
 gpp_status gpp_ctx_create(gpp_ctx **out, int device);
 
 /* Releases the context and every device buffer it owns. Null is a no-op. */
@@ -383,8 +383,9 @@ gpp_status gpp_ctx_set_option(gpp_ctx *ctx, gpp_option option, int value);
 gpp_status gpp_ctx_get_option(const gpp_ctx *ctx, gpp_option option, int *value);
 
 /*
- * GPU time of the last gpp_sigma in milliseconds, measured with HIP events
- * on the context's stream: total, and per stage (stage_ms[i] for i <
+ * GPU time of the last gpp_sigma in milliseconds, from the device clock as the
+ * stages' own launches note it (10 ns steps; waits for the context's enqueued
+ * work): total, and per stage (stage_ms[i] for i <
  * *nstages, at most max_stages written; stage names via
  * gpp_ctx_stage_name).  Any pointer may be NULL.
  */
