@@ -77,9 +77,9 @@ __global__ __launch_bounds__(C::NT) __attribute__((amdgpu_waves_per_eu(C::OCC)))
         const GramItem it = items[w];
         const BInst &b = insts[it.inst];
         if (C::SJ == 2 && b.ngpown - it.j0 <= 16 * C::WJN)
-            gram_ring_tile<C, 1>(b.bg, b.aqsn, b.ngpown, b.ncouls, b.nv, b.nb, it.j0, it.i0, lds, true, b.mu);
+            gram_ring_tile<C, 1, true>(b.bg, b.aqsn, b.ngpown, b.ncouls, b.nv, b.nb, it.j0, it.i0, lds, b.mu);
         else
-            gram_ring_tile<C, C::SJ>(b.bg, b.aqsn, b.ngpown, b.ncouls, b.nv, b.nb, it.j0, it.i0, lds, true, b.mu);
+            gram_ring_tile<C, C::SJ, true>(b.bg, b.aqsn, b.ngpown, b.ncouls, b.nv, b.nb, it.j0, it.i0, lds, b.mu);
         __syncthreads();  // every wave is done with lds
     }
 }

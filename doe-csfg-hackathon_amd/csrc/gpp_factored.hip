@@ -95,10 +95,11 @@ bool fused_reduce(const DevProblem &p, const GramKind &k)
            p.nv <= kFuseNv;
 }
 
-// Mu is stored past the caches when it is larger than them (256 MB): it is
-// written once and read back once, by the pole reduce (C1, 859 MB: reduce
-// 0.486-0.502 -> 0.469 ms); a smaller one is read back from them.
-bool mu_streams(const DevProblem &p) { return sizeof(cplx) * (size_t)p.ngpown * p.ncouls > ((size_t)256 << 20); }
+// Mu is stored past the caches when it is larger than the L2s (32 MB): it is
+// written once and read back once, by the pole reduce.  us, plain against
+// non-temporal stores: 512/2/32768/1638 (859 MB) reduce 510 -> 422, Gram alike;
+// 512/2/32768/205 (107 MB) reduce 80 -> 72, Gram 357 -> 363.
+bool mu_streams(const DevProblem &p) { return sizeof(cplx) * (size_t)p.ngpown * p.ncouls > ((size_t)32 << 20); }
 
 // G-vectors per block of k_acht_occ: the reduce's range, halved while the
 // launch has fewer than 2048 blocks (each thread waits on its own loads:
@@ -155,29 +156,29 @@ FactLayout fact_layout(const DevProblem &p, const GramKind &k)
 // fastest in tile order and tiles spread over the XCDs by xcd_tile, so the
 // blocks sharing one aqsn tile run on one XCD.  The last G' tile runs SJR <= SJ
 // sub-tiles per wave, as many as its columns need (the launcher picks SJR).
-template <class C, int SJR>
+template <class C, int SJR, bool NTS>
 __global__ __launch_bounds__(C::NT) __attribute__((amdgpu_waves_per_eu(C::OCC))) void k_gram_f64(
     const cplx *__restrict__ bg, const cplx *__restrict__ aqsn, int ngpown, int ncouls, int k_begin, int k_end,
-    bool nts, cplx *__restrict__ mout, Stamp stamp)
+    cplx *__restrict__ mout, Stamp stamp)
 {
     stamp_start(stamp);
     __shared__ cplx lds[C::LDS];
     const int nj = (ngpown + C::TJ - 1) / C::TJ, ni = (ncouls + C::TI - 1) / C::TI;
     if constexpr (SJR == C::SJ) {
         const int t = xcd_tile(blockIdx.x, nj * ni);
-        gram_ring_tile<C, C::SJ>(bg, aqsn, ngpown, ncouls, k_begin, k_end, (t % nj) * C::TJ, (t / nj) * C::TI, lds,
-                                 nts, mout);
+        gram_ring_tile<C, C::SJ, NTS>(bg, aqsn, ngpown, ncouls, k_begin, k_end, (t % nj) * C::TJ, (t / nj) * C::TI,
+                                      lds, mout);
     } else {
         // the shorter tiles come last, so that they fill the last round
         const int full = (nj - 1) * ni, b = blockIdx.x;
         if (b < full) {
             const int t = xcd_tile(b, full);
-            gram_ring_tile<C, C::SJ>(bg, aqsn, ngpown, ncouls, k_begin, k_end, (t % (nj - 1)) * C::TJ,
-                                     (t / (nj - 1)) * C::TI, lds, nts, mout);
+            gram_ring_tile<C, C::SJ, NTS>(bg, aqsn, ngpown, ncouls, k_begin, k_end, (t % (nj - 1)) * C::TJ,
+                                          (t / (nj - 1)) * C::TI, lds, mout);
         } else {
             const int t = xcd_tile(b - full, ni);
-            gram_ring_tile<C, SJR>(bg, aqsn, ngpown, ncouls, k_begin, k_end, (nj - 1) * C::TJ, t * C::TI, lds, nts,
-                                   mout);
+            gram_ring_tile<C, SJR, NTS>(bg, aqsn, ngpown, ncouls, k_begin, k_end, (nj - 1) * C::TJ, t * C::TI, lds,
+                                        mout);
         }
     }
 }
@@ -373,18 +374,26 @@ __global__ __launch_bounds__(256) void k_acht_final(const cplx *__restrict__ par
     stamp_end(end);
 }
 
+template <class C, bool NTS>
+void launch_gram_nts(const DevProblem &p, const cplx *bg, cplx *mu, Stamp stamp, hipStream_t s)
+{
+    const unsigned tiles = (unsigned)((p.ngpown + C::TJ - 1) / C::TJ) * (unsigned)((p.ncouls + C::TI - 1) / C::TI);
+    const int rem = p.ngpown % C::TJ;
+    if (C::SJ == 2 && rem > 0 && rem <= 16 * C::WJN)
+        hipLaunchKernelGGL((k_gram_f64<C, 1, NTS>), dim3(tiles), dim3(C::NT), 0, s, bg, p.aqsn, p.ngpown, p.ncouls,
+                           p.nv, p.nb, mu, stamp);
+    else
+        hipLaunchKernelGGL((k_gram_f64<C, C::SJ, NTS>), dim3(tiles), dim3(C::NT), 0, s, bg, p.aqsn, p.ngpown,
+                           p.ncouls, p.nv, p.nb, mu, stamp);
+}
+
 template <class C>
 void launch_gram_ring(const DevProblem &p, const cplx *bg, cplx *mu, Stamp stamp, hipStream_t s)
 {
-    const unsigned tiles = (unsigned)((p.ngpown + C::TJ - 1) / C::TJ) * (unsigned)((p.ncouls + C::TI - 1) / C::TI);
-    const bool nts = mu_streams(p);
-    const int rem = p.ngpown % C::TJ;
-    if (C::SJ == 2 && rem > 0 && rem <= 16 * C::WJN)
-        hipLaunchKernelGGL((k_gram_f64<C, 1>), dim3(tiles), dim3(C::NT), 0, s, bg, p.aqsn, p.ngpown, p.ncouls, p.nv,
-                           p.nb, nts, mu, stamp);
+    if (mu_streams(p))
+        launch_gram_nts<C, true>(p, bg, mu, stamp, s);
     else
-        hipLaunchKernelGGL((k_gram_f64<C, C::SJ>), dim3(tiles), dim3(C::NT), 0, s, bg, p.aqsn, p.ngpown, p.ncouls,
-                           p.nv, p.nb, nts, mu, stamp);
+        launch_gram_nts<C, false>(p, bg, mu, stamp, s);
 }
 
 template <class C, bool CUT>

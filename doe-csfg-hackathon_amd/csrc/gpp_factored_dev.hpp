@@ -87,12 +87,14 @@ typedef GramRing<2, 2, 2, 2, 8, 4, 2> GramM;   // 64 x 64
 typedef GramRing<2, 4, 1, 1, 16, 3, 4> GramS;  // 32 x 64
 
 // One tile with SJC <= SJ sub-tile rows per wave: the first 16 SJC WJN columns
-// from j0, for a last tile whose columns need no more.  nts: non-temporal
-// stores of Mu.  The block's waves must be done with lds before the call.
-template <class C, int SJC>
+// from j0, for a last tile whose columns need no more.  NTS: non-temporal
+// stores of Mu (a template parameter: under a run-time flag the compiler merged
+// both kinds into plain stores, and the C1 reduce took 510 us instead of 424).
+// The block's waves must be done with lds before the call.
+template <class C, int SJC, bool NTS>
 __device__ __forceinline__ void gram_ring_tile(const cplx *__restrict__ bg, const cplx *__restrict__ aqsn, int ngpown,
                                                int ncouls, int k_begin, int k_end, int j0, int i0, cplx *lds,
-                                               bool nts, cplx *__restrict__ mout)
+                                               cplx *__restrict__ mout)
 {
     constexpr int KS = C::KS, NB = C::NB, TJ = C::TJ, TI = C::TI, SI = C::SI, NW = C::NW;
     constexpr int QB = KS * TJ / 64 / NW, QA = KS * TI / 64 / NW, LD = QB + QA;  // loads per wave and stage
@@ -230,7 +232,7 @@ __device__ __forceinline__ void gram_ring_tile(const cplx *__restrict__ bg, cons
                 if (j < ngpown && ig < ncouls) {
                     const cplx v = {acc1[s][t][r] + acc2[s][t][r], (acc3[s][t][r] - acc1[s][t][r]) + acc2[s][t][r]};
                     cplx *o = &mout[(size_t)j * ncouls + ig];
-                    if (nts) {
+                    if constexpr (NTS) {
                         __builtin_nontemporal_store(v.re, &o->re);
                         __builtin_nontemporal_store(v.im, &o->im);
                     } else {
