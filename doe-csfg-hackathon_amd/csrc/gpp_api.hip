@@ -1414,19 +1414,22 @@ gpp_status gpp_batch_destroy(gpp_batch *b)
 
 // ---------------------------------------------------------------------------
 // Reference-compatible launchers.  They share one grow-only scratch area per
-// device (partials, results, index flag), guarded by a mutex: calls from
-// several host threads serialise on it.
+// device (partials, index flag), guarded by a mutex: calls from several host
+// threads serialise on it.
 namespace {
 
 struct CompatScratch {
-    gpp::Workspace work, results, flag;
+    gpp::Workspace work, flag;
+    int *host_bad = nullptr;  // pinned: the index check's result, polled by the host
 };
 
 std::mutex g_compat_mu;
 std::vector<CompatScratch> g_compat;
 
-gpp_status compat_run(int which, const gpp::DevProblem &dp, double *ach_re, double *ach_im, cplx *asx,
-                      cplx *acht_n1, double *achs_re, double *achs_im)
+// Enqueues the index check and then the evaluation, whose last launch adds
+// nothing when the check failed (the kernels clamp negative indices), and waits
+// for the check alone: the evaluation runs on while the caller enqueues more.
+gpp_status compat_run(int which, const gpp::DevProblem &dp, gpp::CompatOut co)
 {
     std::lock_guard<std::mutex> lock(g_compat_mu);
     int dev = 0;
@@ -1435,20 +1438,31 @@ gpp_status compat_run(int which, const gpp::DevProblem &dp, double *ach_re, doub
     CompatScratch &cs = g_compat[dev];
     hipStream_t s = nullptr;  // null stream, as the reference launches
     HIP_OR_FAIL(cs.flag.reserve(sizeof(int)), "hipMalloc flag");
-    HIP_OR_FAIL(hipMemsetAsync(cs.flag.ptr, 0, sizeof(int), s), "hipMemsetAsync");
-    HIP_OR_FAIL(gpp::launch_check_index(dp.idx, dp.ngpown, static_cast<int *>(cs.flag.ptr), s), "check_index");
-    int bad = 0;
-    HIP_OR_FAIL(hipMemcpy(&bad, cs.flag.ptr, sizeof(int), hipMemcpyDeviceToHost), "D2H flag");
-    if (bad) return fail(GPP_ERR_BAD_INDEX, "%d negative inv_igp_index entries", bad);
+    if (!cs.host_bad)
+        HIP_OR_FAIL(hipHostMalloc(reinterpret_cast<void **>(&cs.host_bad), sizeof(int), hipHostMallocDefault),
+                    "pinned flag allocation");
     HIP_OR_FAIL(cs.work.reserve(gpp::direct_workspace_bytes(dp)), "workspace allocation");
-    gpp::DevResults res;
-    res.nfreq = dp.nfreq;
-    res.nb = dp.nb;
-    HIP_OR_FAIL(cs.results.reserve(sizeof(cplx) * res.count()), "results allocation");
-    res.base = static_cast<cplx *>(cs.results.ptr);
-    HIP_OR_FAIL(gpp::run_direct_part(dp, which, cs.work.ptr, res, s), "direct launch");
-    HIP_OR_FAIL(gpp::launch_accumulate_compat(res, which, dp.nv, ach_re, ach_im, asx, acht_n1, achs_re, achs_im, s),
-                "accumulate launch");
+    __atomic_store_n(cs.host_bad, -1, __ATOMIC_RELEASE);
+    co.bad = static_cast<const int *>(cs.flag.ptr);
+    HIP_OR_FAIL(gpp::launch_check_index_once(dp.idx, dp.ngpown, static_cast<int *>(cs.flag.ptr), cs.host_bad, s),
+                "check_index");
+    const hipError_t launched = gpp::run_direct_part(dp, which, cs.work.ptr, co, s);
+    if (launched != hipSuccess) {
+        (void)hipStreamSynchronize(s);  // the check's result must not arrive in a later call
+        return fail_hip(launched, "direct launch");
+    }
+    int bad = -1;
+    for (unsigned spin = 1; (bad = __atomic_load_n(cs.host_bad, __ATOMIC_ACQUIRE)) < 0; ++spin) {
+        if (spin % 4096) continue;
+        // an error, or a stream that went idle without the check's result, ends the wait
+        const hipError_t e = hipStreamQuery(s);
+        if (e == hipErrorNotReady) continue;
+        if (e != hipSuccess) return fail_hip(e, "index check");
+        if ((bad = __atomic_load_n(cs.host_bad, __ATOMIC_ACQUIRE)) < 0)
+            return fail(GPP_ERR_LAUNCH, "the index check left no result");
+        break;
+    }
+    if (bad) return fail(GPP_ERR_BAD_INDEX, "%d negative inv_igp_index entries", bad);
     return GPP_OK;
 }
 
@@ -1483,8 +1497,12 @@ gpp_status d_till_nvband(int nvband, int ngpown, int ncouls, int *inv_igp_index,
         return fail(GPP_ERR_INVALID_ARGUMENT, "NULL device array");
     gpp::DevProblem dp = compat_problem(nvband, nvband, ncouls, ngpown, inv_igp_index, wx_array, vcoul, aqsmtemp,
                                         aqsntemp, I_eps_array, wtilde_array, occ);
-    return compat_run(0, dp, achtemp_re, achtemp_im, reinterpret_cast<cplx *>(asxtemp),
-                      reinterpret_cast<cplx *>(acht_n1_loc), nullptr, nullptr);
+    gpp::CompatOut co;
+    co.achtemp_re = achtemp_re;
+    co.achtemp_im = achtemp_im;
+    co.asxtemp = reinterpret_cast<cplx *>(asxtemp);
+    co.acht_n1 = reinterpret_cast<cplx *>(acht_n1_loc);
+    return compat_run(0, dp, co);
 }
 
 gpp_status d_reduce_achstemp(int number_bands, int *inv_igp_index, int ncouls, gpp_complex *aqsmtemp,
@@ -1498,7 +1516,10 @@ gpp_status d_reduce_achstemp(int number_bands, int *inv_igp_index, int ncouls, g
         return fail(GPP_ERR_INVALID_ARGUMENT, "NULL device array");
     gpp::DevProblem dp = compat_problem(number_bands, 0, ncouls, ngpown, inv_igp_index, nullptr, vcoul, aqsmtemp,
                                         aqsntemp, I_eps_array, nullptr, 1.0);
-    return compat_run(2, dp, nullptr, nullptr, nullptr, nullptr, achstemp_re, achstemp_im);
+    gpp::CompatOut co;
+    co.achstemp_re = achstemp_re;
+    co.achstemp_im = achstemp_im;
+    return compat_run(2, dp, co);
 }
 
 gpp_status d_noFlagOCCSolver(int number_bands, int nvband, int ngpown, int ncouls, int *inv_igp_index,
@@ -1515,8 +1536,11 @@ gpp_status d_noFlagOCCSolver(int number_bands, int nvband, int ngpown, int ncoul
         return fail(GPP_ERR_INVALID_ARGUMENT, "NULL device array");
     gpp::DevProblem dp = compat_problem(number_bands, nvband, ncouls, ngpown, inv_igp_index, wx_array, vcoul,
                                         aqsmtemp, aqsntemp, I_eps_array, wtilde_array, 1.0);
-    return compat_run(1, dp, achtemp_re, achtemp_im, nullptr, reinterpret_cast<cplx *>(acht_n1_loc), nullptr,
-                      nullptr);
+    gpp::CompatOut co;
+    co.achtemp_re = achtemp_re;
+    co.achtemp_im = achtemp_im;
+    co.acht_n1 = reinterpret_cast<cplx *>(acht_n1_loc);
+    return compat_run(1, dp, co);
 }
 
 }  // extern "C"
@@ -1575,12 +1599,8 @@ gpp_status d_noFlagOCCSolver_noalloc(int number_bands, int nvband, int ngpown, i
         return fail(GPP_ERR_INVALID_ARGUMENT, "NULL device array");
     const gpp::DevProblem dp = compat_problem(number_bands, nvband, ncouls, ngpown, inv_igp_index, wx_array, vcoul,
                                               aqsmtemp, aqsntemp, I_eps_array, wtilde_array, 1.0);
-    // scratch: [index flag: 256 B][results][direct-form partial sums]
-    gpp::DevResults res;
-    res.nfreq = dp.nfreq;
-    res.nb = dp.nb;
-    const size_t res_bytes = (sizeof(cplx) * res.count() + 255) & ~(size_t)255;
-    const size_t need = 256 + res_bytes + gpp::direct_workspace_bytes(dp);
+    // scratch: [index flag: 256 B][direct-form partial sums]
+    const size_t need = 256 + gpp::direct_workspace_bytes(dp);
     if (need > kNoAllocScratchBytes)
         return fail(GPP_ERR_INVALID_ARGUMENT,
                     "number_bands=%d ngpown=%d needs %zu bytes of scratch; d_noFlagOCCSolver_noalloc holds %zu "
@@ -1599,11 +1619,11 @@ gpp_status d_noFlagOCCSolver_noalloc(int number_bands, int nvband, int ngpown, i
     int bad = 0;
     HIP_OR_FAIL(hipMemcpy(&bad, flag, sizeof(int), hipMemcpyDeviceToHost), "D2H flag");
     if (bad) return fail(GPP_ERR_BAD_INDEX, "%d negative inv_igp_index entries", bad);
-    res.base = reinterpret_cast<cplx *>(base + 256);
-    HIP_OR_FAIL(gpp::run_direct_part(dp, 1, base + 256 + res_bytes, res, s), "direct launch");
-    HIP_OR_FAIL(gpp::launch_accumulate_compat(res, 1, dp.nv, achtemp_re, achtemp_im, nullptr,
-                                              reinterpret_cast<cplx *>(acht_n1_loc), nullptr, nullptr, s),
-                "accumulate launch");
+    gpp::CompatOut co;
+    co.achtemp_re = achtemp_re;
+    co.achtemp_im = achtemp_im;
+    co.acht_n1 = reinterpret_cast<cplx *>(acht_n1_loc);
+    HIP_OR_FAIL(gpp::run_direct_part(dp, 1, base + 256, co, s), "direct launch");
     return GPP_OK;
 }
 

@@ -9,39 +9,55 @@
 // a = conj(aqsm[n1,igp]) * aqsn[n1,ig] is shared across the frequencies of
 // one (n1, j, ig), which the reference also computes identically per iw.
 //
-// Work decomposition (unoccupied bands, the hot loop):
-//   block  = NW waves; block (x, y) owns bands nv + x*NW .. +NW-1 (one band
-//            per wave) and the G'-column tile j0 = y*BJ .. +BJ-1;
-//   lane   = one G-vector ig of a 64-wide chunk; the chunk loop streams all
-//            ncouls G-vectors;
-//   LDS    = the chunk's wtilde / I_eps rows of the BJ columns, loaded once
-//            per block and read by all NW waves (double-buffered, one barrier
-//            per chunk);
-//   VGPRs  = the BJ x FC per-frequency complex accumulators of each lane.
-// After the chunk loop each wave reduces its accumulators by xor butterfly,
-// scales by 0.5*vcoul[igp] and sums its BJ columns in column order, writing
-// one partial per (band, column tile, frequency).  Two fixed-order tree
-// passes then reduce the partials, so results are bitwise reproducible.
+// One launch holds three kinds of blocks, the long chains first:
+//   occupied bands   block = 4 G'-columns of one band, two waves per column
+//                    (each half of the block's G range), lane = one G-vector;
+//   achstemp         one wave per (band, column group), gpp_device.hpp;
+//   unoccupied bands (the hot loop)
+//     block  = NW waves = NW bands (one per wave) x BJ G'-columns;
+//     lane   = one G-vector ig of a 64-wide chunk; the chunk loop streams the
+//              block's G range;
+//     LDS    = the chunk's wtilde / I_eps rows of the BJ columns, loaded once
+//              per block and read by all NW waves (double-buffered, one barrier
+//              per chunk);
+//     VGPRs  = the BJ x F per-frequency complex accumulators of each lane.
+// The G range is split (DirectArgs::gs) where whole ranges would leave the last
+// round of blocks nearly empty.  After its range each wave reduces its
+// accumulators by xor butterfly, scales by 0.5*vcoul[igp] and sums its BJ
+// columns in column order, writing one partial per (band, column tile, range,
+// frequency).  Two fixed-order passes then reduce the partials, so results are
+// bitwise reproducible.
+//
+// The unoccupied bands' loop is bound by the FP64 VALU (about 18 issue slots
+// per update, the reciprocal four of them); the occupied ones' by the latency
+// of their division chain, so they run beside it: us per call, occupied and
+// unoccupied as two launches against one, 512/2/1600/80 33 + 152 -> 161.
+#include <algorithm>
+#include <cmath>
+#include <type_traits>
+
 #include "gpp_internal.hpp"
 
 namespace gpp {
 namespace {
 
-constexpr int kBJ = 4;   // G' columns per block (unoccupied kernel tile)
-constexpr int kNW = 8;   // waves (bands) per block, unoccupied kernel
-constexpr int kOccWaves = 4;
-constexpr int kOccCols = kBJ / kOccWaves;  // columns per wave, occupied kernel
+constexpr int kBJ = 4;   // G' columns per block
+constexpr int kNW = 8;   // waves per block (bands, unoccupied; half-columns, occupied)
 constexpr int kReduceThreads = 256;
+constexpr int kDirectSlots = 512;  // blocks in flight: two per CU
 
 struct DirectArgs {
     const cplx *aqsm, *aqsn, *ieps, *wtilde;
     const int32_t *idx;
     const double *vcoul, *wx;
-    int nb, nv, ncouls, ngpown, nfreq, njt;
-    int wx_stride;  // 0: shared wx row; nfreq: band n1 reads wx[n1 * nfreq + iw]
+    int nb, nv, ncouls, ngpown, nfreq;
+    int njt, gs, nt;  // column tiles, G ranges, partials per (band, frequency): njt * gs
+    int nz;           // frequency passes
+    int wx_stride;    // 0: shared wx row; nfreq: band n1 reads wx[n1 * nfreq + iw]
+    int occ_blocks, ach_blocks;  // of the launch, before the unoccupied bands'
     double occ;
-    cplx *part_ach;   // [nb][njt][nfreq]
-    cplx *part_asx;   // [max(nv,1)][njt][nfreq]
+    cplx *part_ach;   // [nb][nt][nfreq]
+    cplx *part_asx;   // [max(nv,1)][nt][nfreq]
     cplx *part_achs;  // [nb][kAchSplit], then the AchCol entries (ach_cols_entry)
     cplx *band_ach;   // [nb][nfreq]
     cplx *band_asx;   // [max(nv,1)][nfreq]
@@ -56,14 +72,39 @@ struct WorkLayout {
 
 __host__ inline size_t align256(size_t x) { return (x + 255) & ~(size_t)255; }
 
+// Frequencies per pass: four, in the strict form three (its kernel of four
+// spills 40 registers beside the occupied bands' code: 541 against 499 us at
+// 131/5/2477/123 with 7 frequencies).
+constexpr int pass_width(bool strict) { return strict ? 3 : 4; }
+
+// G ranges per (band, column tile): the split that leaves the blocks in flight
+// least idle in the last round, with at least six chunks of 64 G-vectors per
+// range (a range costs its staging's start and a reduction of its
+// accumulators, about 1 % of a block per extra range).  Launches of more than
+// 4096 blocks stay whole.
+int direct_split(const DevProblem &p)
+{
+    const int njt = (p.ngpown + kBJ - 1) / kBJ, nun = p.nb - p.nv;
+    const double blocks = (double)(nun > 0 ? (nun + kNW - 1) / kNW : p.nv) * njt * ((p.nfreq + 3) / 4);
+    if (blocks > 4096) return 1;
+    const int chunks = (p.ncouls + kWave - 1) / kWave;
+    int best_gs = 1;
+    double best = 1e300;
+    for (int gs = 1; gs <= 16 && gs * 6 <= std::max(6, chunks) && (gs == 1 || blocks * gs <= 8192); ++gs) {
+        const double t = std::ceil(blocks * gs / kDirectSlots) / gs * (1.0 + 0.01 * gs);
+        if (t < best) best = t, best_gs = gs;
+    }
+    return best_gs;
+}
+
 WorkLayout layout_for(const DevProblem &p)
 {
-    const size_t njt = (size_t)(p.ngpown + kBJ - 1) / kBJ;
+    const size_t nt = (size_t)((p.ngpown + kBJ - 1) / kBJ) * direct_split(p);
     const size_t nvx = p.nv > 0 ? (size_t)p.nv : 1;
     WorkLayout L;
     size_t off = 0;
-    L.part_ach = off;  off += align256(sizeof(cplx) * (size_t)p.nb * njt * p.nfreq + sizeof(cplx));
-    L.part_asx = off;  off += align256(sizeof(cplx) * nvx * njt * p.nfreq);
+    L.part_ach = off;  off += align256(sizeof(cplx) * (size_t)p.nb * nt * p.nfreq + sizeof(cplx));
+    L.part_asx = off;  off += align256(sizeof(cplx) * nvx * nt * p.nfreq);
     L.part_achs = off; off += align256(sizeof(cplx) * ach_region_entries(p.nb, p.ngpown));
     L.band_ach = off;  off += align256(sizeof(cplx) * ((size_t)p.nb * p.nfreq + 1));
     L.band_asx = off;  off += align256(sizeof(cplx) * nvx * p.nfreq);
@@ -80,6 +121,10 @@ DirectArgs make_args(const DevProblem &p, void *work)
     a.idx = p.idx; a.vcoul = p.vcoul; a.wx = p.wx; a.wx_stride = p.wx_stride;
     a.nb = p.nb; a.nv = p.nv; a.ncouls = p.ncouls; a.ngpown = p.ngpown; a.nfreq = p.nfreq;
     a.njt = (p.ngpown + kBJ - 1) / kBJ;
+    a.gs = direct_split(p);
+    a.nt = a.njt * a.gs;
+    a.nz = 1;
+    a.occ_blocks = a.ach_blocks = 0;
     a.occ = p.occ;
     a.part_ach = reinterpret_cast<cplx *>(w + L.part_ach);
     a.part_asx = reinterpret_cast<cplx *>(w + L.part_asx);
@@ -139,25 +184,31 @@ __device__ __forceinline__ void unocc_update_strict(cplx (&acc)[FC], cplx cm, cp
 }
 
 // ---------------------------------------------------------------------------
-// Unoccupied bands.  Grid (ceil((nb-nv)/NW), njt, ceil(nfreq/FC)), block
-// NW*64 threads.
-template <int FC, bool STRICT>
-__global__ __launch_bounds__(kNW *kWave) void k_unocc(DirectArgs a)
+// Chunks [c0, c1) of 64 G-vectors of range g.
+__device__ __forceinline__ void range_chunks(const DirectArgs &a, int ncouls, int g, int &c0, int &c1)
+{
+    const int nchunks = (ncouls + kWave - 1) / kWave;
+    c0 = (int)((long long)nchunks * g / a.gs);
+    c1 = (int)((long long)nchunks * (g + 1) / a.gs);
+}
+
+// Unoccupied bands: block b of their share of the launch, frequencies
+// [iw0, iw0 + F).  lds: 4 kBJ kWave entries.
+template <int F, bool STRICT>
+__device__ __forceinline__ void unocc_block(const DirectArgs &a, int ncouls, int b, int iw0, cplx *lds)
 {
     constexpr int TILE = kBJ * kWave;  // (column, G-vector) positions per chunk
     static_assert(TILE <= kNW * kWave, "one position per staging thread");
-    int ncouls = a.ncouls;
-    const StampStart stamp(a.stamp, ncouls);
-    __shared__ cplx s_wt[2][kBJ][kWave];
-    __shared__ cplx s_ie[2][kBJ][kWave];  // I_eps (strict) or wtilde * I_eps (fast)
+    auto *s_wt = reinterpret_cast<cplx(*)[kBJ][kWave]>(lds);
+    auto *s_ie = s_wt + 2;  // I_eps (strict) or wtilde * I_eps (fast)
 
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
     const int lane = threadIdx.x % kWave;
-    const int n1 = a.nv + blockIdx.x * kNW + wave;
+    const int ngroups = (a.nb - a.nv + kNW - 1) / kNW;
+    const int n1 = a.nv + (b % ngroups) * kNW + wave;
     const bool band_ok = n1 < a.nb;
-    const int jt = blockIdx.y;
+    const int jt = (b / ngroups) % a.njt, g = b / (ngroups * a.njt);
     const int j0 = jt * kBJ;
-    const int iw0 = blockIdx.z * FC;
 
     // conj(aqsm[n1, igp(j)]) per column (mygpvar1, gppComplex.cpp:134).
     cplx cm[kBJ];
@@ -167,16 +218,15 @@ __global__ __launch_bounds__(kNW *kWave) void k_unocc(DirectArgs a)
         cm[jj] = czero();
         if (band_ok && j < a.ngpown) cm[jj] = cconj(a.aqsm[(size_t)n1 * ncouls + igp_of(a.idx, j, ncouls)]);
     }
-    double wxv[FC];
+    double wxv[F];
 #pragma unroll
-    for (int f = 0; f < FC; ++f)
-        wxv[f] = (band_ok && iw0 + f < a.nfreq) ? a.wx[(size_t)n1 * a.wx_stride + iw0 + f] : 0.0;
+    for (int f = 0; f < F; ++f) wxv[f] = band_ok ? a.wx[(size_t)n1 * a.wx_stride + iw0 + f] : 0.0;
 
-    cplx acc[kBJ][FC];
+    cplx acc[kBJ][F];
 #pragma unroll
     for (int jj = 0; jj < kBJ; ++jj)
 #pragma unroll
-        for (int f = 0; f < FC; ++f) acc[jj][f] = czero();
+        for (int f = 0; f < F; ++f) acc[jj][f] = czero();
 
     // Staging of one chunk's wtilde/I_eps tile: thread t < TILE loads both at
     // position t; the fast form stores wtilde * I_eps, formed here once
@@ -198,133 +248,200 @@ __global__ __launch_bounds__(kNW *kWave) void k_unocc(DirectArgs a)
         s_ie[buf][s_jj][s_l] = STRICT ? st_ie : cmul_fast(st_wt, st_ie);
     };
 
-    const int nchunks = (ncouls + kWave - 1) / kWave;
-    load_chunk(0);
+    auto load_an = [&](int c) {
+        const int ig = c * kWave + lane;
+        return band_ok && ig < ncouls ? a.aqsn[(size_t)n1 * ncouls + ig] : czero();
+    };
+    int c0, c1;
+    range_chunks(a, ncouls, g, c0, c1);
+    // the fast form loads aqsn of the next chunk while this one is evaluated
+    // (171 -> 161 us at 512/2/1600/80; the strict form has no registers for it)
+    cplx an_next = czero();
+    if (!STRICT) an_next = load_an(c0);
+    load_chunk(c0);
     store_chunk(0);
     __syncthreads();
-    for (int c = 0; c < nchunks; ++c) {
-        const int buf = c & 1;
-        if (c + 1 < nchunks) load_chunk(c + 1);
+    for (int c = c0; c < c1; ++c) {
+        const int buf = (c - c0) & 1;
+        cplx an = an_next;
+        if (c + 1 < c1) {
+            load_chunk(c + 1);
+            if (!STRICT) an_next = load_an(c + 1);
+        }
+        if (STRICT) an = load_an(c);
         if (band_ok) {
-            const int ig = c * kWave + lane;
-            const cplx an = ig < ncouls ? a.aqsn[(size_t)n1 * ncouls + ig] : czero();
 #pragma unroll
             for (int jj = 0; jj < kBJ; ++jj) {
                 const cplx wt = s_wt[buf][jj][lane];
                 const cplx ie = s_ie[buf][jj][lane];
-                if (STRICT) unocc_update_strict<FC>(acc[jj], cm[jj], an, wt, ie, wxv);
-                else unocc_update_fast<FC>(acc[jj], cm[jj], an, wt, ie, wxv);
+                if (STRICT) unocc_update_strict<F>(acc[jj], cm[jj], an, wt, ie, wxv);
+                else unocc_update_fast<F>(acc[jj], cm[jj], an, wt, ie, wxv);
             }
         }
-        if (c + 1 < nchunks) store_chunk(buf ^ 1);
+        if (c + 1 < c1) store_chunk(buf ^ 1);
         __syncthreads();
     }
 
     if (!band_ok) return;
     // scht per (column, frequency); then sum_j (0.5*scht)*vcoul[igp] in
-    // column order (gppComplex.cpp:374, :379).
+    // column order (gppComplex.cpp:374, :379).  The wave's sums by the xor
+    // butterfly of wave_sum (the same additions), each step on the half of the
+    // values this lane goes on with: after three steps lane l holds F of its
+    // column's 2 F parts (10 F exchanges of doubles instead of 48 F).
+    static_assert(kBJ == 4, "two steps split the columns, one the parts");
+    double v[kBJ * 2 * F];
 #pragma unroll
-    for (int f = 0; f < FC; ++f) {
-        cplx s = czero();
+    for (int jj = 0; jj < kBJ; ++jj)
+#pragma unroll
+        for (int f = 0; f < F; ++f) {
+            v[(jj * F + f) * 2] = acc[jj][f].re;
+            v[(jj * F + f) * 2 + 1] = acc[jj][f].im;
+        }
+    int n = kBJ * F;  // half of the values held
+#pragma unroll
+    for (int m = 1; m <= 4; m <<= 1, n /= 2) {
+        const bool up = lane & m;
+#pragma unroll
+        for (int i = 0; i < n; ++i) {
+            const double keep = up ? v[n + i] : v[i], give = up ? v[i] : v[n + i];
+            v[i] = keep + __shfl_xor(give, m, kWave);
+        }
+    }
+    const int col = 2 * (lane & 1) + ((lane >> 1) & 1);  // this lane's column
+    const double vc = a.vcoul[igp_of(a.idx, min(j0 + col, a.ngpown - 1), ncouls)];
+    double s[F];
+#pragma unroll
+    for (int i = 0; i < F; ++i) {
+        for (int m = 8; m < kWave; m <<= 1) v[i] += __shfl_xor(v[i], m, kWave);
+        v[i] = v[i] * 0.5 * vc;
+        s[i] = 0.0;
 #pragma unroll
         for (int jj = 0; jj < kBJ; ++jj) {
-            const cplx scht = wave_sum(acc[jj][f]);
-            const int j = j0 + jj;
-            if (j < a.ngpown) cacc(s, cscale(cscale(scht, 0.5), a.vcoul[igp_of(a.idx, j, ncouls)]));
+            const double t = __shfl(v[i], (lane & ~3) | (jj >> 1) | ((jj & 1) << 1), kWave);
+            if (j0 + jj < a.ngpown) s[i] = t + s[i];
         }
-        if (lane == 0 && iw0 + f < a.nfreq) a.part_ach[((size_t)n1 * a.njt + jt) * a.nfreq + iw0 + f] = s;
     }
-    stamp.store();
+    if ((lane & ~4) == 0) {  // lane 0: the first F parts, lane 4: the others
+        double *o = &a.part_ach[((size_t)n1 * a.nt + jt * a.gs + g) * a.nfreq + iw0].re + (lane ? F : 0);
+#pragma unroll
+        for (int i = 0; i < F; ++i) o[i] = s[i];
+    }
 }
 
-// ---------------------------------------------------------------------------
-// Occupied bands n1 < nv.  Grid (njt, nv, ceil(nfreq/FC)), block 4 waves;
-// wave w owns columns j0 + w*kOccCols .. +kOccCols-1 of the block's tile and
-// strides over ig itself.  The four waves' column sums are combined in
-// column order through LDS.
-template <int FC>
-__global__ __launch_bounds__(kOccWaves *kWave) void k_occ(DirectArgs a)
+// Occupied bands n1 < nv: block b of their share, 4 columns of one band over
+// one G range; waves jj and jj + 4 take column jj over the range's halves.  The
+// sums are combined half by half, then in column order, through LDS.
+template <int F>
+__device__ __forceinline__ void occ_block(const DirectArgs &a, int ncouls, int b, int iw0, cplx *lds)
 {
-    int ncouls = a.ncouls;
-    const StampStart stamp(a.stamp, ncouls);
-    __shared__ cplx s_ach[kBJ][FC];
-    __shared__ cplx s_asx[kBJ][FC];
+    auto *s_sum = reinterpret_cast<cplx(*)[2][kBJ][F]>(lds);  // [ach, asx][half][column]
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
     const int lane = threadIdx.x % kWave;
-    const int jt = blockIdx.x;
-    const int n1 = blockIdx.y;
-    const int iw0 = blockIdx.z * FC;
+    const int jj = wave % kBJ, half = wave / kBJ;
+    const int jt = b % a.njt, n1 = (b / a.njt) % a.nv, g = b / (a.njt * a.nv);
+    const int j = jt * kBJ + jj;
+    const bool ok = j < a.ngpown;
 
-    double wxv[FC], wx2[FC], rwx4[FC];
+    double wxv[F], wx2[F], rwx4[F];
 #pragma unroll
-    for (int f = 0; f < FC; ++f) {
-        wxv[f] = (iw0 + f < a.nfreq) ? a.wx[(size_t)n1 * a.wx_stride + iw0 + f] : 1.0;
+    for (int f = 0; f < F; ++f) {
+        wxv[f] = a.wx[(size_t)n1 * a.wx_stride + iw0 + f];
         // std::pow(wxt,2) and std::pow(cden,2), gppComplex.cpp:38-40
         wx2[f] = wxv[f] * wxv[f];
         rwx4[f] = 1.00 / (wx2[f] * wx2[f]);
     }
-
-    cplx ssxt[kOccCols][FC], scht[kOccCols][FC];
+    cplx ssxt[F], scht[F];
 #pragma unroll
-    for (int c = 0; c < kOccCols; ++c)
+    for (int f = 0; f < F; ++f) ssxt[f] = scht[f] = czero();
+    if (ok) {
+        const cplx mv1 = cconj(a.aqsm[(size_t)n1 * ncouls + igp_of(a.idx, j, ncouls)]);
+        int c0, c1;
+        range_chunks(a, ncouls, g, c0, c1);
+        const int mid = (c0 + c1 + 1) / 2;
+        const int end = (half ? c1 : mid) * kWave < ncouls ? (half ? c1 : mid) * kWave : ncouls;
+        for (int ig = (half ? mid : c0) * kWave + lane; ig < end; ig += kWave) {
+            const cplx an = a.aqsn[(size_t)n1 * ncouls + ig];
+            const cplx wt = a.wtilde[(size_t)j * ncouls + ig];
+            const cplx ie = a.ieps[(size_t)j * ncouls + ig];
+            const cplx m = cmul(an, mv1);  // matngmatmgp, gppComplex.cpp:121
 #pragma unroll
-        for (int f = 0; f < FC; ++f) ssxt[c][f] = scht[c][f] = czero();
-
-    int jcol[kOccCols];
-    cplx mv1[kOccCols];
-#pragma unroll
-    for (int c = 0; c < kOccCols; ++c) {
-        jcol[c] = jt * kBJ + wave * kOccCols + c;
-        mv1[c] = czero();
-        if (jcol[c] < a.ngpown) mv1[c] = cconj(a.aqsm[(size_t)n1 * ncouls + igp_of(a.idx, jcol[c], ncouls)]);
-    }
-
-    for (int ig = lane; ig < ncouls; ig += kWave) {
-        const cplx an = a.aqsn[(size_t)n1 * ncouls + ig];
-#pragma unroll
-        for (int c = 0; c < kOccCols; ++c) {
-            if (jcol[c] >= a.ngpown) continue;
-            const size_t off = (size_t)jcol[c] * ncouls + ig;
-            const cplx wt = a.wtilde[off];
-            const cplx ie = a.ieps[off];
-            const cplx m = cmul(an, mv1[c]);  // matngmatmgp, gppComplex.cpp:121
-#pragma unroll
-            for (int f = 0; f < FC; ++f) {
+            for (int f = 0; f < F; ++f) {
                 cplx sch, ssx;
                 occ_pole_terms(wxv[f], wx2[f], rwx4[f], wt, ie, sch, ssx);
-                cacc(ssxt[c][f], cmul(m, ssx));  // :61, :125
-                cacc(scht[c][f], cmul(m, sch));  // :62, :126
+                cacc(ssxt[f], cmul(m, ssx));  // :61, :125
+                cacc(scht[f], cmul(m, sch));  // :62, :126
             }
         }
     }
-
 #pragma unroll
-    for (int c = 0; c < kOccCols; ++c) {
-        const int jj = wave * kOccCols + c;
-        const bool ok = jcol[c] < a.ngpown;
-        const double vc = ok ? a.vcoul[igp_of(a.idx, jcol[c], ncouls)] : 0.0;
-#pragma unroll
-        for (int f = 0; f < FC; ++f) {
-            const cplx sx = wave_sum(ssxt[c][f]);
-            const cplx sc = wave_sum(scht[c][f]);
-            if (lane == 0) {
-                // achtemp: (0.5*scht)*vcoul (:361, :379); asxtemp: ssxt*(occ*vcoul) (:363)
-                s_ach[jj][f] = ok ? cscale(cscale(sc, 0.5), vc) : czero();
-                s_asx[jj][f] = ok ? cscale(sx, a.occ * vc) : czero();
-            }
+    for (int f = 0; f < F; ++f) {
+        const cplx sx = wave_sum(ssxt[f]);
+        const cplx sc = wave_sum(scht[f]);
+        if (lane == 0) {
+            s_sum[0][half][jj][f] = sc;
+            s_sum[1][half][jj][f] = sx;
         }
     }
     __syncthreads();
-    if (threadIdx.x < FC && iw0 + (int)threadIdx.x < a.nfreq) {
+    if (threadIdx.x < F) {
         const int f = threadIdx.x;
         cplx sa = czero(), sx = czero();
-        for (int jj = 0; jj < kBJ; ++jj) {
-            cacc(sa, s_ach[jj][f]);
-            cacc(sx, s_asx[jj][f]);
+        for (int q = 0; q < kBJ && jt * kBJ + q < a.ngpown; ++q) {
+            // achtemp: (0.5*scht)*vcoul (:361, :379); asxtemp: ssxt*(occ*vcoul) (:363)
+            const double vc = a.vcoul[igp_of(a.idx, jt * kBJ + q, ncouls)];
+            cacc(sa, cscale(cscale(cadd(s_sum[0][0][q][f], s_sum[0][1][q][f]), 0.5), vc));
+            cacc(sx, cscale(cadd(s_sum[1][0][q][f], s_sum[1][1][q][f]), a.occ * vc));
         }
-        const size_t o = ((size_t)n1 * a.njt + jt) * a.nfreq + iw0 + f;
+        const size_t o = ((size_t)n1 * a.nt + jt * a.gs + g) * a.nfreq + iw0 + f;
         a.part_ach[o] = sa;
         a.part_asx[o] = sx;
+    }
+}
+
+// One band kind's block `b` of frequency pass z: W frequencies, the last pass
+// as many as remain.
+template <int W, bool STRICT, bool OCC>
+__device__ __forceinline__ void direct_pass(const DirectArgs &a, int ncouls, int b, int z, cplx *lds)
+{
+    const int iw0 = W * z, left = a.nfreq - iw0;
+    const auto run = [&](auto f) {
+        if constexpr (OCC)
+            occ_block<decltype(f)::value>(a, ncouls, b, iw0, lds);
+        else
+            unocc_block<decltype(f)::value, STRICT>(a, ncouls, b, iw0, lds);
+    };
+    if (left >= W) {
+        run(std::integral_constant<int, W>());
+    } else if (W > 3 && left == 3) {
+        run(std::integral_constant<int, (W > 3 ? 3 : W)>());
+    } else if (W > 2 && left == 2) {
+        run(std::integral_constant<int, (W > 2 ? 2 : W)>());
+    } else if (W > 1) {
+        run(std::integral_constant<int, 1>());
+    }
+}
+
+// 1-D grid: occ_blocks, ach_blocks, then the unoccupied bands'.
+template <int W, bool STRICT>
+__global__ __launch_bounds__(kNW *kWave) __attribute__((amdgpu_waves_per_eu(4))) void k_direct(DirectArgs a)
+{
+    int ncouls = a.ncouls;
+    const StampStart stamp(a.stamp, ncouls);
+    __shared__ cplx lds[4 * kBJ * kWave];
+    const int b = blockIdx.x;
+    if (b < a.occ_blocks) {
+        direct_pass<W, STRICT, true>(a, ncouls, b / a.nz, b % a.nz, lds);
+    } else if (b < a.occ_blocks + a.ach_blocks) {
+        const int item = (b - a.occ_blocks) * kNW + threadIdx.x / kWave;  // band * kAchSplit + column group
+        if (item < a.nb * kAchSplit) {
+            const auto col = [&](int j) { return ach_col(a.ieps, a.idx, a.vcoul, ncouls, j); };
+            const cplx s = achstemp_band(a.aqsm, a.aqsn, col, ncouls, a.ngpown, item / kAchSplit, item % kAchSplit,
+                                         nullptr);
+            if (threadIdx.x % kWave == 0) a.part_achs[item] = s;
+        }
+    } else {
+        const int u = b - a.occ_blocks - a.ach_blocks;
+        direct_pass<W, STRICT, false>(a, ncouls, u / a.nz, u % a.nz, lds);
     }
     stamp.store();
 }
@@ -372,37 +489,39 @@ hipError_t launch_ach(const DirectArgs &a, hipStream_t s)
     return hipGetLastError();
 }
 
-// Per band: partials over column tiles -> band_ach[n1][iw] (and band_asx
-// for occupied bands).  Grid nb, block kReduceThreads.
-__global__ __launch_bounds__(kReduceThreads) void k_reduce_bands(DirectArgs a, int n1_begin)
+// Per (band, frequency), one wave: the partials over column tiles and G ranges
+// -> band_ach[n1][iw] (and band_asx for occupied bands).
+__global__ __launch_bounds__(kReduceThreads) void k_reduce_bands(DirectArgs a, int n1_begin, int n1_end)
 {
-    __shared__ cplx scratch[kReduceThreads / kWave];
-    const int n1 = n1_begin + blockIdx.x;
-    for (int iw = 0; iw < a.nfreq; ++iw) {
-        cplx s = czero(), x = czero();
-        for (int t = threadIdx.x; t < a.njt; t += blockDim.x) {
-            const size_t o = ((size_t)n1 * a.njt + t) * a.nfreq + iw;
-            s = cadd(s, a.part_ach[o]);
-            if (n1 < a.nv) x = cadd(x, a.part_asx[o]);
-        }
-        s = block_sum(s, scratch);
-        if (threadIdx.x == 0) a.band_ach[(size_t)n1 * a.nfreq + iw] = s;
-        if (n1 < a.nv) {
-            x = block_sum(x, scratch);
-            if (threadIdx.x == 0) a.band_asx[(size_t)n1 * a.nfreq + iw] = x;
-        }
+    stamp_start(a.stamp);
+    const int pair = blockIdx.x * (kReduceThreads / kWave) + threadIdx.x / kWave;
+    const int n1 = n1_begin + pair / a.nfreq, iw = pair % a.nfreq, lane = threadIdx.x % kWave;
+    if (n1 >= n1_end) return;
+    cplx s = czero(), x = czero();
+    for (int t = lane; t < a.nt; t += kWave) {
+        const size_t o = ((size_t)n1 * a.nt + t) * a.nfreq + iw;
+        s = cadd(s, a.part_ach[o]);
+        if (n1 < a.nv) x = cadd(x, a.part_asx[o]);
+    }
+    s = wave_sum(s);
+    x = wave_sum(x);
+    if (lane == 0) {
+        a.band_ach[(size_t)n1 * a.nfreq + iw] = s;
+        if (n1 < a.nv) a.band_asx[(size_t)n1 * a.nfreq + iw] = x;
     }
 }
 
-// Final pass, one block: achtemp, asxtemp, acht_n1_loc, achstemp for bands
-// [n1_begin, n1_end) (achstemp only when with_achs).
-__global__ __launch_bounds__(kReduceThreads) void k_reduce_final(DirectArgs a, cplx *out, int n1_begin,
+// Final pass over bands [n1_begin, n1_end): block iw < nfreq forms achtemp[iw]
+// and asxtemp[iw], block nfreq acht_n1_loc and (with_achs) achstemp -- written
+// to out (DevResults), or, with out null, added to the reference launchers'
+// split outputs unless the index check found negative entries.
+__global__ __launch_bounds__(kReduceThreads) void k_reduce_final(DirectArgs a, cplx *out, CompatOut co, int n1_begin,
                                                                  int n1_end, int with_achs)
 {
     __shared__ cplx scratch[kReduceThreads / kWave];
-    const int nf = a.nfreq;
-    const int acht_iw = nf > 2 ? 2 : nf - 1;  // gppComplex.cpp:381
-    for (int iw = 0; iw < nf; ++iw) {
+    const int nf = a.nfreq, iw = blockIdx.x;
+    const bool add = !out && !(co.bad && *co.bad);
+    if (iw < nf) {
         cplx s = czero(), x = czero();
         for (int n1 = n1_begin + threadIdx.x; n1 < n1_end; n1 += blockDim.x) {
             s = cadd(s, a.band_ach[(size_t)n1 * nf + iw]);
@@ -411,17 +530,37 @@ __global__ __launch_bounds__(kReduceThreads) void k_reduce_final(DirectArgs a, c
         s = block_sum(s, scratch);
         x = block_sum(x, scratch);
         if (threadIdx.x == 0) {
-            out[iw] = s;
-            out[nf + iw] = x;
+            if (out) {
+                out[iw] = s;
+                out[nf + iw] = x;
+            } else if (add) {
+                if (co.achtemp_re) co.achtemp_re[iw] += s.re;
+                if (co.achtemp_im) co.achtemp_im[iw] += s.im;
+                if (co.asxtemp) cacc(co.asxtemp[iw], x);
+            }
+        }
+    } else {
+        const int acht_iw = nf > 2 ? 2 : nf - 1;  // gppComplex.cpp:381
+        if (out) {
+            for (int n1 = threadIdx.x; n1 < a.nb; n1 += blockDim.x)
+                out[2 * nf + n1] = (n1 >= n1_begin && n1 < n1_end) ? a.band_ach[(size_t)n1 * nf + acht_iw] : czero();
+        } else if (add && co.acht_n1) {
+            for (int n1 = n1_begin + threadIdx.x; n1 < n1_end; n1 += blockDim.x)
+                cacc(co.acht_n1[n1], a.band_ach[(size_t)n1 * nf + acht_iw]);
+        }
+        cplx h = czero();
+        if (with_achs)
+            for (int t = threadIdx.x; t < a.nb * kAchSplit; t += blockDim.x) h = cadd(h, a.part_achs[t]);
+        h = block_sum(h, scratch);
+        if (threadIdx.x == 0) {
+            if (out) {
+                out[2 * nf + a.nb] = h;
+            } else if (add && with_achs) {
+                co.achstemp_re[0] += h.re;
+                co.achstemp_im[0] += h.im;
+            }
         }
     }
-    for (int n1 = threadIdx.x; n1 < a.nb; n1 += blockDim.x)
-        out[2 * nf + n1] = (n1 >= n1_begin && n1 < n1_end) ? a.band_ach[(size_t)n1 * nf + acht_iw] : czero();
-    cplx h = czero();
-    if (with_achs)
-        for (int t = threadIdx.x; t < a.nb * kAchSplit; t += blockDim.x) h = cadd(h, a.part_achs[t]);
-    h = block_sum(h, scratch);
-    if (threadIdx.x == 0) out[2 * nf + a.nb] = h;
     stamp_end(a.end);
 }
 
@@ -437,70 +576,67 @@ __global__ void k_check_index(const int32_t *idx, int n, int *count)
     if (bad) atomicAdd(count, bad);
 }
 
-// Accumulates results into the reference launchers' split outputs.
-// which: 0 occupied (achtemp, asxtemp, acht_n1_loc[0..nv)), 1 unoccupied
-// (achtemp, acht_n1_loc[nv..nb)), 2 achstemp.
-__global__ void k_accumulate_compat(const cplx *res, int nfreq, int nb, int which, int nv,
-                                    double *ach_re, double *ach_im, cplx *asx, cplx *acht_n1,
-                                    double *achs_re, double *achs_im)
+// One block: the negative entries counted into *count and, for a host that
+// polls it, *host (pinned memory).
+__global__ __launch_bounds__(1024) void k_check_index_once(const int32_t *idx, int n, int *count, int *host)
 {
-    const int t = threadIdx.x;
-    if (which == 2) {
-        if (t == 0) {
-            achs_re[0] += res[2 * nfreq + nb].re;
-            achs_im[0] += res[2 * nfreq + nb].im;
+    __shared__ int total;
+    if (threadIdx.x == 0) total = 0;
+    __syncthreads();
+    int bad = 0;
+    for (int i = threadIdx.x; i < n; i += blockDim.x) bad += idx[i] < 0;
+    if (bad) atomicAdd(&total, bad);
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        *count = total;
+        __hip_atomic_store(host, total, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+    }
+}
+
+// The bands' blocks (occ, unocc) and the achstemp partials (achs) in one launch.
+hipError_t launch_direct(DirectArgs &a, bool strict, bool occ, bool achs, bool unocc, hipStream_t s)
+{
+    const int w = std::min(a.nfreq, pass_width(strict));
+    a.nz = (a.nfreq + w - 1) / w;
+    a.occ_blocks = occ ? a.nt * a.nv * a.nz : 0;
+    a.ach_blocks = achs ? (a.nb * kAchSplit + kNW - 1) / kNW : 0;
+    const int nun = unocc ? a.nb - a.nv : 0;
+    const unsigned blocks =
+        (unsigned)a.occ_blocks + (unsigned)a.ach_blocks + (unsigned)((nun + kNW - 1) / kNW) * (unsigned)(a.nt * a.nz);
+    if (blocks == 0) return hipSuccess;
+    const dim3 grid(blocks), block(kNW * kWave);
+    if (strict)
+        switch (w) {
+        case 1: hipLaunchKernelGGL((k_direct<1, true>), grid, block, 0, s, a); break;
+        case 2: hipLaunchKernelGGL((k_direct<2, true>), grid, block, 0, s, a); break;
+        default: hipLaunchKernelGGL((k_direct<3, true>), grid, block, 0, s, a); break;
         }
-        return;
-    }
-    if (t < nfreq) {
-        ach_re[t] += res[t].re;
-        ach_im[t] += res[t].im;
-        if (which == 0 && asx) cacc(asx[t], res[nfreq + t]);
-    }
-    if (acht_n1) {
-        const int lo = which == 0 ? 0 : nv, hi = which == 0 ? nv : nb;
-        for (int n1 = lo + t; n1 < hi; n1 += blockDim.x) cacc(acht_n1[n1], res[2 * nfreq + n1]);
-    }
-}
-
-template <int FC>
-hipError_t launch_unocc_fc(const DirectArgs &a, bool strict, hipStream_t s)
-{
-    const int nun = a.nb - a.nv;
-    if (nun <= 0 || a.ngpown <= 0) return hipSuccess;
-    dim3 grid((nun + kNW - 1) / kNW, a.njt, (a.nfreq + FC - 1) / FC);
-    if (strict) hipLaunchKernelGGL((k_unocc<FC, true>), grid, dim3(kNW * kWave), 0, s, a);
-    else hipLaunchKernelGGL((k_unocc<FC, false>), grid, dim3(kNW * kWave), 0, s, a);
+    else
+        switch (w) {
+        case 1: hipLaunchKernelGGL((k_direct<1, false>), grid, block, 0, s, a); break;
+        case 2: hipLaunchKernelGGL((k_direct<2, false>), grid, block, 0, s, a); break;
+        case 3: hipLaunchKernelGGL((k_direct<3, false>), grid, block, 0, s, a); break;
+        default: hipLaunchKernelGGL((k_direct<4, false>), grid, block, 0, s, a); break;
+        }
     return hipGetLastError();
 }
 
-template <int FC>
-hipError_t launch_occ_fc(const DirectArgs &a, hipStream_t s)
+// Bands [n1_begin, n1_end) of the partials to the results.
+hipError_t launch_reduce(const DirectArgs &a, cplx *out, const CompatOut &co, int n1_begin, int n1_end, int with_achs,
+                         hipStream_t s)
 {
-    if (a.nv <= 0 || a.ngpown <= 0) return hipSuccess;
-    dim3 grid(a.njt, a.nv, (a.nfreq + FC - 1) / FC);
-    hipLaunchKernelGGL((k_occ<FC>), grid, dim3(kOccWaves * kWave), 0, s, a);
+    const long long pairs = (long long)(n1_end - n1_begin) * a.nfreq;
+    DirectArgs f = a;
+    f.stamp = Stamp{};
+    if (pairs > 0) {
+        DirectArgs b = a;
+        b.end = nullptr;
+        hipLaunchKernelGGL(k_reduce_bands, dim3((unsigned)((pairs + 3) / 4)), dim3(kReduceThreads), 0, s, b, n1_begin,
+                           n1_end);
+    }
+    hipLaunchKernelGGL(k_reduce_final, dim3(a.nfreq + 1), dim3(kReduceThreads), 0, s, f, out, co, n1_begin, n1_end,
+                       with_achs);
     return hipGetLastError();
-}
-
-hipError_t launch_unocc(const DirectArgs &a, bool strict, hipStream_t s)
-{
-    switch (a.nfreq) {
-    case 1: return launch_unocc_fc<1>(a, strict, s);
-    case 2: return launch_unocc_fc<2>(a, strict, s);
-    case 3: return launch_unocc_fc<3>(a, strict, s);
-    default: return launch_unocc_fc<4>(a, strict, s);
-    }
-}
-
-hipError_t launch_occ(const DirectArgs &a, hipStream_t s)
-{
-    switch (a.nfreq) {
-    case 1: return launch_occ_fc<1>(a, s);
-    case 2: return launch_occ_fc<2>(a, s);
-    case 3: return launch_occ_fc<3>(a, s);
-    default: return launch_occ_fc<4>(a, s);
-    }
 }
 
 #define GPP_TRY(x)                         \
@@ -519,42 +655,21 @@ hipError_t run_direct(const DevProblem &p, bool strict, void *work, const DevRes
     DirectArgs a = make_args(p, work);
     const auto stage = [&](const char *nm) { a.stamp = timer ? timer->stage(nm) : Stamp{}; };
     if (timer) timer->begin();
-    if (p.nv > 0) stage("direct_occupied");
-    GPP_TRY(launch_occ(a, s));
-    if (p.nb > p.nv) stage(strict ? "direct_unoccupied_strict" : "direct_unoccupied");
-    GPP_TRY(launch_unocc(a, strict, s));
+    stage(p.nb == p.nv ? "direct_occupied" : strict ? "direct_unoccupied_strict" : "direct_unoccupied");
+    GPP_TRY(launch_direct(a, strict, true, true, true, s));
     stage("direct_reduce");
-    GPP_TRY(launch_ach(a, s));
-    hipLaunchKernelGGL(k_reduce_bands, dim3(p.nb), dim3(kReduceThreads), 0, s, a, 0);
-    GPP_TRY(hipGetLastError());
     if (timer) a.end = timer->end();
-    hipLaunchKernelGGL(k_reduce_final, dim3(1), dim3(kReduceThreads), 0, s, a, res.base, 0, p.nb, 1);
-    return hipGetLastError();
+    return launch_reduce(a, res.base, CompatOut{}, 0, p.nb, 1, s);
 }
 
-hipError_t run_direct_part(const DevProblem &p, int which, void *work, const DevResults &res,
-                           hipStream_t s)
+hipError_t run_direct_part(const DevProblem &p, int which, void *work, const CompatOut &co, hipStream_t s)
 {
-    const DirectArgs a = make_args(p, work);
-    if (which == 0) {
-        GPP_TRY(launch_occ(a, s));
-        if (p.nv > 0) {
-            hipLaunchKernelGGL(k_reduce_bands, dim3(p.nv), dim3(kReduceThreads), 0, s, a, 0);
-            GPP_TRY(hipGetLastError());
-        }
-        hipLaunchKernelGGL(k_reduce_final, dim3(1), dim3(kReduceThreads), 0, s, a, res.base, 0, p.nv, 0);
-    } else if (which == 1) {
-        GPP_TRY(launch_unocc(a, false, s));
-        if (p.nb > p.nv) {
-            hipLaunchKernelGGL(k_reduce_bands, dim3(p.nb - p.nv), dim3(kReduceThreads), 0, s, a, p.nv);
-            GPP_TRY(hipGetLastError());
-        }
-        hipLaunchKernelGGL(k_reduce_final, dim3(1), dim3(kReduceThreads), 0, s, a, res.base, p.nv, p.nb, 0);
-    } else {
-        if (p.nb > 0) GPP_TRY(launch_ach(a, s));
-        hipLaunchKernelGGL(k_reduce_final, dim3(1), dim3(kReduceThreads), 0, s, a, res.base, 0, 0, 1);
-    }
-    return hipGetLastError();
+    DirectArgs a = make_args(p, work);
+    a.stamp = Stamp{};
+    GPP_TRY(launch_direct(a, false, which == 0, which == 2, which == 1, s));
+    if (which == 0) return launch_reduce(a, nullptr, co, 0, p.nv, 0, s);
+    if (which == 1) return launch_reduce(a, nullptr, co, p.nv, p.nb, 0, s);
+    return launch_reduce(a, nullptr, co, 0, 0, 1, s);
 }
 
 hipError_t launch_achstemp(const DevProblem &p, cplx *part_achs, cplx *bg, Stamp stamp, hipStream_t s)
@@ -581,12 +696,9 @@ hipError_t launch_zero_ints(int *d_p, int n, hipStream_t s)
     return hipGetLastError();
 }
 
-hipError_t launch_accumulate_compat(const DevResults &res, int which, int nv, double *achtemp_re,
-                                    double *achtemp_im, cplx *asxtemp, cplx *acht_n1_loc,
-                                    double *achstemp_re, double *achstemp_im, hipStream_t s)
+hipError_t launch_check_index_once(const int32_t *d_idx, int ngpown, int *d_count, int *host, hipStream_t s)
 {
-    hipLaunchKernelGGL(k_accumulate_compat, dim3(1), dim3(256), 0, s, res.base, res.nfreq, res.nb, which,
-                       nv, achtemp_re, achtemp_im, asxtemp, acht_n1_loc, achstemp_re, achstemp_im);
+    hipLaunchKernelGGL(k_check_index_once, dim3(1), dim3(1024), 0, s, d_idx, ngpown, d_count, host);
     return hipGetLastError();
 }
 

@@ -95,11 +95,19 @@ size_t direct_workspace_bytes(const DevProblem &p);
 hipError_t run_direct(const DevProblem &p, bool strict, void *work, const DevResults &res,
                       hipStream_t s, StageTimer *timer);
 
-// Only the occupied bands (n1 < nv) / only the unoccupied bands of the direct
-// form, plus achstemp, for the reference-compatible launchers.  `which`
-// selects 0 = occupied, 1 = unoccupied, 2 = achstemp.
-hipError_t run_direct_part(const DevProblem &p, int which, void *work, const DevResults &res,
-                           hipStream_t s);
+// The reference launchers' split outputs (nfreq = 3), added to; bad: device
+// count of negative indices, nonzero leaves them alone (null: none).
+struct CompatOut {
+    double *achtemp_re = nullptr, *achtemp_im = nullptr;
+    cplx *asxtemp = nullptr, *acht_n1 = nullptr;
+    double *achstemp_re = nullptr, *achstemp_im = nullptr;
+    const int *bad = nullptr;
+};
+
+// Only the occupied bands (n1 < nv) / only the unoccupied bands / only
+// achstemp of the direct form, for the reference-compatible launchers.
+// `which` selects 0 = occupied, 1 = unoccupied, 2 = achstemp.
+hipError_t run_direct_part(const DevProblem &p, int which, void *work, const CompatOut &co, hipStream_t s);
 
 // achstemp per band into part_achs[nb] (fixed-order sums over j); with bg non-null also the gathered
 // rows Bg[n1][j] = aqsm[n1][igp(j)] [nb][ngpown].
@@ -111,10 +119,9 @@ hipError_t launch_zero_ints(int *d_p, int n, hipStream_t s);
 // Counts negative inv_igp_index entries on the device (result in *d_count).
 hipError_t launch_check_index(const int32_t *d_idx, int ngpown, int *d_count, hipStream_t s);
 
-// Adds res (nfreq=3 layout) into reference-style split outputs.
-hipError_t launch_accumulate_compat(const DevResults &res, int which, int nv, double *achtemp_re,
-                                    double *achtemp_im, cplx *asxtemp, cplx *acht_n1_loc,
-                                    double *achstemp_re, double *achstemp_im, hipStream_t s);
+// The same in one launch, into *d_count (overwritten) and *host, pinned memory
+// that the caller polls.
+hipError_t launch_check_index_once(const int32_t *d_idx, int ngpown, int *d_count, int *host, hipStream_t s);
 
 // Seeded input generation on the device (counter-based hash, identical bits
 // to the host generator).
