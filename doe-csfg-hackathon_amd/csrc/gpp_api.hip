@@ -9,6 +9,7 @@
 #include <mutex>
 #include <new>
 #include <tuple>
+#include <utility>
 #include <errno.h>
 #include <stdarg.h>
 #include <stdio.h>
@@ -205,6 +206,7 @@ struct gpp_ctx {
     // band-dependent frequencies (gpp_set_band_frequencies)
     bool per_band = false;
     DevBuf wxb;                     // [nb][nfreq]
+    DevBuf btab;                    // the bucket plan's tables
     gpp::BucketPlan bplan;          // bands grouped by identical rows
     gpp_form last_form = GPP_FORM_DIRECT;
     bool have_last_form = false;  // an evaluation was enqueued on the current inputs
@@ -338,7 +340,7 @@ gpp_status gpp_ctx_destroy(gpp_ctx *ctx)
     if (ctx->stream) (void)hipStreamSynchronize(ctx->stream);
     ctx->idx.release(); ctx->wx.release(); ctx->vcoul.release();
     ctx->aqsm.release(); ctx->aqsn.release(); ctx->ieps.release(); ctx->wtilde.release();
-    ctx->results.release(); ctx->flag.release(); ctx->wxb.release();
+    ctx->results.release(); ctx->flag.release(); ctx->wxb.release(); ctx->btab.release();
     ctx->work.release();
     if (ctx->host_results) (void)hipHostFree(ctx->host_results);
     ctx->timer.destroy();
@@ -658,11 +660,19 @@ gpp_status gpp_set_band_frequencies(gpp_ctx *ctx, const double *wx_bands)
             return fail(GPP_ERR_INVALID_ARGUMENT, "wx_bands[%zu] is NaN", i);
     gpp_status st = set_device(ctx);
     if (st) return st;
+    ctx->per_band = false;  // a failure below leaves the shared row
     HIP_OR_FAIL(ctx->wxb.ensure(sizeof(double) * nb * nf), "hipMalloc wx_bands");
     HIP_OR_FAIL(hipMemcpyAsync(ctx->wxb.ptr, wx_bands, sizeof(double) * nb * nf, hipMemcpyHostToDevice, ctx->stream),
                 "H2D wx_bands");
+    gpp::BucketPlan plan = gpp::plan_buckets(wx_bands, nb, ctx->dp.nv, nf);
+    const std::vector<int32_t> tables = plan.tables();
+    HIP_OR_FAIL(ctx->btab.ensure(sizeof(int32_t) * tables.size()), "hipMalloc band groups");
+    HIP_OR_FAIL(hipMemcpyAsync(ctx->btab.ptr, tables.data(), sizeof(int32_t) * tables.size(), hipMemcpyHostToDevice,
+                               ctx->stream),
+                "H2D band groups");
     HIP_OR_FAIL(hipStreamSynchronize(ctx->stream), "wx_bands synchronize");
-    ctx->bplan = gpp::plan_buckets(wx_bands, nb, ctx->dp.nv, nf);
+    plan.dev = static_cast<const int32_t *>(ctx->btab.ptr);
+    ctx->bplan = std::move(plan);
     ctx->per_band = true;
     return GPP_OK;
 }

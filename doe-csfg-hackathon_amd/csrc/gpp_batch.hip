@@ -61,7 +61,8 @@ __global__ __launch_bounds__(kRedThreads) void k_batch_achstemp(const BInst *__r
         const BInst &b = insts[it.x];  // it.y = band * kAchSplit + column group
         const AchCol *cols = reinterpret_cast<const AchCol *>(b.part_achs + ach_cols_entry(b.nb));
         const cplx s = achstemp_band(b.aqsm, b.aqsn, [&](int j) { return cols[j]; }, b.ncouls, b.ngpown,
-                                     it.y / kAchSplit, it.y % kAchSplit, b.bg);
+                                     it.y / kAchSplit, it.y % kAchSplit,
+                                     b.bg + (size_t)(it.y / kAchSplit) * b.ngpown);
         if (threadIdx.x % kWave == 0) b.part_achs[it.y] = s;
     }
 }

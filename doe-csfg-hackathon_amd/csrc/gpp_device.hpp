@@ -350,7 +350,7 @@ __device__ __forceinline__ cplx achstemp_band(const cplx *aqsm, const cplx *aqsn
     for (int j = q * kWave + threadIdx.x % kWave; j < ngpown; j += kAchSplit * kWave) {
         const AchCol c = col(j);
         const cplx m = aqsm[(size_t)n1 * ncouls + c.igp];
-        if (bg) bg[(size_t)n1 * ngpown + j] = m;
+        if (bg) bg[j] = m;
         if (c.sre != 0.0 || c.sim != 0.0) {  // |schs| > to1: schs is nonzero
             const cplx matngmatmgp = cmul(aqsn[(size_t)n1 * ncouls + c.igp], cconj(m));  // :84, :89
             cplx schstemp = czero();

@@ -62,6 +62,7 @@ struct DirectArgs {
     cplx *band_ach;   // [nb][nfreq]
     cplx *band_asx;   // [max(nv,1)][nfreq]
     cplx *bg;         // optional gathered rows of aqsm (factored forms), else null
+    const int32_t *perm;  // achstemp launch: row r of bg and part_achs is band perm[r] (null: r)
     Stamp stamp;      // the launch's stage start
     unsigned long long *end;  // the evaluation's end (last launch)
 };
@@ -132,6 +133,7 @@ DirectArgs make_args(const DevProblem &p, void *work)
     a.band_ach = reinterpret_cast<cplx *>(w + L.band_ach);
     a.band_asx = reinterpret_cast<cplx *>(w + L.band_asx);
     a.bg = nullptr;
+    a.perm = nullptr;
     a.end = nullptr;
     return a;
 }
@@ -460,7 +462,9 @@ __global__ __launch_bounds__(kAchWaves * kWave) void k_achstemp(DirectArgs a)
     if (item >= a.nb * kAchSplit) return;
     const AchCol *cols = reinterpret_cast<const AchCol *>(a.part_achs + ach_cols_entry(a.nb));
     const auto col = [&](int j) { return COLS ? cols[j] : ach_col(a.ieps, a.idx, a.vcoul, a.ncouls, j); };
-    const cplx s = achstemp_band(a.aqsm, a.aqsn, col, a.ncouls, a.ngpown, item / kAchSplit, item % kAchSplit, a.bg);
+    const int r = item / kAchSplit, n1 = a.perm ? a.perm[r] : r;
+    const cplx s = achstemp_band(a.aqsm, a.aqsn, col, a.ncouls, a.ngpown, n1, item % kAchSplit,
+                                 a.bg ? a.bg + (size_t)r * a.ngpown : nullptr);
     if (threadIdx.x % kWave == 0) a.part_achs[item] = s;
 }
 
@@ -672,11 +676,13 @@ hipError_t run_direct_part(const DevProblem &p, int which, void *work, const Com
     return launch_reduce(a, nullptr, co, 0, 0, 1, s);
 }
 
-hipError_t launch_achstemp(const DevProblem &p, cplx *part_achs, cplx *bg, Stamp stamp, hipStream_t s)
+hipError_t launch_achstemp(const DevProblem &p, cplx *part_achs, cplx *bg, Stamp stamp, hipStream_t s,
+                           const int32_t *perm)
 {
     DirectArgs a = make_args(p, nullptr);
     a.part_achs = part_achs;
     a.bg = bg;
+    a.perm = perm;
     a.stamp = stamp;
     return launch_ach(a, s);
 }

@@ -5,7 +5,7 @@
 //   1. k_achstemp      Bg[n1][j] = aqsm[n1][igp(j)] (13 MB at 512x1638) and the
 //                      achstemp band sums (reduce_achstemp, gppComplex.cpp:66-101)
 //   2. Gram product    Mu = conj(Bg)^T * aqsn over bands [nv, nb):
-//        FP64 MFMA (k_gram_f64, tile chosen by GramKind::tile), or the Ozaki
+//        FP64 MFMA (k_gram_f64 or k_gram_small, tile by gram_tile_for), or the Ozaki
 //        split of gpp_ozaki.hip; written to HBM as [ngpown][ncouls]
 //   3. k_pole_reduce   streams wtilde, I_eps, Mu (and the nv occupied aqsn rows),
 //                      evaluates the pole factors in FP64, reduces per column
@@ -99,7 +99,16 @@ bool fused_reduce(const DevProblem &p, const GramKind &k)
 // written once and read back once, by the pole reduce.  us, plain against
 // non-temporal stores: 512/2/32768/1638 (859 MB) reduce 510 -> 422, Gram alike;
 // 512/2/32768/205 (107 MB) reduce 80 -> 72, Gram 357 -> 363.
-bool mu_streams(const DevProblem &p) { return sizeof(cplx) * (size_t)p.ngpown * p.ncouls > ((size_t)32 << 20); }
+// n products of one launch count together.
+bool mu_streams(const DevProblem &p, int n) { return sizeof(cplx) * (size_t)p.ngpown * p.ncouls * n > ((size_t)32 << 20); }
+
+// The products of one Gram launch: one over bands [nv, nb), or n of them over
+// the rows in dev (gram_slot), `bands` in all.
+struct GramSlots {
+    const int32_t *dev = nullptr;
+    int n = 1;
+    long long bands = 0;
+};
 
 // G-vectors per block of k_acht_occ: the reduce's range, halved while the
 // launch has fewer than 2048 blocks (each thread waits on its own loads:
@@ -110,6 +119,9 @@ int acht_occ_chunk(const DevProblem &p, int red_chunk)
     while (chunk > 512 && (long long)p.ngpown * ((p.ncouls + chunk - 1) / chunk) < 2048) chunk /= 2;
     return chunk;
 }
+
+// The frequency of acht_n1_loc: sch_array[2], gppComplex.cpp:381.
+int acht_frequency(const DevProblem &p) { return p.nfreq > 2 ? 2 : p.nfreq - 1; }
 
 struct FactLayout {
     size_t bg, m, col_ach, col_asx, col2_ach, col2_asx, part_achs, p2, br1, acht_part, acht_occ, total;
@@ -152,17 +164,29 @@ FactLayout fact_layout(const DevProblem &p, const GramKind &k)
     return L;
 }
 
-// 1-D grid over the ceil(ngpown/TJ) x ceil(ncouls/TI) tiles, G' tiles
+// Product blockIdx.y of a launch over several (band-dependent frequencies):
+// its bands are rows [slots[3y], slots[3y+1]), its Mu is the y-th.
+__device__ __forceinline__ void gram_slot(const int32_t *slots, int ngpown, int ncouls, int &k_begin, int &k_end,
+                                          cplx *__restrict__ &mout)
+{
+    if (!slots) return;
+    k_begin = slots[3 * blockIdx.y];
+    k_end = slots[3 * blockIdx.y + 1];
+    mout += (size_t)blockIdx.y * ngpown * ncouls;
+}
+
+// Grid x over the ceil(ngpown/TJ) x ceil(ncouls/TI) tiles, G' tiles
 // fastest in tile order and tiles spread over the XCDs by xcd_tile, so the
 // blocks sharing one aqsn tile run on one XCD.  The last G' tile runs SJR <= SJ
 // sub-tiles per wave, as many as its columns need (the launcher picks SJR).
 template <class C, int SJR, bool NTS>
 __global__ __launch_bounds__(C::NT) __attribute__((amdgpu_waves_per_eu(C::OCC))) void k_gram_f64(
     const cplx *__restrict__ bg, const cplx *__restrict__ aqsn, int ngpown, int ncouls, int k_begin, int k_end,
-    cplx *__restrict__ mout, Stamp stamp)
+    const int32_t *__restrict__ slots, cplx *__restrict__ mout, Stamp stamp)
 {
     stamp_start(stamp);
     __shared__ cplx lds[C::LDS];
+    gram_slot(slots, ngpown, ncouls, k_begin, k_end, mout);
     const int nj = (ngpown + C::TJ - 1) / C::TJ, ni = (ncouls + C::TI - 1) / C::TI;
     if constexpr (SJR == C::SJ) {
         const int t = xcd_tile(blockIdx.x, nj * ni);
@@ -186,9 +210,11 @@ __global__ __launch_bounds__(C::NT) __attribute__((amdgpu_waves_per_eu(C::OCC)))
 // 16 x 16 tiles, three waves each (gram_small_product); same tile order.
 __global__ __launch_bounds__(kSmThreads) void k_gram_small(const cplx *__restrict__ bg, const cplx *__restrict__ aqsn,
                                                            int ngpown, int ncouls, int k_begin, int k_end,
+                                                           const int32_t *__restrict__ slots,
                                                            cplx *__restrict__ mout, Stamp stamp)
 {
     stamp_start(stamp);
+    gram_slot(slots, ngpown, ncouls, k_begin, k_end, mout);
     // one array (with a second one the compiler waits for every outstanding
     // load before each fragment read): the stages, then P2 and P3
     __shared__ cplx lds[kSmBuf * kSmStage];
@@ -281,13 +307,13 @@ __global__ __launch_bounds__(kRedThreads, (FC <= 3 && !P2 && !NEG) ? 4 : FC > 8 
 }
 
 __global__ __launch_bounds__(kRedThreads) void k_fact_final(const cplx *col_ach, const cplx *col_asx,
-                                                            const cplx *part_achs, int ncols, int nfreq, int nb,
-                                                            int nv, cplx *out, Stamp stamp,
+                                                            const cplx *part_achs, long long ncols, int nfreq, int nb,
+                                                            int nv, cplx *out, bool nan_acht, Stamp stamp,
                                                             unsigned long long *end)
 {
     stamp_start(stamp);
     __shared__ cplx scratch[kRedThreads / kWave];
-    final_block(col_ach, col_asx, part_achs, ncols, nfreq, nb, nv, out, scratch, blockIdx.x);
+    final_block(col_ach, col_asx, part_achs, ncols, nfreq, nb, nv, out, scratch, blockIdx.x, nan_acht);
     stamp_end(end);
 }
 
@@ -341,10 +367,12 @@ __global__ __launch_bounds__(kRedThreads) void k_acht_occ(const cplx *__restrict
 // partials of the product (bands n1 >= nv), groups combined in order.
 // Blocks after them: one per occupied band n1 < nv, its (column, split)
 // partials of k_acht_occ strided over the 256 threads, then block_sum.
+// perm: row n1 is band perm[n1] of out (null: n1).
 constexpr int kAchtFinalBands = 16;
 __global__ __launch_bounds__(256) void k_acht_final(const cplx *__restrict__ part, int nparts,
                                                     const cplx *__restrict__ part_occ, int nparts_occ, int nb,
-                                                    int nv, cplx *__restrict__ out, unsigned long long *end)
+                                                    int nv, const int32_t *__restrict__ perm,
+                                                    cplx *__restrict__ out, unsigned long long *end)
 {
     __shared__ cplx grp[256 / kAchtFinalBands][kAchtFinalBands];
     const int nblk = (nb + kAchtFinalBands - 1) / kAchtFinalBands;
@@ -362,38 +390,38 @@ __global__ __launch_bounds__(256) void k_acht_final(const cplx *__restrict__ par
         if (g == 0 && n1 >= nv && n1 < nb) {
             cplx t = grp[0][threadIdx.x];
             for (int k = 1; k < NG; ++k) t = cadd(t, grp[k][threadIdx.x]);
-            out[n1] = t;
+            out[perm ? perm[n1] : n1] = t;
         }
     } else {
         const int n1 = (int)blockIdx.x - nblk;  // < nv
         cplx s = czero();
         for (int q = threadIdx.x; q < nparts_occ; q += blockDim.x) s = cadd(s, part_occ[(size_t)q * nv + n1]);
         s = block_sum(s, &grp[0][0]);
-        if (threadIdx.x == 0) out[n1] = s;
+        if (threadIdx.x == 0) out[perm ? perm[n1] : n1] = s;
     }
     stamp_end(end);
 }
 
 template <class C, bool NTS>
-void launch_gram_nts(const DevProblem &p, const cplx *bg, cplx *mu, Stamp stamp, hipStream_t s)
+void launch_gram_nts(const DevProblem &p, const GramSlots &g, const cplx *bg, cplx *mu, Stamp stamp, hipStream_t s)
 {
     const unsigned tiles = (unsigned)((p.ngpown + C::TJ - 1) / C::TJ) * (unsigned)((p.ncouls + C::TI - 1) / C::TI);
     const int rem = p.ngpown % C::TJ;
     if (C::SJ == 2 && rem > 0 && rem <= 16 * C::WJN)
-        hipLaunchKernelGGL((k_gram_f64<C, 1, NTS>), dim3(tiles), dim3(C::NT), 0, s, bg, p.aqsn, p.ngpown, p.ncouls,
-                           p.nv, p.nb, mu, stamp);
+        hipLaunchKernelGGL((k_gram_f64<C, 1, NTS>), dim3(tiles, g.n), dim3(C::NT), 0, s, bg, p.aqsn, p.ngpown,
+                           p.ncouls, p.nv, p.nb, g.dev, mu, stamp);
     else
-        hipLaunchKernelGGL((k_gram_f64<C, C::SJ, NTS>), dim3(tiles), dim3(C::NT), 0, s, bg, p.aqsn, p.ngpown,
-                           p.ncouls, p.nv, p.nb, mu, stamp);
+        hipLaunchKernelGGL((k_gram_f64<C, C::SJ, NTS>), dim3(tiles, g.n), dim3(C::NT), 0, s, bg, p.aqsn, p.ngpown,
+                           p.ncouls, p.nv, p.nb, g.dev, mu, stamp);
 }
 
 template <class C>
-void launch_gram_ring(const DevProblem &p, const cplx *bg, cplx *mu, Stamp stamp, hipStream_t s)
+void launch_gram_ring(const DevProblem &p, const GramSlots &g, const cplx *bg, cplx *mu, Stamp stamp, hipStream_t s)
 {
-    if (mu_streams(p))
-        launch_gram_nts<C, true>(p, bg, mu, stamp, s);
+    if (mu_streams(p, g.n))
+        launch_gram_nts<C, true>(p, g, bg, mu, stamp, s);
     else
-        launch_gram_nts<C, false>(p, bg, mu, stamp, s);
+        launch_gram_nts<C, false>(p, g, bg, mu, stamp, s);
 }
 
 template <class C, bool CUT>
@@ -469,8 +497,10 @@ size_t factored_workspace_bytes(const DevProblem &p, GramKind kind)
 // 358 / 354; 512/2/800/40 16 x 16 9.6 / 9.7, 32 x 64 35 / 38).  Larger tiles
 // re-read less and turn stages over less often; smaller ones leave fewer CUs
 // idle, and the 16 x 16 tile has the shortest chain of MFMAs per wave.
+// Several products in one launch count with their mean number of bands.
+namespace {
 enum GramTile { kTileL = 0, kTileLt, kTileM, kTileS, kTileX };
-int gram_tile_for(const DevProblem &p)
+int gram_tile_for(const DevProblem &p, const GramSlots &g)
 {
     struct Kind {
         int tile, tj, ti, short_j;  // short_j: rows of a short last tile (0: none)
@@ -481,15 +511,15 @@ int gram_tile_for(const DevProblem &p)
                                  {kTileM, GramM::TJ, GramM::TI, GramM::TJ / 2, 0.0287, 0.0247},
                                  {kTileS, GramS::TJ, GramS::TI, 0, 0.0344, 0.0273},
                                  {kTileX, 16, 16, 0, 0.0547, 0.0469}};
-    const double ksteps = (p.nb - p.nv + 3) / 4;
+    const double ksteps = g.dev ? std::max(1.0, (double)g.bands / (4 * g.n)) : (p.nb - p.nv + 3) / 4;
     double best = 1e300;
     int tile = kTileL;
     for (const Kind &k : kinds) {
         const int rem = p.ngpown % k.tj;
         const bool cut = rem > 0 && rem <= k.short_j;
         const double ni = (p.ncouls + k.ti - 1) / k.ti, sub = k.tj / 16 * (k.ti / 16);
-        const double whole = ni * ((p.ngpown + k.tj - 1) / k.tj - (cut ? 1 : 0));
-        const double rounds = tile_rounds(whole, cut ? ni : 0);
+        const double whole = g.n * ni * ((p.ngpown + k.tj - 1) / k.tj - (cut ? 1 : 0));
+        const double rounds = tile_rounds(whole, cut ? g.n * ni : 0);
         double us = rounds * sub * ksteps * (rounds <= 1 ? k.one : k.many);
         if (k.tile == kTileX) us += 1.2 * ceil(rounds / 2);  // the first loads of its ring, two blocks at a time
         if (us < best) best = us, tile = k.tile;
@@ -497,20 +527,21 @@ int gram_tile_for(const DevProblem &p)
     return tile;
 }
 
-hipError_t launch_gram_f64(const DevProblem &p, int tile, const cplx *bg, cplx *mu, Stamp stamp, hipStream_t s)
+hipError_t launch_gram_f64(const DevProblem &p, const GramSlots &g, int tile, const cplx *bg, cplx *mu, Stamp stamp,
+                           hipStream_t s)
 {
     // GPP_OPT_GRAM_TILE: 0 by size, then the ring tiles
     static const int kinds[kGramTiles] = {-1, kTileL, kTileLt, kTileM};
     if (tile < 0 || tile >= kGramTiles) return hipErrorInvalidValue;
-    switch (tile == 0 ? gram_tile_for(p) : kinds[tile]) {
-    case kTileL: launch_gram_ring<GramL>(p, bg, mu, stamp, s); break;
-    case kTileLt: launch_gram_ring<GramLt>(p, bg, mu, stamp, s); break;
-    case kTileM: launch_gram_ring<GramM>(p, bg, mu, stamp, s); break;
-    case kTileS: launch_gram_ring<GramS>(p, bg, mu, stamp, s); break;
+    switch (tile == 0 ? gram_tile_for(p, g) : kinds[tile]) {
+    case kTileL: launch_gram_ring<GramL>(p, g, bg, mu, stamp, s); break;
+    case kTileLt: launch_gram_ring<GramLt>(p, g, bg, mu, stamp, s); break;
+    case kTileM: launch_gram_ring<GramM>(p, g, bg, mu, stamp, s); break;
+    case kTileS: launch_gram_ring<GramS>(p, g, bg, mu, stamp, s); break;
     default: {
         const unsigned tiles = (unsigned)((p.ngpown + 15) / 16) * (unsigned)((p.ncouls + 15) / 16);
-        hipLaunchKernelGGL(k_gram_small, dim3(tiles), dim3(kSmThreads), 0, s, bg, p.aqsn, p.ngpown, p.ncouls, p.nv,
-                           p.nb, mu, stamp);
+        hipLaunchKernelGGL(k_gram_small, dim3(tiles, g.n), dim3(kSmThreads), 0, s, bg, p.aqsn, p.ngpown, p.ncouls,
+                           p.nv, p.nb, g.dev, mu, stamp);
         break;
     }
     }
@@ -535,8 +566,84 @@ hipError_t launch_pole_reduce(const ReduceArgs &ra, int red_fc, hipStream_t s)
     return hipGetLastError();
 }
 
+// Where stage 3 puts what acht_n1_loc needs, and the later stages' partials.
+struct AchtBufs {
+    cplx *p2 = nullptr;  // null: acht_n1_loc is not requested
+    uint8_t *br1 = nullptr;
+    cplx *part = nullptr, *part_occ = nullptr;
+};
+
+// Stage 3 of one problem; its partials to col_ach/col_asx [ngpown][nsplit][nfreq].
+hipError_t run_pole_reduce(const DevProblem &p, const GramKind &kind, const cplx *mu, const cplx *bg, cplx *col_ach,
+                           cplx *col_asx, int nsplit, const AchtBufs &ab, Stamp stamp, hipStream_t s)
+{
+    ReduceArgs ra;
+    ra.mu = mu; ra.ieps = p.ieps; ra.wtilde = p.wtilde; ra.aqsn = p.aqsn; ra.bg = bg; ra.idx = p.idx;
+    ra.vcoul = p.vcoul; ra.wx = p.wx; ra.nv = p.nv; ra.ncouls = p.ncouls; ra.ngpown = p.ngpown;
+    ra.nfreq = p.nfreq; ra.occ = p.occ; ra.col_ach = col_ach; ra.col_asx = col_asx;
+    ra.nsplit = nsplit; ra.chunk = kind.red_chunk;
+    ra.fpb = kind.red_fpb > 0 ? kind.red_fpb : p.nfreq;
+    ra.p2 = ab.p2;
+    const bool occ_in_reduce = ab.p2 && p.nv > 0 && reduce_sums_acht_occ(p.nv, p.wx_neg);
+    ra.br1 = ab.p2 && p.nv > 0 && !occ_in_reduce ? ab.br1 : nullptr;
+    ra.part_occ = occ_in_reduce ? ab.part_occ : nullptr;
+    ra.acht_iw = acht_frequency(p);
+    ra.neg = p.wx_neg;
+    ra.stamp = stamp;
+    return launch_pole_reduce(ra, kind.red_fc, s);
+}
+
+// Stages 2 and 3 fused; column sums to col_ach/col_asx [ngpown][nfreq].
+// tile_ach/tile_asx: [ngpown][nsplit][nfreq].
+hipError_t run_gram_pole(const DevProblem &p, const cplx *bg, cplx *tile_ach, cplx *tile_asx, int nsplit,
+                         cplx *col_ach, cplx *col_asx, Stamp stamp, StageTimer *timer, hipStream_t s)
+{
+    PoleTileArgs pa;
+    pa.aqsn = p.aqsn; pa.ieps = p.ieps; pa.wtilde = p.wtilde; pa.bg = bg; pa.wx = p.wx;
+    pa.nb = p.nb; pa.nv = p.nv; pa.ncouls = p.ncouls; pa.ngpown = p.ngpown; pa.nsplit = nsplit;
+    pa.col_ach = tile_ach; pa.col_asx = tile_asx;
+    pa.stamp = stamp;
+    switch (p.nfreq) {
+    case 1: launch_gram_pole_f<1>(p, pa, s); break;
+    case 2: launch_gram_pole_f<2>(p, pa, s); break;
+    default: launch_gram_pole_f<3>(p, pa, s); break;
+    }
+    GPP_TRY(hipGetLastError());
+    hipLaunchKernelGGL(k_pole_cols, dim3((p.ngpown + 3) / 4), dim3(256), 0, s, tile_ach, tile_asx, nsplit, p.nfreq,
+                       p.idx, p.vcoul, p.ncouls, p.ngpown, p.occ, col_ach, col_asx,
+                       timer ? timer->stage("factored_pole_cols") : Stamp{});
+    return hipGetLastError();
+}
+
+// Stages 5 and 6: acht_n1_loc of the problem's bands, row n1 to
+// out[perm ? perm[n1] : n1].  st: for the first launch.
+hipError_t run_acht(const DevProblem &p, const AchtSplit &as, int occ_chunk, int occ_nsplit, const AchtBufs &ab,
+                    const cplx *bg, const int32_t *perm, cplx *out, Stamp st, unsigned long long *end, hipStream_t s)
+{
+    if (p.nb > p.nv) {
+        if (as.narrow)
+            as.cut ? launch_acht<GramM, true>(p, as, ab.p2, bg, ab.part, st, s)
+                   : launch_acht<GramM, false>(p, as, ab.p2, bg, ab.part, st, s);
+        else
+            as.cut ? launch_acht<GramL, true>(p, as, ab.p2, bg, ab.part, st, s)
+                   : launch_acht<GramL, false>(p, as, ab.p2, bg, ab.part, st, s);
+        GPP_TRY(hipGetLastError());
+        st = Stamp{};
+    }
+    if (p.nv > 0 && !reduce_sums_acht_occ(p.nv, p.wx_neg)) {  // else summed by the reduce
+        hipLaunchKernelGGL(k_acht_occ, dim3(p.ngpown, occ_nsplit), dim3(kRedThreads), 0, s, ab.p2, ab.br1, p.aqsn,
+                           bg, p.idx, p.vcoul, p.ngpown, p.ncouls, p.nv, occ_chunk, occ_nsplit, ab.part_occ, st);
+        GPP_TRY(hipGetLastError());
+    }
+    hipLaunchKernelGGL(k_acht_final, dim3((p.nb + kAchtFinalBands - 1) / kAchtFinalBands + p.nv), dim3(256), 0, s,
+                       ab.part, as.jtiles * as.nks, ab.part_occ, p.ngpown * occ_nsplit, p.nb, p.nv, perm, out, end);
+    return hipGetLastError();
+}
+
+}  // namespace
+
 hipError_t run_factored(const DevProblem &p, GramKind kind, void *work, const DevResults &res, hipStream_t s,
-                        StageTimer *timer, Stamp first)
+                        StageTimer *timer)
 {
     if (p.wx_stride != 0) return hipErrorInvalidValue;  // the band sum factors only for a shared wx row
     const FactLayout L = fact_layout(p, kind);
@@ -551,96 +658,58 @@ hipError_t run_factored(const DevProblem &p, GramKind kind, void *work, const De
     const auto end = [&]() { return timer ? timer->end() : nullptr; };
     if (timer) timer->begin();
     // also gathers Bg
-    GPP_TRY(launch_achstemp(p, part_achs, bg, timer ? stage("factored_gather_achstemp") : first, s));
+    GPP_TRY(launch_achstemp(p, part_achs, bg, stage("factored_gather_achstemp"), s));
     if (L.fused) {
-        PoleTileArgs pa;
-        pa.aqsn = p.aqsn; pa.ieps = p.ieps; pa.wtilde = p.wtilde; pa.bg = bg; pa.wx = p.wx;
-        pa.nb = p.nb; pa.nv = p.nv; pa.ncouls = p.ncouls; pa.ngpown = p.ngpown; pa.nsplit = L.nsplit;
-        pa.col_ach = col_ach; pa.col_asx = col_asx;
-        pa.stamp = stage("factored_gram_pole");
-        switch (p.nfreq) {
-        case 1: launch_gram_pole_f<1>(p, pa, s); break;
-        case 2: launch_gram_pole_f<2>(p, pa, s); break;
-        default: launch_gram_pole_f<3>(p, pa, s); break;
-        }
-        GPP_TRY(hipGetLastError());
         cplx *c2a = reinterpret_cast<cplx *>(w + L.col2_ach);
         cplx *c2x = reinterpret_cast<cplx *>(w + L.col2_asx);
-        hipLaunchKernelGGL(k_pole_cols, dim3((p.ngpown + 3) / 4), dim3(256), 0, s, col_ach, col_asx, L.nsplit,
-                           p.nfreq, p.idx, p.vcoul, p.ncouls, p.ngpown, p.occ, c2a, c2x, stage("factored_pole_cols"));
-        GPP_TRY(hipGetLastError());
+        GPP_TRY(run_gram_pole(p, bg, col_ach, col_asx, L.nsplit, c2a, c2x, stage("factored_gram_pole"), timer, s));
         const Stamp st = stage("factored_final");
         hipLaunchKernelGGL(k_fact_final, dim3(p.nfreq + 1), dim3(kRedThreads), 0, s, c2a, c2x, part_achs, p.ngpown,
-                           p.nfreq, p.nb, p.nv, res.base, st, end());
+                           p.nfreq, p.nb, p.nv, res.base, true, st, end());
         return hipGetLastError();
     }
     if (kind.ozaki_slices) {
         GPP_TRY(launch_gram_ozaki(p, kind.ozaki_slices, kind.int8, kind.layout, kind.group, bg, w + L.total, mu,
                                   stage(kind.int8 ? "factored_gram_ozaki_i8" : "factored_gram_ozaki"), s));
     } else {
-        GPP_TRY(launch_gram_f64(p, kind.tile, bg, mu, stage("factored_gram_f64"), s));
+        GPP_TRY(launch_gram_f64(p, GramSlots{}, kind.tile, bg, mu, stage("factored_gram_f64"), s));
     }
-    ReduceArgs ra;
-    ra.mu = mu; ra.ieps = p.ieps; ra.wtilde = p.wtilde; ra.aqsn = p.aqsn; ra.bg = bg; ra.idx = p.idx;
-    ra.vcoul = p.vcoul; ra.wx = p.wx; ra.nv = p.nv; ra.ncouls = p.ncouls; ra.ngpown = p.ngpown;
-    ra.nfreq = p.nfreq; ra.occ = p.occ; ra.col_ach = col_ach; ra.col_asx = col_asx;
-    ra.nsplit = L.nsplit; ra.chunk = kind.red_chunk;
-    ra.fpb = kind.red_fpb > 0 ? kind.red_fpb : p.nfreq;
-    ra.p2 = kind.acht ? reinterpret_cast<cplx *>(w + L.p2) : nullptr;
-    const bool occ_in_reduce = kind.acht && p.nv > 0 && reduce_sums_acht_occ(p.nv, p.wx_neg);
-    ra.br1 = kind.acht && p.nv > 0 && !occ_in_reduce ? reinterpret_cast<uint8_t *>(w + L.br1) : nullptr;
-    ra.part_occ = occ_in_reduce ? reinterpret_cast<cplx *>(w + L.acht_occ) : nullptr;
-    ra.acht_iw = p.nfreq > 2 ? 2 : p.nfreq - 1;  // sch_array[2], gppComplex.cpp:381
-    ra.neg = p.wx_neg;
-    ra.stamp = stage("factored_pole_reduce");
-    GPP_TRY(launch_pole_reduce(ra, kind.red_fc, s));
+    AchtBufs ab;
+    if (kind.acht) {
+        ab.p2 = reinterpret_cast<cplx *>(w + L.p2);
+        ab.br1 = reinterpret_cast<uint8_t *>(w + L.br1);
+        ab.part = reinterpret_cast<cplx *>(w + L.acht_part);
+        ab.part_occ = reinterpret_cast<cplx *>(w + L.acht_occ);
+    }
+    GPP_TRY(run_pole_reduce(p, kind, mu, bg, col_ach, col_asx, L.nsplit, ab, stage("factored_pole_reduce"), s));
     const Stamp st_final = stage("factored_final");
     hipLaunchKernelGGL(k_fact_final, dim3(p.nfreq + 1), dim3(kRedThreads), 0, s, col_ach, col_asx, part_achs,
-                       p.ngpown * L.nsplit, p.nfreq, p.nb, p.nv, res.base, st_final, kind.acht ? nullptr : end());
+                       p.ngpown * L.nsplit, p.nfreq, p.nb, p.nv, res.base, true, st_final,
+                       kind.acht ? nullptr : end());
     GPP_TRY(hipGetLastError());
-    if (kind.acht) {
-        Stamp st = stage("factored_acht");  // for the first launch of the stage
-        const AchtSplit &as = L.as;
-        cplx *part = reinterpret_cast<cplx *>(w + L.acht_part);
-        cplx *part_occ = reinterpret_cast<cplx *>(w + L.acht_occ);
-        if (p.nb > p.nv) {
-            if (as.narrow)
-                as.cut ? launch_acht<GramM, true>(p, as, ra.p2, bg, part, st, s)
-                       : launch_acht<GramM, false>(p, as, ra.p2, bg, part, st, s);
-            else
-                as.cut ? launch_acht<GramL, true>(p, as, ra.p2, bg, part, st, s)
-                       : launch_acht<GramL, false>(p, as, ra.p2, bg, part, st, s);
-            GPP_TRY(hipGetLastError());
-            st = Stamp{};
-        }
-        if (p.nv > 0 && !occ_in_reduce) {  // else summed by the reduce
-            hipLaunchKernelGGL(k_acht_occ, dim3(p.ngpown, L.occ_nsplit), dim3(kRedThreads), 0, s, ra.p2, ra.br1,
-                               p.aqsn, bg, p.idx, p.vcoul, p.ngpown, p.ncouls, p.nv, L.occ_chunk, L.occ_nsplit,
-                               part_occ, st);
-            GPP_TRY(hipGetLastError());
-        }
-        hipLaunchKernelGGL(k_acht_final, dim3((p.nb + kAchtFinalBands - 1) / kAchtFinalBands + p.nv), dim3(256), 0,
-                           s, part, as.jtiles * as.nks, part_occ,
-                           p.ngpown * L.occ_nsplit, p.nb, p.nv, res.acht_n1_loc(), end());
-        GPP_TRY(hipGetLastError());
-    }
-    return hipSuccess;
+    if (!kind.acht) return hipSuccess;
+    const Stamp st = stage("factored_acht");
+    return run_acht(p, L.as, L.occ_chunk, L.occ_nsplit, ab, bg, nullptr, res.acht_n1_loc(), st, end(), s);
 }
 
 // ---------------------------------------------------------------------------
 // Band-dependent frequencies.  The band sum factors over any set of bands
-// that share one wx row, so bands are grouped by identical rows ("buckets")
-// and each bucket is one factored sub-problem: its bands are gathered into a
-// contiguous block (occupied bands first), the sub-problem runs through
-// run_factored with that bucket's row, and the per-bucket results are summed
-// in bucket order (acht_n1_loc scattered back to the original band order).
+// that share one wx row, so bands are grouped by identical rows ("buckets"),
+// each a factored sub-problem of its own Mu and row.  Bg and aqsn are laid out
+// with each bucket's bands contiguous, occupied ones first (as they are where
+// the bands already lie so).  One launch forms every bucket's Mu, one more
+// pass adds up the pole terms of all buckets without occupied bands
+// (pole_reduce_bare); a bucket with occupied bands runs the reduce of the
+// plain form.  The Mu of at most kBucketMuBytes of buckets are held at a time.
+// 512/8/8192/409/3 in 8 buckets: 704 us with a factored evaluation per
+// bucket and both arrays permuted, 368 so (Gram 215 of them, with 429 MB of Mu
+// to store; the reduces 56 and 84, the latter at 5.7 TB/s).
 
 namespace {
 
 __global__ void k_permute_rows(const cplx *__restrict__ src, const int32_t *__restrict__ perm, int nrows,
-                               int ncols, cplx *__restrict__ dst, Stamp stamp)
+                               int ncols, cplx *__restrict__ dst)
 {
-    stamp_start(stamp);
     const size_t n = (size_t)nrows * ncols;
     for (size_t t = (size_t)blockIdx.x * blockDim.x + threadIdx.x; t < n; t += (size_t)gridDim.x * blockDim.x) {
         const size_t r = t / ncols, c = t % ncols;
@@ -648,63 +717,140 @@ __global__ void k_permute_rows(const cplx *__restrict__ src, const int32_t *__re
     }
 }
 
-// One block.  tab[3b..3b+2] = (result offset, first permuted row, bands) of
-// bucket b; bres holds each bucket's DevResults back to back.
-__global__ void k_bucket_combine(const cplx *__restrict__ bres, const int32_t *__restrict__ tab,
-                                 const int32_t *__restrict__ perm, int nbuckets, int nfreq, int nb,
-                                 cplx *__restrict__ out, Stamp stamp, unsigned long long *end)
+template <int F> __global__ __launch_bounds__(kRedThreads, 4) void k_reduce_bare(BareArgs a)
 {
-    stamp_start(stamp);
-    for (int iw = threadIdx.x; iw < 2 * nfreq; iw += blockDim.x) {
-        cplx s = czero();
-        for (int b = 0; b < nbuckets; ++b) s = cadd(s, bres[tab[3 * b] + iw]);
-        out[iw] = s;  // achtemp[iw] for iw < nfreq, then asxtemp
-    }
-    if (threadIdx.x == 0) {
-        cplx s = czero();
-        for (int b = 0; b < nbuckets; ++b) s = cadd(s, bres[tab[3 * b] + 2 * nfreq + tab[3 * b + 2]]);
-        out[2 * nfreq + nb] = s;  // achstemp
-    }
-    for (int b = 0; b < nbuckets; ++b)
-        for (int k = threadIdx.x; k < tab[3 * b + 2]; k += blockDim.x)
-            out[2 * nfreq + perm[tab[3 * b + 1] + k]] = bres[tab[3 * b] + 2 * nfreq + k];
-    stamp_end(end);
+    __shared__ cplx scratch[kRedThreads / kWave];
+    pole_reduce_bare<F>(a, scratch);
 }
 
+// P = delw I_eps of one frequency (the p2 of the reduce), for the buckets
+// whose reduce does not write it.
+__global__ __launch_bounds__(256) void k_pole_p2(const cplx *__restrict__ wtilde, const cplx *__restrict__ ieps,
+                                                 const double *__restrict__ wx, size_t n, cplx *__restrict__ p2)
+{
+    const double w = *wx;
+    for (size_t t = (size_t)blockIdx.x * blockDim.x + threadIdx.x; t < n; t += (size_t)gridDim.x * blockDim.x) {
+        const cplx wt = wtilde[t], q = cmul_fast(wt, ieps[t]);
+        const double wdr = w - wt.re, rden = rcp_1nr(__builtin_fma(wdr, wdr, wt.im * wt.im));
+        __builtin_nontemporal_store(__builtin_fma(q.re, wdr, -(q.im * wt.im)) * rden, &p2[t].re);
+        __builtin_nontemporal_store(__builtin_fma(q.im, wdr, q.re * wt.im) * rden, &p2[t].im);
+    }
+}
+
+// Frequencies per block of k_reduce_bare: equal passes of at most 8.
+int bare_width(int nfreq)
+{
+    const int passes = (nfreq + 7) / 8, f = (nfreq + passes - 1) / passes;
+    return f <= 4 ? f : f <= 6 ? 6 : 8;
+}
+
+void launch_reduce_bare(const BareArgs &a, hipStream_t s)
+{
+    const int f = bare_width(a.nfreq);
+    const dim3 grid(a.ngpown, a.nsplit, (a.nfreq + f - 1) / f);
+    switch (f) {
+    case 1: hipLaunchKernelGGL(k_reduce_bare<1>, grid, dim3(kRedThreads), 0, s, a); break;
+    case 2: hipLaunchKernelGGL(k_reduce_bare<2>, grid, dim3(kRedThreads), 0, s, a); break;
+    case 3: hipLaunchKernelGGL(k_reduce_bare<3>, grid, dim3(kRedThreads), 0, s, a); break;
+    case 4: hipLaunchKernelGGL(k_reduce_bare<4>, grid, dim3(kRedThreads), 0, s, a); break;
+    case 6: hipLaunchKernelGGL(k_reduce_bare<6>, grid, dim3(kRedThreads), 0, s, a); break;
+    default: hipLaunchKernelGGL(k_reduce_bare<8>, grid, dim3(kRedThreads), 0, s, a); break;
+    }
+}
+
+constexpr size_t kBucketMuBytes = (size_t)4 << 30;
+
+// How a slot's stage 3 runs: fused with its Gram product, with the plain
+// form's reduce, or together with the other buckets without occupied bands.
+// With GPP_OPT_FUSED_REDUCE no bucket runs together with others.
+enum SlotKind { kSlotFused, kSlotPlain, kSlotBare };
+
 struct BucketLayout {
-    size_t aqsm, aqsn, perm, tab, bres, sub, total;
+    size_t aqsn, bg, mu, part_achs, col_ach, col_asx, tile_ach, tile_asx, p2, br1, acht_part, acht_occ, sub, total;
+    int group;   // buckets whose Mu are held at a time
+    int nsplit;  // G-vector ranges of a plain reduce
+    int bare_chunk, bare_nsplit;
+    long long ncols;  // column partials of all buckets
 };
 
-DevProblem bucket_problem(const DevProblem &p, const BucketPlan &bp, int b, const cplx *aqsm_p, const cplx *aqsn_p)
+// Bucket b over its rows of the permuted aqsn.
+DevProblem bucket_problem(const DevProblem &p, const BucketPlan &bp, int b, const cplx *aqsn_p)
 {
     DevProblem q = p;
     q.nb = bp.size[b];
     q.nv = bp.nocc[b];
-    q.aqsm = aqsm_p + (size_t)bp.start[b] * p.ncouls;
+    q.aqsm = nullptr;  // Bg is gathered for all buckets
     q.aqsn = aqsn_p + (size_t)bp.start[b] * p.ncouls;
     q.wx = p.wx + (size_t)bp.row[b] * p.nfreq;
     q.wx_stride = 0;
-    q.wx_neg = bp.neg.empty() ? 1 : bp.neg[b];
+    q.wx_neg = bp.neg[b];
     return q;
+}
+
+SlotKind slot_kind(const DevProblem &q, const GramKind &k)
+{
+    if (fused_reduce(q, k)) return kSlotFused;
+    return q.nv > 0 || k.fuse ? kSlotPlain : kSlotBare;
 }
 
 BucketLayout bucket_layout(const DevProblem &p, const GramKind &k, const BucketPlan &bp)
 {
     BucketLayout L;
-    const int nbk = (int)bp.size.size();
-    size_t off = 0;
-    L.aqsm = off; off += align256(sizeof(cplx) * (size_t)p.nb * p.ncouls);
-    L.aqsn = off; off += align256(sizeof(cplx) * (size_t)p.nb * p.ncouls);
-    L.perm = off; off += align256(sizeof(int32_t) * (size_t)p.nb);
-    L.tab = off;  off += align256(sizeof(int32_t) * 3 * (size_t)nbk);
-    size_t sub = 0;
-    for (int b = 0; b < nbk; ++b) {
-        const DevProblem q = bucket_problem(p, bp, b, nullptr, nullptr);
-        sub = std::max(sub, factored_workspace_bytes(q, k));
+    const int nbk = (int)bp.slot.size();
+    const size_t mu_bytes = sizeof(cplx) * (size_t)p.ngpown * p.ncouls;
+    L.group = (int)std::max<size_t>(1, std::min<size_t>(std::min(nbk, 4096), kBucketMuBytes / mu_bytes));
+    L.nsplit = (p.ncouls + k.red_chunk - 1) / k.red_chunk;
+    // G ranges of the reduce over the bare buckets: whole steps of a block,
+    // about 2048 blocks
+    const int steps = (p.ncouls + kBareStep - 1) / kBareStep;
+    const int want = std::max(1, std::min(steps, 2048 / p.ngpown));
+    L.bare_chunk = (steps + want - 1) / want * kBareStep;
+    L.bare_nsplit = (p.ncouls + L.bare_chunk - 1) / L.bare_chunk;
+    bool mu = false, fused = false;
+    L.ncols = 0;
+    size_t br1 = 0, part = 0, occ = 0, sub = 0;
+    for (int s0 = 0; s0 < nbk; s0 += L.group) {
+        bool bare = false;
+        for (int sl = s0; sl < std::min(nbk, s0 + L.group); ++sl) {
+            const DevProblem q = bucket_problem(p, bp, bp.slot[sl], nullptr);
+            const SlotKind kind = slot_kind(q, k);
+            (kind == kSlotFused ? fused : mu) = true;
+            if (kind == kSlotBare) bare = true;
+            else L.ncols += (long long)p.ngpown * (kind == kSlotFused ? 1 : L.nsplit);
+            if (k.ozaki_slices) sub = std::max(sub, ozaki_workspace_bytes(q, k.ozaki_slices, k.int8));
+            if (!k.acht) continue;
+            const AchtSplit as = acht_split(q);
+            part = std::max(part, sizeof(cplx) * (size_t)as.jtiles * as.nks * q.nb);
+            if (q.nv == 0) continue;
+            const bool in_reduce = reduce_sums_acht_occ(q.nv, q.wx_neg);
+            const int chunk = acht_occ_chunk(q, k.red_chunk);
+            const int nsplit = in_reduce ? L.nsplit : (p.ncouls + chunk - 1) / chunk;
+            if (!in_reduce) br1 = (size_t)p.ngpown * p.ncouls;
+            occ = std::max(occ, sizeof(cplx) * (size_t)p.ngpown * nsplit * q.nv);
+        }
+        if (bare) L.ncols += (long long)p.ngpown * L.bare_nsplit;
     }
-    L.bres = off; off += align256(sizeof(cplx) * bp.nres);
-    L.sub = off;  off += sub;
-    L.total = off;
+    size_t off = 0;
+    const auto take = [&off](size_t bytes) {
+        const size_t at = off;
+        off += align256(bytes);
+        return at;
+    };
+    const size_t tiles = fused ? sizeof(cplx) * (size_t)p.ngpown * ((p.ncouls + FuseCfg::TI - 1) / FuseCfg::TI) * p.nfreq : 0;
+    L.aqsn = take(bp.identity ? 0 : sizeof(cplx) * (size_t)p.nb * p.ncouls);
+    L.bg = take(sizeof(cplx) * (size_t)p.nb * p.ngpown);
+    L.mu = take(mu ? mu_bytes * L.group : 0);
+    L.part_achs = take(sizeof(cplx) * ach_region_entries(p.nb, p.ngpown));
+    L.col_ach = take(sizeof(cplx) * (size_t)L.ncols * p.nfreq);
+    L.col_asx = take(sizeof(cplx) * (size_t)L.ncols * p.nfreq);
+    L.tile_ach = take(tiles);
+    L.tile_asx = take(tiles);
+    L.p2 = take(k.acht ? mu_bytes : 0);
+    L.br1 = take(br1);
+    L.acht_part = take(part);
+    L.acht_occ = take(occ);
+    L.sub = off;
+    L.total = off + sub;
     return L;
 }
 
@@ -731,8 +877,6 @@ BucketPlan plan_buckets(const double *wx_rows, int nb, int nv, int nfreq)
     bp.start.assign(nbk, 0);
     bp.size.assign(nbk, 0);
     bp.nocc.assign(nbk, 0);
-    bp.tab.assign(3 * (size_t)nbk, 0);
-    bp.nres = 0;
     for (int b = 0; b < nbk; ++b) {
         bp.start[b] = (int)bp.perm.size();
         for (int pass = 0; pass < 2; ++pass)  // occupied bands first, each in band order
@@ -742,12 +886,26 @@ BucketPlan plan_buckets(const double *wx_rows, int nb, int nv, int nfreq)
                     ++bp.size[b];
                     if (pass == 0) ++bp.nocc[b];
                 }
-        bp.tab[3 * b] = (int32_t)bp.nres;
-        bp.tab[3 * b + 1] = bp.start[b];
-        bp.tab[3 * b + 2] = bp.size[b];
-        bp.nres += (size_t)2 * nfreq + bp.size[b] + 1;
+        bp.slot.push_back(b);
     }
+    std::stable_sort(bp.slot.begin(), bp.slot.end(), [&](int x, int y) {
+        if ((bp.nocc[x] > 0) != (bp.nocc[y] > 0)) return bp.nocc[x] > 0;
+        return bp.size[x] - bp.nocc[x] > bp.size[y] - bp.nocc[y];
+    });
+    bp.identity = true;
+    for (int n1 = 0; n1 < nb; ++n1) bp.identity = bp.identity && bp.perm[n1] == n1;
     return bp;
+}
+
+std::vector<int32_t> BucketPlan::tables() const
+{
+    std::vector<int32_t> t = perm;
+    for (int b : slot) {
+        t.push_back(start[b] + nocc[b]);
+        t.push_back(start[b] + size[b]);
+        t.push_back(row[b]);
+    }
+    return t;
 }
 
 size_t bucketed_workspace_bytes(const DevProblem &p, GramKind kind, const BucketPlan &bp)
@@ -758,42 +916,105 @@ size_t bucketed_workspace_bytes(const DevProblem &p, GramKind kind, const Bucket
 hipError_t run_factored_bucketed(const DevProblem &p, GramKind kind, const BucketPlan &bp, void *work,
                                  const DevResults &res, hipStream_t s, StageTimer *timer)
 {
-    if (p.wx_stride != p.nfreq || (int)bp.perm.size() != p.nb || bp.tab.size() != 3 * bp.size.size())
-        return hipErrorInvalidValue;
+    if (p.wx_stride != p.nfreq || (int)bp.perm.size() != p.nb || !bp.dev) return hipErrorInvalidValue;
     const BucketLayout L = bucket_layout(p, kind, bp);
     char *w = static_cast<char *>(work);
-    cplx *aqsm_p = reinterpret_cast<cplx *>(w + L.aqsm);
-    cplx *aqsn_p = reinterpret_cast<cplx *>(w + L.aqsn);
-    int32_t *perm = reinterpret_cast<int32_t *>(w + L.perm);
-    int32_t *tab = reinterpret_cast<int32_t *>(w + L.tab);
-    cplx *bres = reinterpret_cast<cplx *>(w + L.bres);
-    const int nbk = (int)bp.size.size();
-
+    const auto at = [w](size_t off) { return reinterpret_cast<cplx *>(w + off); };
+    cplx *const bg = at(L.bg), *const mu = at(L.mu), *const part_achs = at(L.part_achs);
+    AchtBufs ab;
+    if (kind.acht) {
+        ab.p2 = at(L.p2);
+        ab.br1 = reinterpret_cast<uint8_t *>(w + L.br1);
+        ab.part = at(L.acht_part);
+        ab.part_occ = at(L.acht_occ);
+    }
+    const int nbk = (int)bp.slot.size();
+    const int32_t *const perm = bp.identity ? nullptr : bp.dev_perm();
     const auto stage = [&](const char *nm) { return timer ? timer->stage(nm) : Stamp{}; };
     if (timer) timer->begin();
-    GPP_TRY(hipMemcpyAsync(perm, bp.perm.data(), sizeof(int32_t) * p.nb, hipMemcpyHostToDevice, s));
-    GPP_TRY(hipMemcpyAsync(tab, bp.tab.data(), sizeof(int32_t) * 3 * nbk, hipMemcpyHostToDevice, s));
-    {
-        const size_t n = (size_t)p.nb * p.ncouls;
-        size_t blocks = (n + 255) / 256;
-        if (blocks > 8192) blocks = 8192;
-        hipLaunchKernelGGL(k_permute_rows, dim3((unsigned)blocks), dim3(256), 0, s, p.aqsm, perm, p.nb, p.ncouls,
-                           aqsm_p, stage("bucket_permute"));
+    GPP_TRY(launch_achstemp(p, part_achs, bg, stage("bucket_permute"), s, perm));  // also gathers Bg
+    const cplx *aqsn_p = p.aqsn;
+    if (!bp.identity) {
+        const size_t blocks = std::min<size_t>(8192, ((size_t)p.nb * p.ncouls + 255) / 256);
         hipLaunchKernelGGL(k_permute_rows, dim3((unsigned)blocks), dim3(256), 0, s, p.aqsn, perm, p.nb, p.ncouls,
-                           aqsn_p, Stamp{});
+                           at(L.aqsn));
         GPP_TRY(hipGetLastError());
+        aqsn_p = at(L.aqsn);
     }
-    Stamp st = stage("bucket_factored");
-    for (int b = 0; b < nbk; ++b) {
-        const DevProblem q = bucket_problem(p, bp, b, aqsm_p, aqsn_p);
-        DevResults r;
-        r.base = bres + bp.tab[3 * b];
-        r.nfreq = p.nfreq;
-        r.nb = q.nb;
-        GPP_TRY(run_factored(q, kind, w + L.sub, r, s, nullptr, b == 0 ? st : Stamp{}));
+    DevProblem all = p;
+    all.aqsn = aqsn_p;
+    Stamp st = stage("bucket_factored");  // for the first launch of the stage
+    const auto first = [&st]() {
+        const Stamp f = st;
+        st = Stamp{};
+        return f;
+    };
+    size_t col = 0;  // next free column partial
+    for (int s0 = 0; s0 < nbk; s0 += L.group) {
+        const int s1 = std::min(nbk, s0 + L.group);
+        GramSlots g;
+        g.dev = bp.dev_slots() + 3 * s0;
+        g.n = s1 - s0;
+        int bare0 = s1;  // first slot of the group's bare buckets (they come last)
+        for (int sl = s1; sl-- > s0;) {
+            const DevProblem q = bucket_problem(p, bp, bp.slot[sl], aqsn_p);
+            if (slot_kind(q, kind) == kSlotBare) bare0 = sl;
+            g.bands += q.nb - q.nv;
+        }
+        const bool together = !kind.ozaki_slices && !kind.fuse;
+        if (together) GPP_TRY(launch_gram_f64(all, g, kind.tile, bg, mu, first(), s));
+        for (int sl = s0; sl < s1; ++sl) {
+            const int b = bp.slot[sl];
+            const DevProblem q = bucket_problem(p, bp, b, aqsn_p);
+            const cplx *const bgq = bg + (size_t)bp.start[b] * p.ngpown;
+            cplx *const muq = mu + (size_t)(sl - s0) * p.ngpown * p.ncouls;
+            cplx *const ca = at(L.col_ach) + col * p.nfreq, *const cx = at(L.col_asx) + col * p.nfreq;
+            const SlotKind k = slot_kind(q, kind);
+            if (k == kSlotFused) {
+                GPP_TRY(run_gram_pole(q, bgq, at(L.tile_ach), at(L.tile_asx), (p.ncouls + FuseCfg::TI - 1) / FuseCfg::TI,
+                                      ca, cx, first(), nullptr, s));
+                col += p.ngpown;
+                continue;
+            }
+            if (kind.ozaki_slices)
+                GPP_TRY(launch_gram_ozaki(q, kind.ozaki_slices, kind.int8, kind.layout, kind.group, bgq, w + L.sub, muq,
+                                          first(), s));
+            else if (!together)
+                GPP_TRY(launch_gram_f64(all, GramSlots{bp.dev_slots() + 3 * sl, 1, q.nb - q.nv}, kind.tile, bg, muq,
+                                        first(), s));
+            if (k == kSlotPlain) {
+                GPP_TRY(run_pole_reduce(q, kind, muq, bgq, ca, cx, L.nsplit, ab, Stamp{}, s));
+                col += (size_t)p.ngpown * L.nsplit;
+            } else if (kind.acht) {
+                hipLaunchKernelGGL(k_pole_p2, dim3(2048), dim3(256), 0, s, q.wtilde, q.ieps, q.wx + acht_frequency(q),
+                                   (size_t)p.ngpown * p.ncouls, ab.p2);
+                GPP_TRY(hipGetLastError());
+            }
+            if (kind.acht) {
+                const int chunk = acht_occ_chunk(q, kind.red_chunk);
+                const int nsplit = reduce_sums_acht_occ(q.nv, q.wx_neg) ? L.nsplit : (p.ncouls + chunk - 1) / chunk;
+                GPP_TRY(run_acht(q, acht_split(q), chunk, nsplit, ab, bgq, bp.dev_perm() + bp.start[b],
+                                 res.acht_n1_loc(), Stamp{}, nullptr, s));
+            }
+        }
+        if (bare0 < s1) {
+            BareArgs a;
+            a.mu = mu + (size_t)(bare0 - s0) * p.ngpown * p.ncouls;
+            a.slots = bp.dev_slots() + 3 * bare0;
+            a.nslots = s1 - bare0;
+            a.ieps = p.ieps; a.wtilde = p.wtilde; a.idx = p.idx; a.vcoul = p.vcoul; a.wx = p.wx;
+            a.ncouls = p.ncouls; a.ngpown = p.ngpown; a.nfreq = p.nfreq;
+            a.nsplit = L.bare_nsplit; a.chunk = L.bare_chunk;
+            a.col_ach = at(L.col_ach) + col * p.nfreq;
+            a.col_asx = at(L.col_asx) + col * p.nfreq;
+            launch_reduce_bare(a, s);
+            GPP_TRY(hipGetLastError());
+            col += (size_t)p.ngpown * L.bare_nsplit;
+        }
     }
     st = stage("bucket_combine");
-    hipLaunchKernelGGL(k_bucket_combine, dim3(1), dim3(256), 0, s, bres, tab, perm, nbk, p.nfreq, p.nb, res.base, st,
+    hipLaunchKernelGGL(k_fact_final, dim3(p.nfreq + 1), dim3(kRedThreads), 0, s, at(L.col_ach), at(L.col_asx),
+                       part_achs, L.ncols, p.nfreq, p.nb, p.nv, res.base, !kind.acht, st,
                        timer ? timer->end() : nullptr);
     return hipGetLastError();
 }

@@ -1317,17 +1317,106 @@ __device__ __forceinline__ void acht_occ_item(const cplx *__restrict__ p2, const
     }
 }
 
+// Stage 3 of buckets without occupied bands (band-dependent frequencies): one
+// pass over the elements of column j and G-vectors [split*chunk, +chunk)
+// evaluates every bucket's pole terms and adds them to the same sums, so
+// wtilde and I_eps are read once for all buckets instead of once for each and
+// a block has only its F sums to reduce.  A thread holds kBareE elements; each
+// bucket's Mu loads while the one before is evaluated.  What bounds it is the
+// memory below about four frequencies, the FP64 units above.  F frequencies
+// from blockIdx.z * F.
+constexpr int kBareE = 4, kBareStep = kBareE * kRedThreads;
+struct BareArgs {
+    const cplx *mu;        // [nslots][ngpown][ncouls]
+    const int32_t *slots;  // [nslots][3]: the third entry is the slot's row of wx
+    int nslots;
+    const cplx *ieps, *wtilde;
+    const int32_t *idx;
+    const double *vcoul, *wx;
+    int ncouls, ngpown, nfreq, nsplit, chunk;
+    cplx *col_ach, *col_asx;  // [ngpown][nsplit][nfreq]
+};
+template <int F> __device__ __forceinline__ void pole_reduce_bare(const BareArgs &a, cplx *scratch)
+{
+    const int j = blockIdx.x, split = blockIdx.y, iw0 = blockIdx.z * F;
+    const int ig_begin = split * a.chunk;
+    const int ig_end = ig_begin + a.chunk < a.ncouls ? ig_begin + a.chunk : a.ncouls;
+    const size_t row = (size_t)j * a.ncouls, mu_step = (size_t)a.ngpown * a.ncouls;
+    cplx sach[F];
+#pragma unroll
+    for (int f = 0; f < F; ++f) sach[f] = czero();
+    auto ld = [](const cplx *p) {  // read once
+        return cplx{__builtin_nontemporal_load(&p->re), __builtin_nontemporal_load(&p->im)};
+    };
+    for (int ig0 = ig_begin + threadIdx.x; ig0 < ig_end; ig0 += kBareStep) {
+        cplx wt[kBareE], q[kBareE], mu[kBareE];
+        double wti2[kBareE];
+        size_t at[kBareE];
+#pragma unroll
+        for (int e = 0; e < kBareE; ++e) {  // elements past the end repeat the last one, with q = 0
+            at[e] = row + min(ig0 + e * kRedThreads, ig_end - 1);
+            wt[e] = a.wtilde[at[e]];
+            q[e] = a.ieps[at[e]];
+            mu[e] = ld(a.mu + at[e]);
+        }
+#pragma unroll
+        for (int e = 0; e < kBareE; ++e) {
+            q[e] = cmul_fast(wt[e], q[e]);
+            wti2[e] = wt[e].im * wt[e].im;
+        }
+        const cplx *mub = a.mu;
+        for (int b = 0; b < a.nslots; ++b) {
+            const double *const wx = a.wx + (size_t)a.slots[3 * b + 2] * a.nfreq;
+            double wxv[F];
+#pragma unroll
+            for (int f = 0; f < F; ++f) wxv[f] = wx[min(iw0 + f, a.nfreq - 1)];
+            if (b + 1 < a.nslots) mub += mu_step;
+            cplx mu_n[kBareE];
+#pragma unroll
+            for (int e = 0; e < kBareE; ++e) mu_n[e] = ld(mub + at[e]);
+#pragma unroll
+            for (int e = 0; e < kBareE; ++e) {
+                if (ig0 + e * kRedThreads >= ig_end) break;
+                // u conj(wdiff) / |wdiff|^2 with u = q Mu (pole_reduce_item)
+                const cplx u = cmul_fast(q[e], mu[e]);
+                const double uiw = u.im * wt[e].im, urw = u.re * wt[e].im;
+#pragma unroll
+                for (int f = 0; f < F; ++f) {
+                    const double wdr = wxv[f] - wt[e].re;
+                    const double rden = rcp_1nr(__builtin_fma(wdr, wdr, wti2[e]));
+                    sach[f].re = __builtin_fma(__builtin_fma(u.re, wdr, -uiw), rden, sach[f].re);
+                    sach[f].im = __builtin_fma(__builtin_fma(u.im, wdr, urw), rden, sach[f].im);
+                }
+            }
+#pragma unroll
+            for (int e = 0; e < kBareE; ++e) mu[e] = mu_n[e];
+        }
+    }
+    const double vc = a.vcoul[igp_of(a.idx, j, a.ncouls)];
+#pragma unroll
+    for (int f = 0; f < F; ++f) {
+        const cplx s = block_sum(sach[f], scratch);
+        if (threadIdx.x == 0 && iw0 + f < a.nfreq) {
+            const size_t o = ((size_t)j * a.nsplit + split) * a.nfreq + iw0 + f;
+            a.col_ach[o] = cscale(cscale(s, 0.5), vc);
+            a.col_asx[o] = czero();
+        }
+    }
+}
+
 // Stage 4: block `part` < nfreq forms achtemp[part] / asxtemp[part] as
 // fixed-order sums over the (column, split) partials; block part == nfreq
-// sets acht_n1_loc to NaN (the factored forms write it in a later stage when
-// it is requested) and sums the per-(band, column group) achstemp partials.
-__device__ __forceinline__ void final_block(const cplx *col_ach, const cplx *col_asx, const cplx *part_achs, int ncols,
-                                            int nfreq, int nb, int nv, cplx *out, cplx *scratch, int part)
+// sets acht_n1_loc to NaN (nan_acht; the factored forms write it in a stage of
+// its own when it is requested) and sums the per-(band, column group) achstemp
+// partials.
+__device__ __forceinline__ void final_block(const cplx *col_ach, const cplx *col_asx, const cplx *part_achs,
+                                            long long ncols, int nfreq, int nb, int nv, cplx *out, cplx *scratch, int part,
+                                            bool nan_acht = true)
 {
     if (part < nfreq) {
         const int iw = part;
         cplx s = czero(), x = czero();
-        for (int c = threadIdx.x; c < ncols; c += blockDim.x) {
+        for (long long c = threadIdx.x; c < ncols; c += blockDim.x) {
             s = cadd(s, col_ach[(size_t)c * nfreq + iw]);
             x = cadd(x, col_asx[(size_t)c * nfreq + iw]);
         }
@@ -1340,7 +1429,7 @@ __device__ __forceinline__ void final_block(const cplx *col_ach, const cplx *col
         return;
     }
     const double nan = __builtin_nan("");
-    for (int n1 = threadIdx.x; n1 < nb; n1 += blockDim.x) out[2 * nfreq + n1] = cplx{nan, nan};
+    for (int n1 = threadIdx.x; nan_acht && n1 < nb; n1 += blockDim.x) out[2 * nfreq + n1] = cplx{nan, nan};
     cplx h = czero();
     for (int t = threadIdx.x; t < nb * kAchSplit; t += blockDim.x) h = cadd(h, part_achs[t]);
     h = block_sum(h, scratch);

@@ -110,8 +110,9 @@ struct CompatOut {
 hipError_t run_direct_part(const DevProblem &p, int which, void *work, const CompatOut &co, hipStream_t s);
 
 // achstemp per band into part_achs[nb] (fixed-order sums over j); with bg non-null also the gathered
-// rows Bg[n1][j] = aqsm[n1][igp(j)] [nb][ngpown].
-hipError_t launch_achstemp(const DevProblem &p, cplx *part_achs, cplx *bg, Stamp stamp, hipStream_t s);
+// rows Bg[n1][j] = aqsm[n1][igp(j)] [nb][ngpown].  perm: row r of both is band perm[r] (null: r).
+hipError_t launch_achstemp(const DevProblem &p, cplx *part_achs, cplx *bg, Stamp stamp, hipStream_t s,
+                           const int32_t *perm = nullptr);
 
 // Zeroes n ints with a fill kernel (no memset node when a caller captures).
 hipError_t launch_zero_ints(int *d_p, int n, hipStream_t s);
@@ -146,9 +147,8 @@ struct GramKind {
 constexpr int kGramTiles = 4;
 
 size_t factored_workspace_bytes(const DevProblem &p, GramKind kind);
-// first: without a timer, the stamp of the first launch.
 hipError_t run_factored(const DevProblem &p, GramKind kind, void *work, const DevResults &res,
-                        hipStream_t s, StageTimer *timer, Stamp first = Stamp{});
+                        hipStream_t s, StageTimer *timer);
 
 // Band-dependent frequencies (gpp_factored.hip): bands grouped by identical
 // wx rows; bucket b holds bands perm[start[b] .. start[b]+size[b]), its
@@ -156,14 +156,25 @@ hipError_t run_factored(const DevProblem &p, GramKind kind, void *work, const De
 struct BucketPlan {
     std::vector<int32_t> perm;
     std::vector<int> start, size, nocc, row;
-    std::vector<int> neg;      // per bucket: its row has a negative frequency
-    std::vector<int32_t> tab;  // per bucket: result offset, start, size
-    size_t nres = 0;           // complex results of all buckets (DevResults each)
+    std::vector<int> neg;   // per bucket: its row has a negative frequency
+    bool identity = false;  // perm leaves every band in place
+    // Buckets in the order they are worked on: the nslot_occ ones with
+    // occupied bands, then the others, each most unoccupied bands first (the
+    // longest Gram tiles start first).
+    std::vector<int> slot;
+    int nslot_occ = 0;
+    // Device copy of tables(): perm, then per slot (first, end) of its
+    // unoccupied rows in permuted order and its frequency row.  The owner of
+    // the plan uploads it.
+    std::vector<int32_t> tables() const;
+    const int32_t *dev = nullptr;
+    const int32_t *dev_perm() const { return dev; }
+    const int32_t *dev_slots() const { return dev + perm.size(); }
 };
 BucketPlan plan_buckets(const double *wx_rows, int nb, int nv, int nfreq);
 size_t bucketed_workspace_bytes(const DevProblem &p, GramKind kind, const BucketPlan &bp);
-// p.wx is [nb][nfreq] (wx_stride == nfreq); the host vectors of bp must stay
-// alive until the stream has run the call.
+// p.wx is [nb][nfreq] (wx_stride == nfreq); bp.dev must be set, and stay alive
+// until the stream has run the call.
 hipError_t run_factored_bucketed(const DevProblem &p, GramKind kind, const BucketPlan &bp, void *work,
                                  const DevResults &res, hipStream_t s, StageTimer *timer);
 
