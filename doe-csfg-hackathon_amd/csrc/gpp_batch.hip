@@ -163,7 +163,7 @@ template <int FC, int NV, bool NEG = false>
 __global__ __launch_bounds__(kRedThreads, FC > 8 || (NEG && FC > 4) ? 2 : 3) void k_batch_reduce(const BInst *__restrict__ insts,
                                                                  const RedItem *__restrict__ items, int chunk)
 {
-    __shared__ cplx scratch[kRedThreads / kWave];
+    __shared__ __attribute__((aligned(16))) cplx lds[pole_lds_entries<FC, NV>()];
     const RedItem it = items[blockIdx.x];
     const BInst &b = insts[it.inst];
     ReduceArgs ra;
@@ -173,7 +173,7 @@ __global__ __launch_bounds__(kRedThreads, FC > 8 || (NEG && FC > 4) ? 2 : 3) voi
     ra.col_ach = b.col_ach; ra.col_asx = b.col_asx;
     ra.p2 = nullptr; ra.br1 = nullptr; ra.acht_iw = -1; ra.part_occ = nullptr;
     ra.fpb = b.nfreq;
-    pole_reduce_item<FC, NV, false, (FC > 4 ? 4 : FC), NEG>(ra, it.j, it.split, 0, b.nfreq, scratch);
+    pole_reduce_item<FC, NV, false, (FC > 4 ? 4 : FC), NEG>(ra, it.j, it.split, 0, b.nfreq, lds);
 }
 
 __global__ __launch_bounds__(kRedThreads) void k_batch_final(const BInst *__restrict__ insts)

@@ -299,10 +299,10 @@ __global__ __launch_bounds__(kRedThreads, (FC <= 3 && !P2 && !NEG) ? 4 : FC > 8 
 {
     int fpb = a.fpb;
     const StampStart stamp(a.stamp, fpb);
-    __shared__ cplx scratch[kRedThreads / kWave];
+    __shared__ __attribute__((aligned(16))) cplx lds[pole_lds_entries<FC, NV>()];
     const int iw_begin = blockIdx.z * fpb;
     const int iw_end = iw_begin + fpb < a.nfreq ? iw_begin + fpb : a.nfreq;
-    pole_reduce_item<FC, NV, P2, (FC > 4 ? 4 : FC), NEG>(a, blockIdx.x, blockIdx.y, iw_begin, iw_end, scratch);
+    pole_reduce_item<FC, NV, P2, (FC > 4 ? 4 : FC), NEG>(a, blockIdx.x, blockIdx.y, iw_begin, iw_end, lds);
     stamp.store();
 }
 

@@ -512,8 +512,8 @@ constexpr double kBand = 1.0 / 1099511627776.0;
 // with the correctly rounded reciprocal (:30-32).  An est of +inf (the
 // product overflowed) means a |delw|^2 of at least about 1.8e308, far above
 // both thresholds, where the reference decides alike (branch 2).
-__device__ __forceinline__ void occ_branch_tests(double wxf, cplx wt, double wdiffr, double rden, double wt2,
-                                                 bool &branch1, bool &above2)
+// The decisions from est alone; false where they are not sure.
+__device__ __forceinline__ bool occ_branch_estimate(double wdiffr, double rden, double wt2, bool &branch1, bool &above2)
 {
 #pragma clang fp contract(off)
     constexpr double limitone = 1.0 / (kTo1 * 4.0);
@@ -522,17 +522,23 @@ __device__ __forceinline__ void occ_branch_tests(double wxf, cplx wt, double wdi
     const double est = wt2 * rden;
     // below the to1 band (|delw|^2 < 1e-6, where |wdiff| exceeds |wt| a
     // thousandfold) is rare enough to take the exact path with the bands
-    const bool sure = ((est > kEstHi2) & (est < kEstLo1)) | (est > kEstHi1);
-    bool below1 = est < kEstLo1;
+    const bool below1 = est < kEstLo1;
     above2 = est > kEstHi2;
-    if (!sure) {
+    branch1 = (wdiffr > 0.25) && below1;
+    return (above2 & below1) | (est > kEstHi1);
+}
+__device__ __forceinline__ void occ_branch_tests(double wxf, cplx wt, double wdiffr, double rden, double wt2,
+                                                 bool &branch1, bool &above2)
+{
+#pragma clang fp contract(off)
+    if (!occ_branch_estimate(wdiffr, rden, wt2, branch1, above2)) {
+        constexpr double limitone = 1.0 / (kTo1 * 4.0);
         const cplx wdiff = cdminus(wxf, wt);
         const cplx delw = cscale(cmul(wt, cconj(wdiff)), rcp_refined(wdiffr));
         const double delwr = cmul(delw, cconj(delw)).re;
-        below1 = delwr < limitone;
+        branch1 = (wdiffr > 0.25) && delwr < limitone;
         above2 = delwr > kTo1;
     }
-    branch1 = (wdiffr > 0.25) && below1;
 }
 
 // One instance's inputs and workspace as seen by the reduce stages.
@@ -566,6 +572,15 @@ struct ReduceArgs {
 // at 8 and 16 frequencies by 45-297 registers).
 __host__ __device__ inline bool reduce_sums_acht_occ(int nv, int neg) { return !neg && nv == 2; }
 
+// LDS of pole_reduce_item: block_sum's scratch, then (pole_stages) one aqsn
+// value per occupied band and thread.
+constexpr int kStageNv = 8;  // most occupied bands staged in LDS
+template <int FC, int NV> constexpr bool pole_stages() { return FC > 3; }
+template <int FC, int NV> constexpr int pole_lds_entries()
+{
+    return kRedThreads / kWave + (pole_stages<FC, NV>() ? (NV > 0 ? NV : kStageNv) * kRedThreads : 0);
+}
+
 // Stage 3: pole terms of column j over G-vectors [split*chunk, +chunk), for
 // frequencies [iw0, iw0+FC).  Per element and frequency: wdiff, |wdiff|^2,
 // delw = wt*conj(wdiff)*rden and |delw|^2 in the reference's order
@@ -586,12 +601,24 @@ __host__ __device__ inline bool reduce_sums_acht_occ(int nv, int neg) { return !
 // whose partials it writes to part_occ).
 template <int FC, int NV = 0, bool P2 = false, int FCT = FC, bool NEG = false>
 __device__ __forceinline__ void pole_reduce_item(const ReduceArgs &a, int j, int split, int iw_begin, int iw_end,
-                                                 cplx *scratch)
+                                                 cplx *lds)
 {
 #pragma clang fp contract(off)
     const int ncouls = a.ncouls;
     const int nv = NV > 0 ? NV : a.nv;
     constexpr bool kOccSum = P2 && NV == 2 && !NEG;  // reduce_sums_acht_occ
+    // The occupied aqsn values of a thread's next G-vector load straight into
+    // LDS (its own entries, so no barrier) while the current one is evaluated.
+    // Loaded where they are used, the waves of these kernels (two or three a
+    // SIMD, no registers to load ahead into) stood 42% of their time waiting:
+    // reduce us 300/8/32768/1638/16 1574 -> 1488, 300/2/16384/819/8 220 -> 194,
+    // 300/5/16384/819/13 (any nv) 642 -> 552.  Not for the kernels of at most
+    // three frequencies, which the streams bound (four waves a SIMD; the
+    // p2-storing one took 203 against 192 us at 300/2/16384/819).
+    constexpr bool kStages = pole_stages<FC, NV>();
+    const bool staged = kStages && nv > 0 && (NV > 0 || nv <= kStageNv);
+    cplx *const scratch = lds, *const occ_wave = lds + kRedThreads / kWave + (threadIdx.x & ~(kWave - 1));
+    cplx *const occ_av = lds + kRedThreads / kWave + threadIdx.x;
 
     const int ig_begin = split * a.chunk;
     const int ig_end = ig_begin + a.chunk < ncouls ? ig_begin + a.chunk : ncouls;
@@ -643,19 +670,68 @@ __device__ __forceinline__ void pole_reduce_item(const ReduceArgs &a, int j, int
             else
                 return *p;
         };
+        // With kStages every lane loads: those past the end repeat the last
+        // G-vector and skip the evaluation.
         cplx wt_n = czero(), ie_n = czero(), mu_n = czero();
-        if (ig_begin + (int)threadIdx.x < ig_end) {
-            wt_n = ld(a.wtilde + row + ig_begin + threadIdx.x);
-            ie_n = ld(a.ieps + row + ig_begin + threadIdx.x);
-            mu_n = ld(a.mu + row + ig_begin + threadIdx.x);
-        }
-        for (int ig = ig_begin + threadIdx.x; ig < ig_end; ig += blockDim.x) {
-            const cplx wt = wt_n, ie = ie_n, mu = mu_n;
-            if (ig + (int)blockDim.x < ig_end) {
-                wt_n = ld(a.wtilde + row + ig + blockDim.x);
-                ie_n = ld(a.ieps + row + ig + blockDim.x);
-                mu_n = ld(a.mu + row + ig + blockDim.x);
+        const int lane0 = kStages ? 0 : (int)threadIdx.x;  // the loop index: the block's, or the lane's
+        auto load_next = [&](int i) {
+            const int ig = kStages ? min(i + (int)threadIdx.x, ig_end - 1) : i;
+            if (staged) {
+#pragma unroll
+                for (int n1 = 0; n1 < (NV > 0 ? NV : kStageNv); ++n1)
+                    if (NV > 0 || n1 < nv) ring_load(a.aqsn + (size_t)n1 * ncouls + ig, occ_wave + n1 * kRedThreads);
             }
+            wt_n = ld(a.wtilde + row + ig);
+            ie_n = ld(a.ieps + row + ig);
+            mu_n = ld(a.mu + row + ig);
+        };
+        if (ig_begin + lane0 < ig_end) load_next(ig_begin + lane0);
+        for (int i = ig_begin + lane0; i < ig_end; i += kStages ? kRedThreads : blockDim.x) {
+            const int ig = kStages ? i + (int)threadIdx.x : i;
+            if constexpr (kStages) {
+                // the loads of this element, all older than the rest
+                __builtin_amdgcn_s_waitcnt((7 << 4) | (15 << 8));  // vmcnt(0)
+                asm volatile("" ::: "memory");
+            }
+            const cplx wt = wt_n, ie = ie_n, mu = mu_n;
+            // Mo over the occupied bands, in band order: folded passes
+            // take four FMAs per band (C3 reduce 7.54 -> 7.33 ms, C4 14.39
+            // -> 14.14 ms), the three-frequency kernel a product and a sum
+            // (0.487 against 0.501 ms at 512/2/32768/1638)
+            cplx mo = czero();
+            cplx av[NV > 0 ? NV : 1];  // the occupied aqsn of this G-vector, loads issued together
+            auto form_mo = [&]() {
+                if constexpr (NV > 0 && kStages) {
+#pragma unroll
+                    for (int h = 0; h < NV; h += 4) {  // four at a time in registers
+#pragma unroll
+                        for (int n1 = h; n1 < NV && n1 < h + 4; ++n1) av[n1] = occ_av[n1 * kRedThreads];
+#pragma unroll
+                        for (int n1 = h; n1 < NV && n1 < h + 4; ++n1)
+                            mo = !FOLD ? cadd(mo, cmul_fast(bgc[n1], av[n1]))
+                                       : n1 == 0 ? cmul_fast(bgc[0], av[0]) : cfma(bgc[n1], av[n1], mo);
+                        asm volatile("" : "+v"(mo.re), "+v"(mo.im));
+                    }
+                } else if constexpr (NV > 0) {
+#pragma unroll
+                    for (int n1 = 0; n1 < NV; ++n1) av[n1] = a.aqsn[(size_t)n1 * ncouls + ig];
+#pragma unroll
+                    for (int n1 = 0; n1 < NV; ++n1) mo = cadd(mo, cmul_fast(bgc[n1], av[n1]));
+                } else {
+                    for (int n1 = 0; n1 < nv; ++n1) {
+                        const cplx b = cconj(a.bg[(size_t)n1 * a.ngpown + j]);
+                        const cplx v =
+                            staged ? occ_av[n1 * kRedThreads] : a.aqsn[(size_t)n1 * ncouls + min(ig, ig_end - 1)];
+                        mo = FOLD ? cfma(b, v, mo) : cadd(mo, cmul_fast(b, v));
+                    }
+                }
+            };
+            if constexpr (kStages) {
+                form_mo();
+                asm volatile("" ::: "memory");  // the reads before the next loads
+            }
+            if (i + (int)(kStages ? kRedThreads : blockDim.x) < ig_end) load_next(i + (kStages ? kRedThreads : blockDim.x));
+            if (kStages && ig >= ig_end) break;
             // P = delw I_eps = q conj(wdiff) / |wdiff|^2 with q = wt I_eps and
             // conj(wdiff) = (wx - wt.re, wt.im) =: (wdr, wt.im).  FOLD (problems
             // with 4 or more frequencies) folds Mu and Mo into the products
@@ -672,38 +748,15 @@ __device__ __forceinline__ void pole_reduce_item(const ReduceArgs &a, int j, int
             // q.im wt.im and q.re wt.im: kept per element when P is formed every
             // frequency, recomputed on the rare paths otherwise
             const double q_im_wti_e = FOLD ? 0.0 : q.im * wt.im, q_re_wti_e = FOLD ? 0.0 : q.re * wt.im;
-            cplx mo = czero(), om2 = czero(), mum = mu, u0 = czero(), uo = czero(), w1 = czero();
+            cplx om2 = czero(), mum = mu, u0 = czero(), uo = czero(), w1 = czero();
             double u0_im_wti = 0.0, u0_re_wti = 0.0, uo_im_wti = 0.0, uo_re_wti = 0.0, ie_cut = 0.0, wt2 = 0.0;
             if constexpr (FOLD) {
                 u0 = cmul_fast(q, mu);
                 u0_im_wti = u0.im * wt.im;
                 u0_re_wti = u0.re * wt.im;
             }
-            cplx av[NV > 0 ? NV : 1];  // the occupied aqsn of this G-vector, loads issued together
             if (nv > 0) {
-                // Mo over the occupied bands, in band order: folded passes
-                // take four FMAs per band (C3 reduce 7.54 -> 7.33 ms, C4 14.39
-                // -> 14.14 ms), the three-frequency kernel a product and a sum
-                // (0.487 against 0.501 ms at 512/2/32768/1638)
-                if constexpr (NV > 0) {
-#pragma unroll
-                    for (int n1 = 0; n1 < NV; ++n1) av[n1] = a.aqsn[(size_t)n1 * ncouls + ig];
-                }
-                if constexpr (NV > 0 && FOLD) {
-                    mo = cmul_fast(bgc[0], av[0]);
-#pragma unroll
-                    for (int n1 = 1; n1 < NV; ++n1) mo = cfma(bgc[n1], av[n1], mo);
-                } else if constexpr (NV > 0) {
-#pragma unroll
-                    for (int n1 = 0; n1 < NV; ++n1) mo = cadd(mo, cmul_fast(bgc[n1], av[n1]));
-                } else if constexpr (FOLD) {
-                    for (int n1 = 0; n1 < nv; ++n1)
-                        mo = cfma(cconj(a.bg[(size_t)n1 * a.ngpown + j]), a.aqsn[(size_t)n1 * ncouls + ig], mo);
-                } else {
-                    for (int n1 = 0; n1 < nv; ++n1)
-                        mo = cadd(mo, cmul_fast(cconj(a.bg[(size_t)n1 * a.ngpown + j]),
-                                                a.aqsn[(size_t)n1 * ncouls + ig]));
-                }
+                if constexpr (!kStages) form_mo();
                 om2 = cmul(csquare(wt), ie);  // Omega2 = wtilde^2 * I_eps, flagOCC_solver :117-118
                 if constexpr (FOLD) {
                     uo = cmul_fast(q, mo);
@@ -721,17 +774,47 @@ __device__ __forceinline__ void pole_reduce_item(const ReduceArgs &a, int j, int
                     ie_cut = cabs_(ie) * kSexcut;
                 }
             }
+            // Frequencies in groups: their reciprocals, u terms and branch
+            // estimates are formed together, before any branch on them, and
+            // overlap (with two or three waves a SIMD nothing else hides a
+            // reciprocal's latency).  Two: 300/8/32768/1638/16 1488 -> 1430 us,
+            // 300/4/16384/819/24 613 -> 583; groups of four need more registers
+            // than three waves have (300/5/16384/819/13 573 against 559).
+            // Masking the occupied terms too instead of branching on them took
+            // 13% longer: it adds more instructions than it overlaps.
+            constexpr int kGrp = FOLD && !NEG ? 2 : 1;
+            double wdrs[kGrp], rdens[kGrp];
+            bool b1s[kGrp], a2s[kGrp];
 #pragma unroll
             for (int f = 0; f < F; ++f) {
-                const double wdr = wxv[f] - wt.re;        // wdiff = (wdr, -wt.im), :27
-                const double wdiffr = wdr * wdr + wti2;   // |wdiff|^2 exactly as the reference rounds it
-                const double rden = rcp_1nr(wdiffr);
-                if constexpr (FOLD) {  // P Mu
-                    sach[f].re = __builtin_fma(__builtin_fma(u0.re, wdr, -u0_im_wti), rden, sach[f].re);
-                    sach[f].im = __builtin_fma(__builtin_fma(u0.im, wdr, u0_re_wti), rden, sach[f].im);
+                if (f % kGrp == 0) {
+                    double wdiffrs[kGrp];
+                    bool unsure = false;
+#pragma unroll
+                    for (int k = 0; k < kGrp && f + k < F; ++k) {
+                        wdrs[k] = wxv[f + k] - wt.re;                // wdiff = (wdr, -wt.im), :27
+                        wdiffrs[k] = wdrs[k] * wdrs[k] + wti2;       // |wdiff|^2 exactly as the reference rounds it
+                        rdens[k] = rcp_1nr(wdiffrs[k]);
+                        if constexpr (FOLD) {  // P Mu
+                            cplx &t = sach[f + k];
+                            t.re = __builtin_fma(__builtin_fma(u0.re, wdrs[k], -u0_im_wti), rdens[k], t.re);
+                            t.im = __builtin_fma(__builtin_fma(u0.im, wdrs[k], u0_re_wti), rdens[k], t.im);
+                        }
+                        b1s[k] = a2s[k] = false;
+                        if constexpr (kGrp == 1) {
+                            if (nv > 0) occ_branch_tests(wxv[f], wt, wdiffrs[k], rdens[k], wt2, b1s[k], a2s[k]);
+                        } else if (nv > 0) {
+                            unsure |= !occ_branch_estimate(wdiffrs[k], rdens[k], wt2, b1s[k], a2s[k]);
+                        }
+                    }
+                    if (unsure) {
+#pragma unroll
+                        for (int k = 0; k < kGrp && f + k < F; ++k)
+                            occ_branch_tests(wxv[f + k], wt, wdiffrs[k], rdens[k], wt2, b1s[k], a2s[k]);
+                    }
                 }
-                bool branch1 = false, above2 = false;
-                if (nv > 0) occ_branch_tests(wxv[f], wt, wdiffr, rden, wt2, branch1, above2);
+                const double wdr = wdrs[f % kGrp], rden = rdens[f % kGrp];
+                const bool branch1 = b1s[f % kGrp], above2 = a2s[f % kGrp];
                 // Branch 2 (:46-50) with cden = 4 wt^2 (0.5 + delw), Omega2 =
                 // wt^2 I_eps and delw = wt / (wx - wt):
                 //   -Omega2 conj(cden) delw / |cden|^2 = -I_eps delw / (2 + 4 delw)
