@@ -706,7 +706,7 @@ gpp_status gpp_ctx_set_stream(gpp_ctx *ctx, struct ihipStream_t *stream)
             return fail(GPP_ERR_INVALID_ARGUMENT, "stream is on device %d, the context on device %d", dev,
                         ctx->device);
     }
-    // the context's earlier work (results, timing events) finishes first
+    // the context's earlier work (results, stage times) finishes first
     HIP_OR_FAIL(hipStreamSynchronize(ctx->stream), "hipStreamSynchronize");
     ctx->stream = next;
     return GPP_OK;
@@ -974,7 +974,7 @@ gpp_status gpp_ctx_autotune(gpp_ctx *ctx, gpp_form form)
     double g, r, best = 1e300;
     if (form == GPP_FORM_FACTORED_F64)
         for (int tile = 0; tile < gpp::kGramTiles; ++tile) {
-            // Gram plus reduce (with GPP_OPT_FUSED_REDUCE the 128x128 tile
+            // Gram plus reduce (with GPP_OPT_FUSED_REDUCE tile 0
             // carries the reduce in its epilogue where it applies)
             if ((st = trial(tile, best_chunk, best_fc, &g, &r))) return st;
             if (g + r < best) best = g + r, best_tile = tile;

@@ -352,7 +352,7 @@ gpp_status gpp_ctx_wait(gpp_ctx *ctx, const gpp_outputs *out);
 
 /*
  * Enqueues the context's work on the caller's HIP stream (hipStream_t of the
- * context's device) instead of its own: uploads, evaluations, timing events,
+ * context's device) instead of its own: uploads, evaluations,
  * result copies and batch replays.  Work the caller enqueued on that stream
  * before gpp_sigma_async runs before the evaluation, and the caller's later
  * work runs after it, so a host application that owns its streams orders the
