@@ -4,7 +4,7 @@ over all of them, acht_n1_loc group by group.  Column and G-vector counts at
 the edges of their blocks (4 elements a thread, 256 threads: 1024), frequency
 counts at each pass width and over two passes, bands whose groups lie together
 (nothing is permuted), interleaved, and with occupied bands in several groups.
-The checker is the oracle's per-band loop; the bound is the factored forms'
+Compared with the oracle's per-band loop; the bound is the factored forms'
 1e-10 per component (tests/test_gpu_band_wx.py)."""
 import numpy as np
 import pytest
