@@ -444,9 +444,26 @@ void launch_reduce_p2(const ReduceArgs &a, dim3 grid, hipStream_t s)
         hipLaunchKernelGGL((k_pole_reduce<(FC > 8 ? 8 : FC), 0, P2, true>), grid, dim3(kRedThreads), 0, s, a);
         return;
     }
-    switch (a.nv) {  // the occupied band counts of the common shapes
+    // Up to eight occupied bands a kernel for each count (their loads issued
+    // together, conj(bg) in scalar registers), beyond it the general one.
+    // Reduce, us, general / own: 300/nv/16384/819, nv = 3 and 3 frequencies 184
+    // / 137, 7 and 3 233 / 177, 1 and 8 229 / 187, 5 and 13 562 / 376, 6 and 24
+    // 917 / 604; the p2-storing one of one band and at most 3 frequencies the
+    // other way, 186 / 194.
+    if constexpr (P2 && FC <= 3) {
+        if (a.nv == 1) {
+            hipLaunchKernelGGL((k_pole_reduce<FC, 0, P2>), grid, dim3(kRedThreads), 0, s, a);
+            return;
+        }
+    }
+    switch (a.nv) {
+    case 1: hipLaunchKernelGGL((k_pole_reduce<FC, (P2 && FC <= 3) ? 0 : 1, P2>), grid, dim3(kRedThreads), 0, s, a); break;
     case 2: hipLaunchKernelGGL((k_pole_reduce<FC, 2, P2>), grid, dim3(kRedThreads), 0, s, a); break;
+    case 3: hipLaunchKernelGGL((k_pole_reduce<FC, 3, P2>), grid, dim3(kRedThreads), 0, s, a); break;
     case 4: hipLaunchKernelGGL((k_pole_reduce<FC, 4, P2>), grid, dim3(kRedThreads), 0, s, a); break;
+    case 5: hipLaunchKernelGGL((k_pole_reduce<FC, 5, P2>), grid, dim3(kRedThreads), 0, s, a); break;
+    case 6: hipLaunchKernelGGL((k_pole_reduce<FC, 6, P2>), grid, dim3(kRedThreads), 0, s, a); break;
+    case 7: hipLaunchKernelGGL((k_pole_reduce<FC, 7, P2>), grid, dim3(kRedThreads), 0, s, a); break;
     case 8: hipLaunchKernelGGL((k_pole_reduce<FC, 8, P2>), grid, dim3(kRedThreads), 0, s, a); break;
     default: hipLaunchKernelGGL((k_pole_reduce<FC, 0, P2>), grid, dim3(kRedThreads), 0, s, a); break;
     }

@@ -14,7 +14,8 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize("nv,nc,nf", [
     (0, 257, 4), (1, 255, 5), (2, 256, 4), (2, 1023, 7), (3, 257, 8), (4, 513, 16), (5, 1, 4), (7, 300, 13),
-    (8, 769, 9), (8, 512, 24), (9, 257, 16), (12, 511, 6),
+    (8, 769, 9), (8, 512, 24), (9, 257, 16), (12, 511, 6), (1, 300, 3), (3, 257, 2), (5, 511, 3), (6, 770, 1),
+    (6, 257, 20), (7, 255, 3),
 ])
 def test_reduce_stages_vs_oracle(ctx, oracle, nv, nc, nf):
     ng = min(nc, 19)
