@@ -574,11 +574,10 @@ __host__ __device__ inline bool reduce_sums_acht_occ(int nv, int neg) { return !
 
 // LDS of pole_reduce_item: block_sum's scratch, then (pole_stages) one aqsn
 // value per occupied band and thread.
-constexpr int kStageNv = 8;  // most occupied bands staged in LDS
-template <int FC, int NV> constexpr bool pole_stages() { return FC > 3; }
+template <int FC, int NV> constexpr bool pole_stages() { return FC > 3 && NV > 0; }
 template <int FC, int NV> constexpr int pole_lds_entries()
 {
-    return kRedThreads / kWave + (pole_stages<FC, NV>() ? (NV > 0 ? NV : kStageNv) * kRedThreads : 0);
+    return kRedThreads / kWave + (pole_stages<FC, NV>() ? NV * kRedThreads : 0);
 }
 
 // Stage 3: pole terms of column j over G-vectors [split*chunk, +chunk), for
@@ -612,11 +611,11 @@ __device__ __forceinline__ void pole_reduce_item(const ReduceArgs &a, int j, int
     // Loaded where they are used, the waves of these kernels (two or three a
     // SIMD, no registers to load ahead into) stood 42% of their time waiting:
     // reduce us 300/8/32768/1638/16 1574 -> 1488, 300/2/16384/819/8 220 -> 194,
-    // 300/5/16384/819/13 (any nv) 642 -> 552.  Not for the kernels of at most
+    // 300/4/16384/819/24 663 -> 613.  Not for the general kernel (without
+    // occupied bands 302 -> 330 us at 200/0/16384/819/16) nor for the kernels of at most
     // three frequencies, which the streams bound (four waves a SIMD; the
     // p2-storing one took 203 against 192 us at 300/2/16384/819).
     constexpr bool kStages = pole_stages<FC, NV>();
-    const bool staged = kStages && nv > 0 && (NV > 0 || nv <= kStageNv);
     cplx *const scratch = lds, *const occ_wave = lds + kRedThreads / kWave + (threadIdx.x & ~(kWave - 1));
     cplx *const occ_av = lds + kRedThreads / kWave + threadIdx.x;
 
@@ -676,10 +675,9 @@ __device__ __forceinline__ void pole_reduce_item(const ReduceArgs &a, int j, int
         const int lane0 = kStages ? 0 : (int)threadIdx.x;  // the loop index: the block's, or the lane's
         auto load_next = [&](int i) {
             const int ig = kStages ? min(i + (int)threadIdx.x, ig_end - 1) : i;
-            if (staged) {
+            if constexpr (kStages) {
 #pragma unroll
-                for (int n1 = 0; n1 < (NV > 0 ? NV : kStageNv); ++n1)
-                    if (NV > 0 || n1 < nv) ring_load(a.aqsn + (size_t)n1 * ncouls + ig, occ_wave + n1 * kRedThreads);
+                for (int n1 = 0; n1 < NV; ++n1) ring_load(a.aqsn + (size_t)n1 * ncouls + ig, occ_wave + n1 * kRedThreads);
             }
             wt_n = ld(a.wtilde + row + ig);
             ie_n = ld(a.ieps + row + ig);
@@ -720,8 +718,7 @@ __device__ __forceinline__ void pole_reduce_item(const ReduceArgs &a, int j, int
                 } else {
                     for (int n1 = 0; n1 < nv; ++n1) {
                         const cplx b = cconj(a.bg[(size_t)n1 * a.ngpown + j]);
-                        const cplx v =
-                            staged ? occ_av[n1 * kRedThreads] : a.aqsn[(size_t)n1 * ncouls + min(ig, ig_end - 1)];
+                        const cplx v = a.aqsn[(size_t)n1 * ncouls + ig];
                         mo = FOLD ? cfma(b, v, mo) : cadd(mo, cmul_fast(b, v));
                     }
                 }
@@ -779,10 +776,10 @@ __device__ __forceinline__ void pole_reduce_item(const ReduceArgs &a, int j, int
             // overlap (with two or three waves a SIMD nothing else hides a
             // reciprocal's latency).  Two: 300/8/32768/1638/16 1488 -> 1430 us,
             // 300/4/16384/819/24 613 -> 583; groups of four need more registers
-            // than three waves have (300/5/16384/819/13 573 against 559).
+            // than three waves have.
             // Masking the occupied terms too instead of branching on them took
             // 13% longer: it adds more instructions than it overlaps.
-            constexpr int kGrp = FOLD && !NEG ? 2 : 1;
+            constexpr int kGrp = FOLD && !NEG && NV > 0 ? 2 : 1;
             double wdrs[kGrp], rdens[kGrp];
             bool b1s[kGrp], a2s[kGrp];
 #pragma unroll

@@ -1,7 +1,6 @@
 """The pole reduce with four or more frequencies loads the occupied bands' rows
 of a block's next 256 G-vectors through LDS: occupied band counts with a
-kernel of their own, the general one up to the eight bands it stages and
-beyond, G-vector counts at the edges of the 256, frequency counts at odd
+kernel of their own (one to eight) and the general one's, G-vector counts at the edges of the 256, frequency counts at odd
 groups of two and over several passes.  Against the oracle at the factored
 forms' 1e-10 per component (tests/test_gpu_factored.py)."""
 import pytest
