@@ -759,6 +759,7 @@ gpp_status sigma_enqueue(gpp_ctx *ctx, gpp_form form, bool acht)
         const bool factored = form != GPP_FORM_DIRECT && form != GPP_FORM_DIRECT_STRICT;
         if (factored && nbk == 1) {
             dp.wx = static_cast<const double *>(ctx->wxb.ptr);
+            dp.wx_neg = ctx->bplan.neg[0];  // dp's flag is the shared row's
         } else {
             dp.wx = static_cast<const double *>(ctx->wxb.ptr);
             dp.wx_stride = dp.nfreq;
