@@ -372,8 +372,9 @@ constexpr int kAchtFinalBands = 16;
 __global__ __launch_bounds__(256) void k_acht_final(const cplx *__restrict__ part, int nparts,
                                                     const cplx *__restrict__ part_occ, int nparts_occ, int nb,
                                                     int nv, const int32_t *__restrict__ perm,
-                                                    cplx *__restrict__ out, unsigned long long *end)
+                                                    cplx *__restrict__ out, Stamp stamp, unsigned long long *end)
 {
+    stamp_start(stamp);  // where no launch of the stage came before
     __shared__ cplx grp[256 / kAchtFinalBands][kAchtFinalBands];
     const int nblk = (nb + kAchtFinalBands - 1) / kAchtFinalBands;
     if ((int)blockIdx.x < nblk) {
@@ -651,9 +652,10 @@ hipError_t run_acht(const DevProblem &p, const AchtSplit &as, int occ_chunk, int
         hipLaunchKernelGGL(k_acht_occ, dim3(p.ngpown, occ_nsplit), dim3(kRedThreads), 0, s, ab.p2, ab.br1, p.aqsn,
                            bg, p.idx, p.vcoul, p.ngpown, p.ncouls, p.nv, occ_chunk, occ_nsplit, ab.part_occ, st);
         GPP_TRY(hipGetLastError());
+        st = Stamp{};
     }
     hipLaunchKernelGGL(k_acht_final, dim3((p.nb + kAchtFinalBands - 1) / kAchtFinalBands + p.nv), dim3(256), 0, s,
-                       ab.part, as.jtiles * as.nks, ab.part_occ, p.ngpown * occ_nsplit, p.nb, p.nv, perm, out, end);
+                       ab.part, as.jtiles * as.nks, ab.part_occ, p.ngpown * occ_nsplit, p.nb, p.nv, perm, out, st, end);
     return hipGetLastError();
 }
 
