@@ -1558,11 +1558,12 @@ gpp_status d_noFlagOCCSolver(int number_bands, int nvband, int ngpown, int ncoul
 
 // ---------------------------------------------------------------------------
 // The launcher that allocates nothing: d_noFlagOCCSolver with its scratch --
-// the index flag, the results and the direct form's partial sums -- in one
+// the index flag and the direct form's partial sums -- in one
 // file-scope device array instead of the grow-only per-device workspace.
 namespace {
 
-constexpr size_t kNoAllocScratchBytes = (size_t)16 << 20;  // 16 MiB per device
+using gpp::kNoAllocHeadBytes;
+using gpp::kNoAllocScratchBytes;
 constexpr int kNoAllocMaxDevices = 64;
 
 }  // namespace
@@ -1610,8 +1611,8 @@ gpp_status d_noFlagOCCSolver_noalloc(int number_bands, int nvband, int ngpown, i
         return fail(GPP_ERR_INVALID_ARGUMENT, "NULL device array");
     const gpp::DevProblem dp = compat_problem(number_bands, nvband, ncouls, ngpown, inv_igp_index, wx_array, vcoul,
                                               aqsmtemp, aqsntemp, I_eps_array, wtilde_array, 1.0);
-    // scratch: [index flag: 256 B][direct-form partial sums]
-    const size_t need = 256 + gpp::direct_workspace_bytes(dp);
+    // scratch: [index flag][direct-form partial sums]
+    const size_t need = kNoAllocHeadBytes + gpp::direct_workspace_bytes(dp);
     if (need > kNoAllocScratchBytes)
         return fail(GPP_ERR_INVALID_ARGUMENT,
                     "number_bands=%d ngpown=%d needs %zu bytes of scratch; d_noFlagOCCSolver_noalloc holds %zu "
@@ -1634,7 +1635,7 @@ gpp_status d_noFlagOCCSolver_noalloc(int number_bands, int nvband, int ngpown, i
     co.achtemp_re = achtemp_re;
     co.achtemp_im = achtemp_im;
     co.acht_n1 = reinterpret_cast<cplx *>(acht_n1_loc);
-    HIP_OR_FAIL(gpp::run_direct_part(dp, 1, base + 256, co, s), "direct launch");
+    HIP_OR_FAIL(gpp::run_direct_part(dp, 1, base + kNoAllocHeadBytes, co, s), "direct launch");
     return GPP_OK;
 }
 

@@ -78,29 +78,10 @@ __host__ inline size_t align256(size_t x) { return (x + 255) & ~(size_t)255; }
 // 131/5/2477/123 with 7 frequencies).
 constexpr int pass_width(bool strict) { return strict ? 3 : 4; }
 
-// G ranges per (band, column tile): the split that leaves the blocks in flight
-// least idle in the last round, with at least six chunks of 64 G-vectors per
-// range (a range costs its staging's start and a reduction of its
-// accumulators, about 1 % of a block per extra range).  Launches of more than
-// 4096 blocks stay whole.
-int direct_split(const DevProblem &p)
+// The workspace with gs G ranges.
+WorkLayout layout_for(const DevProblem &p, int gs)
 {
-    const int njt = (p.ngpown + kBJ - 1) / kBJ, nun = p.nb - p.nv;
-    const double blocks = (double)(nun > 0 ? (nun + kNW - 1) / kNW : p.nv) * njt * ((p.nfreq + 3) / 4);
-    if (blocks > 4096) return 1;
-    const int chunks = (p.ncouls + kWave - 1) / kWave;
-    int best_gs = 1;
-    double best = 1e300;
-    for (int gs = 1; gs <= 16 && gs * 6 <= std::max(6, chunks) && (gs == 1 || blocks * gs <= 8192); ++gs) {
-        const double t = std::ceil(blocks * gs / kDirectSlots) / gs * (1.0 + 0.01 * gs);
-        if (t < best) best = t, best_gs = gs;
-    }
-    return best_gs;
-}
-
-WorkLayout layout_for(const DevProblem &p)
-{
-    const size_t nt = (size_t)((p.ngpown + kBJ - 1) / kBJ) * direct_split(p);
+    const size_t nt = (size_t)((p.ngpown + kBJ - 1) / kBJ) * gs;
     const size_t nvx = p.nv > 0 ? (size_t)p.nv : 1;
     WorkLayout L;
     size_t off = 0;
@@ -113,16 +94,40 @@ WorkLayout layout_for(const DevProblem &p)
     return L;
 }
 
+// G ranges per (band, column tile): the split that leaves the blocks in flight
+// least idle in the last round, with at least six chunks of 64 G-vectors per
+// range (a range costs its staging's start and a reduction of its
+// accumulators, about 1 % of a block per extra range).  Launches of more than
+// 4096 blocks stay whole, and a split's partial sums stay within the scratch of
+// the launcher that allocates nothing (they grow with every band, the blocks
+// only with the unoccupied ones).
+int direct_split(const DevProblem &p)
+{
+    const int njt = (p.ngpown + kBJ - 1) / kBJ, nun = p.nb - p.nv;
+    const double blocks = (double)(nun > 0 ? (nun + kNW - 1) / kNW : p.nv) * njt * ((p.nfreq + 3) / 4);
+    if (blocks > 4096) return 1;
+    const int chunks = (p.ncouls + kWave - 1) / kWave;
+    int best_gs = 1;
+    double best = 1e300;
+    for (int gs = 1; gs <= 16 && gs * 6 <= std::max(6, chunks) && (gs == 1 || blocks * gs <= 8192); ++gs) {
+        if (gs > 1 && kNoAllocHeadBytes + layout_for(p, gs).total > kNoAllocScratchBytes) break;
+        const double t = std::ceil(blocks * gs / kDirectSlots) / gs * (1.0 + 0.01 * gs);
+        if (t < best) best = t, best_gs = gs;
+    }
+    return best_gs;
+}
+
 DirectArgs make_args(const DevProblem &p, void *work)
 {
-    WorkLayout L = layout_for(p);
+    const int gs = direct_split(p);
+    const WorkLayout L = layout_for(p, gs);
     char *w = static_cast<char *>(work);
     DirectArgs a;
     a.aqsm = p.aqsm; a.aqsn = p.aqsn; a.ieps = p.ieps; a.wtilde = p.wtilde;
     a.idx = p.idx; a.vcoul = p.vcoul; a.wx = p.wx; a.wx_stride = p.wx_stride;
     a.nb = p.nb; a.nv = p.nv; a.ncouls = p.ncouls; a.ngpown = p.ngpown; a.nfreq = p.nfreq;
     a.njt = (p.ngpown + kBJ - 1) / kBJ;
-    a.gs = direct_split(p);
+    a.gs = gs;
     a.nt = a.njt * a.gs;
     a.nz = 1;
     a.occ_blocks = a.ach_blocks = 0;
@@ -651,7 +656,7 @@ hipError_t launch_reduce(const DirectArgs &a, cplx *out, const CompatOut &co, in
 
 }  // namespace
 
-size_t direct_workspace_bytes(const DevProblem &p) { return layout_for(p).total; }
+size_t direct_workspace_bytes(const DevProblem &p) { return layout_for(p, direct_split(p)).total; }
 
 hipError_t run_direct(const DevProblem &p, bool strict, void *work, const DevResults &res,
                       hipStream_t s, StageTimer *timer)

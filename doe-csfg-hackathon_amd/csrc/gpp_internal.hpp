@@ -86,6 +86,10 @@ inline int wx_has_negative(const double *wx, int n)
     return 0;
 }
 
+// The scratch of d_noFlagOCCSolver_noalloc per device: its index flag, then the
+// direct form's workspace.
+constexpr size_t kNoAllocScratchBytes = (size_t)16 << 20, kNoAllocHeadBytes = 256;
+
 // Bytes of device workspace the direct form needs for this problem.
 size_t direct_workspace_bytes(const DevProblem &p);
 
