@@ -54,7 +54,7 @@ struct DirectArgs {
     int njt, gs, nt;  // column tiles, G ranges, partials per (band, frequency): njt * gs
     int nz;           // frequency passes
     int wx_stride;    // 0: shared wx row; nfreq: band n1 reads wx[n1 * nfreq + iw]
-    int occ_blocks, ach_blocks;  // of the launch, before the unoccupied bands'
+    unsigned occ_blocks, ach_blocks, blocks;  // of the launch: before the unoccupied bands', and all
     double occ;
     cplx *part_ach;   // [nb][nt][nfreq]
     cplx *part_asx;   // [max(nv,1)][nt][nfreq]
@@ -130,7 +130,7 @@ DirectArgs make_args(const DevProblem &p, void *work)
     a.gs = gs;
     a.nt = a.njt * a.gs;
     a.nz = 1;
-    a.occ_blocks = a.ach_blocks = 0;
+    a.occ_blocks = a.ach_blocks = a.blocks = 0;
     a.occ = p.occ;
     a.part_ach = reinterpret_cast<cplx *>(w + L.part_ach);
     a.part_asx = reinterpret_cast<cplx *>(w + L.part_asx);
@@ -202,7 +202,7 @@ __device__ __forceinline__ void range_chunks(const DirectArgs &a, int ncouls, in
 // Unoccupied bands: block b of their share of the launch, frequencies
 // [iw0, iw0 + F).  lds: 4 kBJ kWave entries.
 template <int F, bool STRICT>
-__device__ __forceinline__ void unocc_block(const DirectArgs &a, int ncouls, int b, int iw0, cplx *lds)
+__device__ __forceinline__ void unocc_block(const DirectArgs &a, int ncouls, unsigned b, int iw0, cplx *lds)
 {
     constexpr int TILE = kBJ * kWave;  // (column, G-vector) positions per chunk
     static_assert(TILE <= kNW * kWave, "one position per staging thread");
@@ -211,10 +211,10 @@ __device__ __forceinline__ void unocc_block(const DirectArgs &a, int ncouls, int
 
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
     const int lane = threadIdx.x % kWave;
-    const int ngroups = (a.nb - a.nv + kNW - 1) / kNW;
-    const int n1 = a.nv + (b % ngroups) * kNW + wave;
+    const unsigned ngroups = (a.nb - a.nv + kNW - 1) / kNW;
+    const int n1 = a.nv + (int)(b % ngroups) * kNW + wave;
     const bool band_ok = n1 < a.nb;
-    const int jt = (b / ngroups) % a.njt, g = b / (ngroups * a.njt);
+    const int jt = (int)(b / ngroups % (unsigned)a.njt), g = (int)(b / ngroups / (unsigned)a.njt);
     const int j0 = jt * kBJ;
 
     // conj(aqsm[n1, igp(j)]) per column (mygpvar1, gppComplex.cpp:134).
@@ -339,13 +339,14 @@ __device__ __forceinline__ void unocc_block(const DirectArgs &a, int ncouls, int
 // one G range; waves jj and jj + 4 take column jj over the range's halves.  The
 // sums are combined half by half, then in column order, through LDS.
 template <int F>
-__device__ __forceinline__ void occ_block(const DirectArgs &a, int ncouls, int b, int iw0, cplx *lds)
+__device__ __forceinline__ void occ_block(const DirectArgs &a, int ncouls, unsigned b, int iw0, cplx *lds)
 {
     auto *s_sum = reinterpret_cast<cplx(*)[2][kBJ][F]>(lds);  // [ach, asx][half][column]
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
     const int lane = threadIdx.x % kWave;
     const int jj = wave % kBJ, half = wave / kBJ;
-    const int jt = b % a.njt, n1 = (b / a.njt) % a.nv, g = b / (a.njt * a.nv);
+    const unsigned njt = a.njt, nv = a.nv;
+    const int jt = (int)(b % njt), n1 = (int)(b / njt % nv), g = (int)(b / njt / nv);
     const int j = jt * kBJ + jj;
     const bool ok = j < a.ngpown;
 
@@ -408,7 +409,7 @@ __device__ __forceinline__ void occ_block(const DirectArgs &a, int ncouls, int b
 // One band kind's block `b` of frequency pass z: W frequencies, the last pass
 // as many as remain.
 template <int W, bool STRICT, bool OCC>
-__device__ __forceinline__ void direct_pass(const DirectArgs &a, int ncouls, int b, int z, cplx *lds)
+__device__ __forceinline__ void direct_pass(const DirectArgs &a, int ncouls, unsigned b, int z, cplx *lds)
 {
     const int iw0 = W * z, left = a.nfreq - iw0;
     const auto run = [&](auto f) {
@@ -428,18 +429,29 @@ __device__ __forceinline__ void direct_pass(const DirectArgs &a, int ncouls, int
     }
 }
 
-// 1-D grid: occ_blocks, ach_blocks, then the unoccupied bands'.
+// Grids of this many blocks a row: HIP takes at most 2^32 threads along one
+// dimension, and many bands and columns over few G-vectors make more.
+constexpr unsigned kGridRow = 1u << 20;
+__host__ inline dim3 grid_rows(unsigned blocks)
+{
+    return blocks <= kGridRow ? dim3(blocks) : dim3(kGridRow, (blocks + kGridRow - 1) / kGridRow);
+}
+__device__ __forceinline__ unsigned block_of_rows() { return blockIdx.y * gridDim.x + blockIdx.x; }
+
+// Blocks in row order (grid_rows): occ_blocks, ach_blocks, then the unoccupied
+// bands'.
 template <int W, bool STRICT>
 __global__ __launch_bounds__(kNW *kWave) __attribute__((amdgpu_waves_per_eu(4))) void k_direct(DirectArgs a)
 {
     int ncouls = a.ncouls;
     const StampStart stamp(a.stamp, ncouls);
     __shared__ cplx lds[4 * kBJ * kWave];
-    const int b = blockIdx.x;
+    const unsigned b = block_of_rows(), nz = a.nz;
+    if (b >= a.blocks) return;
     if (b < a.occ_blocks) {
-        direct_pass<W, STRICT, true>(a, ncouls, b / a.nz, b % a.nz, lds);
+        direct_pass<W, STRICT, true>(a, ncouls, b / nz, b % nz, lds);
     } else if (b < a.occ_blocks + a.ach_blocks) {
-        const int item = (b - a.occ_blocks) * kNW + threadIdx.x / kWave;  // band * kAchSplit + column group
+        const int item = (int)(b - a.occ_blocks) * kNW + threadIdx.x / kWave;  // band * kAchSplit + column group
         if (item < a.nb * kAchSplit) {
             const auto col = [&](int j) { return ach_col(a.ieps, a.idx, a.vcoul, ncouls, j); };
             const cplx s = achstemp_band(a.aqsm, a.aqsn, col, ncouls, a.ngpown, item / kAchSplit, item % kAchSplit,
@@ -447,8 +459,8 @@ __global__ __launch_bounds__(kNW *kWave) __attribute__((amdgpu_waves_per_eu(4)))
             if (threadIdx.x % kWave == 0) a.part_achs[item] = s;
         }
     } else {
-        const int u = b - a.occ_blocks - a.ach_blocks;
-        direct_pass<W, STRICT, false>(a, ncouls, u / a.nz, u % a.nz, lds);
+        const unsigned u = b - a.occ_blocks - a.ach_blocks;
+        direct_pass<W, STRICT, false>(a, ncouls, u / nz, u % nz, lds);
     }
     stamp.store();
 }
@@ -503,9 +515,9 @@ hipError_t launch_ach(const DirectArgs &a, hipStream_t s)
 __global__ __launch_bounds__(kReduceThreads) void k_reduce_bands(DirectArgs a, int n1_begin, int n1_end)
 {
     stamp_start(a.stamp);
-    const int pair = blockIdx.x * (kReduceThreads / kWave) + threadIdx.x / kWave;
-    const int n1 = n1_begin + pair / a.nfreq, iw = pair % a.nfreq, lane = threadIdx.x % kWave;
-    if (n1 >= n1_end) return;
+    const long long pair = (long long)block_of_rows() * (kReduceThreads / kWave) + threadIdx.x / kWave;
+    if (pair >= (long long)(n1_end - n1_begin) * a.nfreq) return;
+    const int n1 = n1_begin + (int)(pair / a.nfreq), iw = (int)(pair % a.nfreq), lane = threadIdx.x % kWave;
     cplx s = czero(), x = czero();
     for (int t = lane; t < a.nt; t += kWave) {
         const size_t o = ((size_t)n1 * a.nt + t) * a.nfreq + iw;
@@ -607,13 +619,16 @@ hipError_t launch_direct(DirectArgs &a, bool strict, bool occ, bool achs, bool u
 {
     const int w = std::min(a.nfreq, pass_width(strict));
     a.nz = (a.nfreq + w - 1) / w;
-    a.occ_blocks = occ ? a.nt * a.nv * a.nz : 0;
-    a.ach_blocks = achs ? (a.nb * kAchSplit + kNW - 1) / kNW : 0;
     const int nun = unocc ? a.nb - a.nv : 0;
-    const unsigned blocks =
-        (unsigned)a.occ_blocks + (unsigned)a.ach_blocks + (unsigned)((nun + kNW - 1) / kNW) * (unsigned)(a.nt * a.nz);
-    if (blocks == 0) return hipSuccess;
-    const dim3 grid(blocks), block(kNW * kWave);
+    const unsigned long long nocc = occ ? (unsigned long long)a.nt * a.nv * a.nz : 0;
+    const unsigned long long nach = achs ? ((unsigned long long)a.nb * kAchSplit + kNW - 1) / kNW : 0;
+    const unsigned long long all = nocc + nach + (unsigned long long)((nun + kNW - 1) / kNW) * a.nt * a.nz;
+    if (all == 0) return hipSuccess;
+    if (all > 0x7fffffffull) return hipErrorInvalidConfiguration;
+    a.occ_blocks = (unsigned)nocc;
+    a.ach_blocks = (unsigned)nach;
+    a.blocks = (unsigned)all;
+    const dim3 grid = grid_rows(a.blocks), block(kNW * kWave);
     if (strict)
         switch (w) {
         case 1: hipLaunchKernelGGL((k_direct<1, true>), grid, block, 0, s, a); break;
@@ -640,8 +655,8 @@ hipError_t launch_reduce(const DirectArgs &a, cplx *out, const CompatOut &co, in
     if (pairs > 0) {
         DirectArgs b = a;
         b.end = nullptr;
-        hipLaunchKernelGGL(k_reduce_bands, dim3((unsigned)((pairs + 3) / 4)), dim3(kReduceThreads), 0, s, b, n1_begin,
-                           n1_end);
+        hipLaunchKernelGGL(k_reduce_bands, grid_rows((unsigned)((pairs + 3) / 4)), dim3(kReduceThreads), 0, s, b,
+                           n1_begin, n1_end);
     }
     hipLaunchKernelGGL(k_reduce_final, dim3(a.nfreq + 1), dim3(kReduceThreads), 0, s, f, out, co, n1_begin, n1_end,
                        with_achs);
