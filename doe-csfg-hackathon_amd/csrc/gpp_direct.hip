@@ -294,7 +294,9 @@ __device__ __forceinline__ void unocc_block(const DirectArgs &a, int ncouls, uns
     // column order (gppComplex.cpp:374, :379).  The wave's sums by the xor
     // butterfly of wave_sum (the same additions), each step on the half of the
     // values this lane goes on with: after three steps lane l holds F of its
-    // column's 2 F parts (10 F exchanges of doubles instead of 48 F).
+    // column's 2 F parts (10 F exchanges of doubles instead of 48 F).  The
+    // halves are constants of each step's code: with a loop over them the
+    // compiler left the passes of two to index v at run time (890 selects).
     static_assert(kBJ == 4, "two steps split the columns, one the parts");
     double v[kBJ * 2 * F];
 #pragma unroll
@@ -304,16 +306,18 @@ __device__ __forceinline__ void unocc_block(const DirectArgs &a, int ncouls, uns
             v[(jj * F + f) * 2] = acc[jj][f].re;
             v[(jj * F + f) * 2 + 1] = acc[jj][f].im;
         }
-    int n = kBJ * F;  // half of the values held
-#pragma unroll
-    for (int m = 1; m <= 4; m <<= 1, n /= 2) {
+    const auto halve = [&](auto half, int m) {
+        constexpr int N = decltype(half)::value;
         const bool up = lane & m;
 #pragma unroll
-        for (int i = 0; i < n; ++i) {
-            const double keep = up ? v[n + i] : v[i], give = up ? v[i] : v[n + i];
+        for (int i = 0; i < N; ++i) {
+            const double keep = up ? v[N + i] : v[i], give = up ? v[i] : v[N + i];
             v[i] = keep + __shfl_xor(give, m, kWave);
         }
-    }
+    };
+    halve(std::integral_constant<int, kBJ * F>(), 1);
+    halve(std::integral_constant<int, kBJ * F / 2>(), 2);
+    halve(std::integral_constant<int, kBJ * F / 4>(), 4);
     const int col = 2 * (lane & 1) + ((lane >> 1) & 1);  // this lane's column
     const double vc = a.vcoul[igp_of(a.idx, min(j0 + col, a.ngpown - 1), ncouls)];
     double s[F];

@@ -1,0 +1,27 @@
+"""Direct forms: what a pass of frequencies costs.  The device clock's stage
+times of one shape at several frequency counts, least of several evaluations,
+against each other."""
+import pytest
+
+import gpp_inputs
+from test_gpu_parity import problem_of
+
+pytestmark = pytest.mark.gpu
+
+
+def stage_ms(ctx, arrs, nv, nf, form):
+    arrs["wx_array"] = gpp_inputs.seeded_inputs(1, 4, 1, nfreq=nf, seed=0, dw=0.3)["wx_array"]
+    ctx.upload(problem_of(arrs, nv), arrs)
+    best = 1e9
+    for _ in range(12):
+        ctx.sigma(form)
+        best = min(best, sum(v for k, v in ctx.last_timing().items() if k.startswith("direct_unoccupied")))
+    return best
+
+
+@pytest.mark.parametrize("form", ["direct", "direct-strict"])
+def test_two_frequencies_cost_less_than_three(ctx, form):
+    """A pass of two runs two thirds of the updates of one of three."""
+    arrs = gpp_inputs.seeded_inputs(200, 3000, 150, seed=44)
+    two, three = stage_ms(ctx, arrs, 3, 2, form), stage_ms(ctx, arrs, 3, 3, form)
+    assert two < three, (two, three)
