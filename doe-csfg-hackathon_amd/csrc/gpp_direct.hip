@@ -443,17 +443,22 @@ __host__ inline dim3 grid_rows(unsigned blocks)
 __device__ __forceinline__ unsigned block_of_rows() { return blockIdx.y * gridDim.x + blockIdx.x; }
 
 // Blocks in row order (grid_rows): occ_blocks, ach_blocks, then the unoccupied
-// bands'.
+// bands'.  Each kind's frequency passes one after the other, not by turns: the
+// dispatcher deals blocks round robin to eight XCDs, and two passes of unequal
+// width by turns gave four of them all the wide ones (us, 200/3/3000/150: five
+// frequencies 511 by turns, 409 so; strict, in passes of three, four
+// frequencies 811, 617).
 template <int W, bool STRICT>
 __global__ __launch_bounds__(kNW *kWave) __attribute__((amdgpu_waves_per_eu(4))) void k_direct(DirectArgs a)
 {
     int ncouls = a.ncouls;
     const StampStart stamp(a.stamp, ncouls);
     __shared__ cplx lds[4 * kBJ * kWave];
-    const unsigned b = block_of_rows(), nz = a.nz;
+    const unsigned b = block_of_rows();
     if (b >= a.blocks) return;
     if (b < a.occ_blocks) {
-        direct_pass<W, STRICT, true>(a, ncouls, b / nz, b % nz, lds);
+        const unsigned pass = a.occ_blocks / (unsigned)a.nz;
+        direct_pass<W, STRICT, true>(a, ncouls, b % pass, b / pass, lds);
     } else if (b < a.occ_blocks + a.ach_blocks) {
         const int item = (int)(b - a.occ_blocks) * kNW + threadIdx.x / kWave;  // band * kAchSplit + column group
         if (item < a.nb * kAchSplit) {
@@ -463,8 +468,8 @@ __global__ __launch_bounds__(kNW *kWave) __attribute__((amdgpu_waves_per_eu(4)))
             if (threadIdx.x % kWave == 0) a.part_achs[item] = s;
         }
     } else {
-        const unsigned u = b - a.occ_blocks - a.ach_blocks;
-        direct_pass<W, STRICT, false>(a, ncouls, u / nz, u % nz, lds);
+        const unsigned before = a.occ_blocks + a.ach_blocks, u = b - before, pass = (a.blocks - before) / (unsigned)a.nz;
+        direct_pass<W, STRICT, false>(a, ncouls, u % pass, u / pass, lds);
     }
     stamp.store();
 }

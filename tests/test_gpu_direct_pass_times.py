@@ -25,3 +25,13 @@ def test_two_frequencies_cost_less_than_three(ctx, form):
     arrs = gpp_inputs.seeded_inputs(200, 3000, 150, seed=44)
     two, three = stage_ms(ctx, arrs, 3, 2, form), stage_ms(ctx, arrs, 3, 3, form)
     assert two < three, (two, three)
+
+
+@pytest.mark.parametrize("form,few,many", [("direct", 5, 8), ("direct-strict", 4, 6), ("direct-strict", 5, 8)])
+def test_a_narrow_last_pass_costs_less_than_a_whole_one(ctx, form, few, many):
+    """The work is few / many of it (at most 0.67) and the pass count the same
+    or less; 0.9 leaves room for what a pass costs whatever its width.  Wide and
+    narrow passes dealt out unevenly over the XCDs cost what two wide ones do."""
+    arrs = gpp_inputs.seeded_inputs(200, 3000, 150, seed=45)
+    a, b = stage_ms(ctx, arrs, 3, few, form), stage_ms(ctx, arrs, 3, many, form)
+    assert a < 0.9 * b, (a, b)
