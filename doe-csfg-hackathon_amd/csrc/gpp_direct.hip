@@ -73,10 +73,7 @@ struct WorkLayout {
 
 __host__ inline size_t align256(size_t x) { return (x + 255) & ~(size_t)255; }
 
-// Frequencies per pass: four, in the strict form three (its kernel of four
-// spills 40 registers beside the occupied bands' code: 541 against 499 us at
-// 131/5/2477/123 with 7 frequencies).
-constexpr int pass_width(bool strict) { return strict ? 3 : 4; }
+constexpr int kPassWidth = 4;  // frequencies per pass, the last one what remains
 
 // The workspace with gs G ranges.
 WorkLayout layout_for(const DevProblem &p, int gs)
@@ -410,27 +407,25 @@ __device__ __forceinline__ void occ_block(const DirectArgs &a, int ncouls, unsig
     }
 }
 
-// One band kind's block `b` of frequency pass z: W frequencies, the last pass
-// as many as remain.
-template <int W, bool STRICT, bool OCC>
+// One band kind's block `b` of frequency pass z: W frequencies, with R > 0 the
+// last pass R.
+template <int W, int R, bool STRICT, bool OCC>
 __device__ __forceinline__ void direct_pass(const DirectArgs &a, int ncouls, unsigned b, int z, cplx *lds)
 {
-    const int iw0 = W * z, left = a.nfreq - iw0;
+    const int iw0 = W * z;
     const auto run = [&](auto f) {
         if constexpr (OCC)
             occ_block<decltype(f)::value>(a, ncouls, b, iw0, lds);
         else
             unocc_block<decltype(f)::value, STRICT>(a, ncouls, b, iw0, lds);
     };
-    if (left >= W) {
-        run(std::integral_constant<int, W>());
-    } else if (W > 3 && left == 3) {
-        run(std::integral_constant<int, (W > 3 ? 3 : W)>());
-    } else if (W > 2 && left == 2) {
-        run(std::integral_constant<int, (W > 2 ? 2 : W)>());
-    } else if (W > 1) {
-        run(std::integral_constant<int, 1>());
+    if constexpr (R > 0) {
+        if (z == a.nz - 1) {
+            run(std::integral_constant<int, R>());
+            return;
+        }
     }
+    run(std::integral_constant<int, W>());
 }
 
 // Grids of this many blocks a row: HIP takes at most 2^32 threads along one
@@ -446,9 +441,12 @@ __device__ __forceinline__ unsigned block_of_rows() { return blockIdx.y * gridDi
 // bands'.  Each kind's frequency passes one after the other, not by turns: the
 // dispatcher deals blocks round robin to eight XCDs, and two passes of unequal
 // width by turns gave four of them all the wide ones (us, 200/3/3000/150: five
-// frequencies 511 by turns, 409 so; strict, in passes of three, four
-// frequencies 811, 617).
-template <int W, bool STRICT>
+// frequencies 511 by turns, 409 so).
+// A kernel for each pair of widths (W, the last pass R; 0: W): one with every
+// width took 4 registers more than it has, the strict one 29, and ran the
+// strict form in passes of three (us, 512/2/16384/819 strict 4 frequencies
+// 37600, with a kernel of its own 32200; 200/3/3000/150 direct 2 242, 216).
+template <int W, int R, bool STRICT>
 __global__ __launch_bounds__(kNW *kWave) __attribute__((amdgpu_waves_per_eu(4))) void k_direct(DirectArgs a)
 {
     int ncouls = a.ncouls;
@@ -458,7 +456,7 @@ __global__ __launch_bounds__(kNW *kWave) __attribute__((amdgpu_waves_per_eu(4)))
     if (b >= a.blocks) return;
     if (b < a.occ_blocks) {
         const unsigned pass = a.occ_blocks / (unsigned)a.nz;
-        direct_pass<W, STRICT, true>(a, ncouls, b % pass, b / pass, lds);
+        direct_pass<W, R, STRICT, true>(a, ncouls, b % pass, b / pass, lds);
     } else if (b < a.occ_blocks + a.ach_blocks) {
         const int item = (int)(b - a.occ_blocks) * kNW + threadIdx.x / kWave;  // band * kAchSplit + column group
         if (item < a.nb * kAchSplit) {
@@ -469,7 +467,7 @@ __global__ __launch_bounds__(kNW *kWave) __attribute__((amdgpu_waves_per_eu(4)))
         }
     } else {
         const unsigned before = a.occ_blocks + a.ach_blocks, u = b - before, pass = (a.blocks - before) / (unsigned)a.nz;
-        direct_pass<W, STRICT, false>(a, ncouls, u % pass, u / pass, lds);
+        direct_pass<W, R, STRICT, false>(a, ncouls, u % pass, u / pass, lds);
     }
     stamp.store();
 }
@@ -623,11 +621,26 @@ __global__ __launch_bounds__(1024) void k_check_index_once(const int32_t *idx, i
     }
 }
 
+// The kernel of the problem's pass widths: one pass of up to three frequencies,
+// or passes of four and what remains.
+template <bool STRICT>
+void launch_direct_widths(const DirectArgs &a, dim3 grid, dim3 block, hipStream_t s)
+{
+    switch (a.nfreq < 4 ? a.nfreq : 4 + a.nfreq % 4) {
+    case 1: hipLaunchKernelGGL((k_direct<1, 0, STRICT>), grid, block, 0, s, a); break;
+    case 2: hipLaunchKernelGGL((k_direct<2, 0, STRICT>), grid, block, 0, s, a); break;
+    case 3: hipLaunchKernelGGL((k_direct<3, 0, STRICT>), grid, block, 0, s, a); break;
+    case 4: hipLaunchKernelGGL((k_direct<4, 0, STRICT>), grid, block, 0, s, a); break;
+    case 5: hipLaunchKernelGGL((k_direct<4, 1, STRICT>), grid, block, 0, s, a); break;
+    case 6: hipLaunchKernelGGL((k_direct<4, 2, STRICT>), grid, block, 0, s, a); break;
+    default: hipLaunchKernelGGL((k_direct<4, 3, STRICT>), grid, block, 0, s, a); break;
+    }
+}
+
 // The bands' blocks (occ, unocc) and the achstemp partials (achs) in one launch.
 hipError_t launch_direct(DirectArgs &a, bool strict, bool occ, bool achs, bool unocc, hipStream_t s)
 {
-    const int w = std::min(a.nfreq, pass_width(strict));
-    a.nz = (a.nfreq + w - 1) / w;
+    a.nz = (a.nfreq + kPassWidth - 1) / kPassWidth;
     const int nun = unocc ? a.nb - a.nv : 0;
     const unsigned long long nocc = occ ? (unsigned long long)a.nt * a.nv * a.nz : 0;
     const unsigned long long nach = achs ? ((unsigned long long)a.nb * kAchSplit + kNW - 1) / kNW : 0;
@@ -639,18 +652,9 @@ hipError_t launch_direct(DirectArgs &a, bool strict, bool occ, bool achs, bool u
     a.blocks = (unsigned)all;
     const dim3 grid = grid_rows(a.blocks), block(kNW * kWave);
     if (strict)
-        switch (w) {
-        case 1: hipLaunchKernelGGL((k_direct<1, true>), grid, block, 0, s, a); break;
-        case 2: hipLaunchKernelGGL((k_direct<2, true>), grid, block, 0, s, a); break;
-        default: hipLaunchKernelGGL((k_direct<3, true>), grid, block, 0, s, a); break;
-        }
+        launch_direct_widths<true>(a, grid, block, s);
     else
-        switch (w) {
-        case 1: hipLaunchKernelGGL((k_direct<1, false>), grid, block, 0, s, a); break;
-        case 2: hipLaunchKernelGGL((k_direct<2, false>), grid, block, 0, s, a); break;
-        case 3: hipLaunchKernelGGL((k_direct<3, false>), grid, block, 0, s, a); break;
-        default: hipLaunchKernelGGL((k_direct<4, false>), grid, block, 0, s, a); break;
-        }
+        launch_direct_widths<false>(a, grid, block, s);
     return hipGetLastError();
 }
 

@@ -35,3 +35,12 @@ def test_a_narrow_last_pass_costs_less_than_a_whole_one(ctx, form, few, many):
     arrs = gpp_inputs.seeded_inputs(200, 3000, 150, seed=45)
     a, b = stage_ms(ctx, arrs, 3, few, form), stage_ms(ctx, arrs, 3, many, form)
     assert a < 0.9 * b, (a, b)
+
+
+@pytest.mark.parametrize("form", ["direct", "direct-strict"])
+def test_four_frequencies_are_one_pass(ctx, form):
+    """A pass of four loads and reduces what one of three does, so it takes at
+    most the time per update of one of three: 4 / 3 in all."""
+    arrs = gpp_inputs.seeded_inputs(200, 3000, 150, seed=46)
+    three, four = stage_ms(ctx, arrs, 3, 3, form), stage_ms(ctx, arrs, 3, 4, form)
+    assert four < 4 / 3 * three, (three, four)
