@@ -703,7 +703,14 @@ hipError_t run_direct_part(const DevProblem &p, int which, void *work, const Com
 {
     DirectArgs a = make_args(p, work);
     a.stamp = Stamp{};
-    GPP_TRY(launch_direct(a, false, which == 0, which == 2, which == 1, s));
+    // achstemp alone: with many columns a band's waves form many entries one
+    // after the other, with no bands' work to hide them, and a launch that forms
+    // the entries first is faster.  d_reduce_achstemp, us, one launch / as the
+    // factored forms do it: 24 bands x 20000 columns 136 / 79, 100 x 2600 32 /
+    // 26, 1536 x 3276 126 / 99, 512 x 1638 40 / 39, 512 x 1024 35 / 35, 1536 x
+    // 200 34 / 35, 4000 x 100 48 / 59.
+    const bool achs = which == 2, entries_first = achs && p.ngpown >= 1024;
+    GPP_TRY(entries_first ? launch_ach(a, s) : launch_direct(a, false, which == 0, achs, which == 1, s));
     if (which == 0) return launch_reduce(a, nullptr, co, 0, p.nv, 0, s);
     if (which == 1) return launch_reduce(a, nullptr, co, p.nv, p.nb, 0, s);
     return launch_reduce(a, nullptr, co, 0, 0, 1, s);
