@@ -503,12 +503,16 @@ __global__ __launch_bounds__(256) void k_ach_cols(DirectArgs a)
 
 // The (band, column group) partials (and the Bg gather when a.bg is set), after
 // the columns' entries where forming them once saves more than their launch
-// costs: at 512 bands x 1638 columns the two launches take 33 us and the one
-// takes 50, at 512 x 40 the one saves a launch of 4-5 us.
+// costs.  Without it each of a band's 256 lanes forms every 256th entry, one
+// after the other, so the number of columns decides, however many bands there
+// are.  Gather stage, us, one launch / two: 512 bands x 40 columns 3.9 / 6.3,
+// 512 x 409 9.0 / 12.0, 512 x 1638 33.0 / 33.9, 1536 x 800 40.6 / 43.6, 100 x
+// 2600 13.6 / 15.0, 1536 x 3276 162.8 / 158.4, 100 x 5000 27.1 / 25.8, 24 x
+// 8000 30.9 / 29.1.
 hipError_t launch_ach(const DirectArgs &a, hipStream_t s)
 {
     const dim3 grid((a.nb * kAchSplit + kAchWaves - 1) / kAchWaves), block(kAchWaves * kWave);
-    if ((long long)a.nb * a.ngpown > (1 << 18)) {
+    if (a.ngpown >= 3072) {
         hipLaunchKernelGGL(k_ach_cols, dim3((a.ngpown + 255) / 256), dim3(256), 0, s, a);
         hipLaunchKernelGGL((k_achstemp<true>), grid, block, 0, s, a);
     } else {
@@ -703,14 +707,13 @@ hipError_t run_direct_part(const DevProblem &p, int which, void *work, const Com
 {
     DirectArgs a = make_args(p, work);
     a.stamp = Stamp{};
-    // achstemp alone: with many columns a band's waves form many entries one
-    // after the other, with no bands' work to hide them, and a launch that forms
-    // the entries first is faster.  d_reduce_achstemp, us, one launch / as the
-    // factored forms do it: 24 bands x 20000 columns 136 / 79, 100 x 2600 32 /
-    // 26, 1536 x 3276 126 / 99, 512 x 1638 40 / 39, 512 x 1024 35 / 35, 1536 x
-    // 200 34 / 35, 4000 x 100 48 / 59.
-    const bool achs = which == 2, entries_first = achs && p.ngpown >= 1024;
-    GPP_TRY(entries_first ? launch_ach(a, s) : launch_direct(a, false, which == 0, achs, which == 1, s));
+    // achstemp alone, with no bands' work to hide it: as the factored forms do it
+    // where the columns are many (blocks of one wave, the entries first from 3072
+    // columns up).  d_reduce_achstemp, us, k_direct / so: 24 bands x 20000
+    // columns 136 / 79, 100 x 2600 32 / 26, 1536 x 3276 126 / 99, 512 x 1638 40 /
+    // 37, 512 x 1024 35 / 33, 1536 x 200 34 / 34, 4000 x 100 48 / 58.
+    const bool achs = which == 2, alone = achs && p.ngpown >= 1024;
+    GPP_TRY(alone ? launch_ach(a, s) : launch_direct(a, false, which == 0, achs, which == 1, s));
     if (which == 0) return launch_reduce(a, nullptr, co, 0, p.nv, 0, s);
     if (which == 1) return launch_reduce(a, nullptr, co, p.nv, p.nb, 0, s);
     return launch_reduce(a, nullptr, co, 0, 0, 1, s);
