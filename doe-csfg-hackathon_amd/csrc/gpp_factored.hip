@@ -817,7 +817,8 @@ BucketLayout bucket_layout(const DevProblem &p, const GramKind &k, const BucketP
     BucketLayout L;
     const int nbk = (int)bp.slot.size();
     const size_t mu_bytes = sizeof(cplx) * (size_t)p.ngpown * p.ncouls;
-    L.group = (int)std::max<size_t>(1, std::min<size_t>(std::min(nbk, 4096), kBucketMuBytes / mu_bytes));
+    // with the fused reduce the buckets run one after the other
+    L.group = k.fuse ? 1 : (int)std::max<size_t>(1, std::min<size_t>(std::min(nbk, 4096), kBucketMuBytes / mu_bytes));
     L.nsplit = (p.ncouls + k.red_chunk - 1) / k.red_chunk;
     // G ranges of the reduce over the bare buckets: whole steps of a block,
     // about 2048 blocks
