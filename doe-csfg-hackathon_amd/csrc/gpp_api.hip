@@ -203,6 +203,7 @@ struct gpp_ctx {
     int fuse_reduce = 0;
     int num_cus = 256;
     int max_buckets = 32;
+    size_t bucket_mu = gpp::GramKind().bucket_mu;
     // band-dependent frequencies (gpp_set_band_frequencies)
     bool per_band = false;
     DevBuf wxb;                     // [nb][nfreq]
@@ -267,6 +268,7 @@ gpp::GramKind gram_kind(const gpp_ctx *ctx, gpp_form form)
     k.red_fc = ctx->red_fc;
     k.red_fpb = ctx->red_fpb;
     k.fuse = ctx->fuse_reduce != 0;
+    k.bucket_mu = ctx->bucket_mu;
     return k;
 }
 
@@ -905,6 +907,10 @@ gpp_status gpp_ctx_set_option(gpp_ctx *ctx, gpp_option option, int value)
     default: return fail(GPP_ERR_INVALID_ARGUMENT, "unknown option %d", (int)option);
     }
 }
+
+// Not part of the interface: the tests reach evaluations of several rounds of
+// band groups with it.
+void gpp_test_bucket_mu(gpp_ctx *ctx, size_t bytes) { ctx->bucket_mu = bytes; }
 
 gpp_status gpp_ctx_get_option(const gpp_ctx *ctx, gpp_option option, int *value)
 {

@@ -719,7 +719,7 @@ hipError_t run_factored(const DevProblem &p, GramKind kind, void *work, const De
 // the bands already lie so).  One launch forms every bucket's Mu, one more
 // pass adds up the pole terms of all buckets without occupied bands
 // (pole_reduce_bare); a bucket with occupied bands runs the reduce of the
-// plain form.  The Mu of at most kBucketMuBytes of buckets are held at a time.
+// plain form.  The Mu of GramKind::bucket_mu bytes of buckets are held at a time.
 // 512/8/8192/409/3 in 8 buckets: 704 us with a factored evaluation per
 // bucket and both arrays permuted, 368 so (Gram 215 of them, with 429 MB of Mu
 // to store; the reduces 56 and 84, the latter at 5.7 TB/s).
@@ -777,8 +777,6 @@ void launch_reduce_bare(const BareArgs &a, hipStream_t s)
     }
 }
 
-constexpr size_t kBucketMuBytes = (size_t)4 << 30;
-
 // How a slot's stage 3 runs: fused with its Gram product, with the plain
 // form's reduce, or together with the other buckets without occupied bands.
 // With GPP_OPT_FUSED_REDUCE no bucket runs together with others.
@@ -818,7 +816,7 @@ BucketLayout bucket_layout(const DevProblem &p, const GramKind &k, const BucketP
     const int nbk = (int)bp.slot.size();
     const size_t mu_bytes = sizeof(cplx) * (size_t)p.ngpown * p.ncouls;
     // with the fused reduce the buckets run one after the other
-    L.group = k.fuse ? 1 : (int)std::max<size_t>(1, std::min<size_t>(std::min(nbk, 4096), kBucketMuBytes / mu_bytes));
+    L.group = k.fuse ? 1 : (int)std::max<size_t>(1, std::min<size_t>(std::min(nbk, 4096), k.bucket_mu / mu_bytes));
     L.nsplit = (p.ncouls + k.red_chunk - 1) / k.red_chunk;
     // G ranges of the reduce over the bare buckets: whole steps of a block,
     // about 2048 blocks

@@ -147,6 +147,7 @@ struct GramKind {
     int red_fpb = 0;       // frequencies per pole-reduce block (0: all, passes looped in the block)
     bool acht = false;     // also produce acht_n1_loc (a second product, R * aqsn^T)
     bool fuse = false;     // pole reduce in the FP64 Gram epilogue where it applies (no Mu workspace)
+    size_t bucket_mu = (size_t)4 << 30;  // band-dependent frequencies: bytes of Mu held at a time (at least one group's)
 };
 constexpr int kGramTiles = 4;
 
