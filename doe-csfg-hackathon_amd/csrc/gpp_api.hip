@@ -121,8 +121,12 @@ hipError_t Workspace::reserve(size_t need)
     ptr = nullptr;
     bytes = 0;
     hipError_t e = hipMalloc(&ptr, need ? need : 256);
-    if (e == hipSuccess) bytes = need;
-    else ptr = nullptr;
+    if (e == hipSuccess) {
+        bytes = need;
+    } else {
+        ptr = nullptr;
+        (void)hipGetLastError();  // reported here, not by the next launch
+    }
     return e;
 }
 
@@ -203,7 +207,7 @@ struct gpp_ctx {
     int fuse_reduce = 0;
     int num_cus = 256;
     int max_buckets = 32;
-    size_t bucket_mu = gpp::GramKind().bucket_mu;
+    size_t bucket_mu = gpp::GramKind().bucket_mu;  // 0 once the groups did not fit together
     // band-dependent frequencies (gpp_set_band_frequencies)
     bool per_band = false;
     DevBuf wxb;                     // [nb][nfreq]
@@ -675,6 +679,7 @@ gpp_status gpp_set_band_frequencies(gpp_ctx *ctx, const double *wx_bands)
     HIP_OR_FAIL(hipStreamSynchronize(ctx->stream), "wx_bands synchronize");
     plan.dev = static_cast<const int32_t *>(ctx->btab.ptr);
     ctx->bplan = std::move(plan);
+    ctx->bucket_mu = gpp::GramKind().bucket_mu;
     ctx->per_band = true;
     return GPP_OK;
 }
@@ -780,13 +785,18 @@ gpp_status sigma_enqueue(gpp_ctx *ctx, gpp_form form, bool acht)
         need = bucketed ? gpp::bucketed_workspace_bytes(dp, kind, ctx->bplan) : gpp::factored_workspace_bytes(dp, kind);
     }
     if (need == 0) return fail(GPP_ERR_UNSUPPORTED, "form %d is not available for this problem", (int)form);
-    HIP_OR_FAIL(ctx->work.reserve(need), "workspace allocation");
+    hipError_t e = ctx->work.reserve(need);
+    if (e == hipErrorOutOfMemory && bucketed && kind.bucket_mu > 0) {
+        // the groups' products one at a time, from here on
+        ctx->bucket_mu = kind.bucket_mu = 0;
+        e = ctx->work.reserve(gpp::bucketed_workspace_bytes(dp, kind, ctx->bplan));
+    }
+    HIP_OR_FAIL(e, "workspace allocation");
     gpp::DevResults res;
     res.nfreq = dp.nfreq;
     res.nb = dp.nb;
     HIP_OR_FAIL(ctx->results.ensure(sizeof(cplx) * res.count()), "results allocation");
     res.base = static_cast<cplx *>(ctx->results.ptr);
-    hipError_t e;
     if (direct)
         e = gpp::run_direct(dp, form == GPP_FORM_DIRECT_STRICT, ctx->work.ptr, res, ctx->stream, &ctx->timer);
     else if (bucketed)
