@@ -13,6 +13,7 @@
 #include <errno.h>
 #include <stdarg.h>
 #include <stdio.h>
+#include <unistd.h>
 #include <string.h>
 #include <vector>
 
@@ -137,12 +138,14 @@ void Workspace::release()
     bytes = 0;
 }
 
-hipError_t StageTimer::init(int device)
+hipError_t StageTimer::init(int device, hipStream_t s)
 {
     hipError_t e = hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, device);
     if (e != hipSuccess) return e;
     if (khz <= 0) return hipErrorInvalidValue;
-    return hipMalloc(reinterpret_cast<void **>(&dev), sizeof(unsigned long long) * kRing * (kMax + 1));
+    const size_t bytes = sizeof(unsigned long long) * kRing * kRow;
+    e = hipMalloc(reinterpret_cast<void **>(&dev), bytes);
+    return e == hipSuccess ? hipMemsetAsync(dev, 0, bytes, s) : e;
 }
 
 void StageTimer::destroy()
@@ -156,6 +159,7 @@ void StageTimer::begin()
     if (filled > 0) cur = (cur + 1) % kRing;
     if (filled < kRing) ++filled;
     slot[cur].n = 0;
+    slot[cur].begin = slot[cur].end = counted ? ++evaluations << 32 : 0;
 }
 
 Stamp StageTimer::stage(const char *nm)
@@ -163,17 +167,29 @@ Stamp StageTimer::stage(const char *nm)
     Slot &sl = slot[cur];
     if (!dev || sl.n >= kMax) return Stamp{};
     sl.name[sl.n] = nm;
-    const Stamp st{dev + cur * (kMax + 1) + sl.n, sl.n == 0 ? kMax : 0};
+    const Stamp st{dev + cur * kRow + sl.n, sl.n == 0 ? kRow - 1 : 0, sl.begin};
     ++sl.n;
     return st;
 }
 
-hipError_t StageTimer::read(int k, double *total, double (&stage_ms)[kMax]) const
+StampEnd StageTimer::end(unsigned blocks)
+{
+    if (!dev) return StampEnd{};
+    Slot &sl = slot[cur];
+    unsigned long long *const row = dev + cur * kRow;
+    if (!sl.begin) return StampEnd{row + sl.n, nullptr};
+    sl.end = sl.begin + blocks;
+    return StampEnd{row + sl.n, row + kRow - 1};
+}
+
+hipError_t StageTimer::read(int k, hipStream_t via, double *total, double (&stage_ms)[kMax], bool *finished) const
 {
     const int i = (cur - k + kRing) % kRing, n = slot[i].n;
-    unsigned long long t[kMax + 1];
-    hipError_t e = hipMemcpy(t, dev + i * (kMax + 1), sizeof(unsigned long long) * (n + 1), hipMemcpyDeviceToHost);
+    unsigned long long t[kRow];
+    hipError_t e = hipMemcpyAsync(t, dev + i * kRow, sizeof(t), hipMemcpyDeviceToHost, via);
+    if (e == hipSuccess) e = hipStreamSynchronize(via);
     if (e != hipSuccess) return e;
+    *finished = !slot[i].begin || (slot[i].end > slot[i].begin && t[kRow - 1] == slot[i].end);
     for (int q = 0; q < n; ++q) stage_ms[q] = (double)(t[q + 1] - t[q]) / khz;
     *total = (double)(t[n] - t[0]) / khz;
     return hipSuccess;
@@ -330,7 +346,7 @@ gpp_status gpp_ctx_create(gpp_ctx **out, int device)
     e = hipSetDevice(device);
     if (e == hipSuccess) e = hipStreamCreateWithFlags(&ctx->own_stream, hipStreamNonBlocking);
     ctx->stream = ctx->own_stream;
-    if (e == hipSuccess) e = ctx->timer.init(device);
+    if (e == hipSuccess) e = ctx->timer.init(device, ctx->own_stream);
     if (e != hipSuccess) {
         gpp_ctx_destroy(ctx);
         return fail_hip(e, "context setup");
@@ -785,6 +801,7 @@ gpp_status sigma_enqueue(gpp_ctx *ctx, gpp_form form, bool acht)
         need = bucketed ? gpp::bucketed_workspace_bytes(dp, kind, ctx->bplan) : gpp::factored_workspace_bytes(dp, kind);
     }
     if (need == 0) return fail(GPP_ERR_UNSUPPORTED, "form %d is not available for this problem", (int)form);
+    ctx->timer.counted = ctx->stream != ctx->own_stream;
     hipError_t e = ctx->work.reserve(need);
     if (e == hipErrorOutOfMemory && bucketed && kind.bucket_mu > 0) {
         // the groups' products one at a time, from here on
@@ -973,7 +990,8 @@ gpp_status gpp_ctx_autotune(gpp_ctx *ctx, gpp_form form)
             HIP_OR_FAIL(hipStreamSynchronize(ctx->stream), "autotune synchronize");
             if (rep == 0) continue;  // warm-up
             double g_ms = 0.0, r_ms = 0.0, total = 0.0, ms[gpp::StageTimer::kMax];
-            HIP_OR_FAIL(ctx->timer.read(0, &total, ms), "autotune stage times");
+            bool finished;
+            HIP_OR_FAIL(ctx->timer.read(0, ctx->stream, &total, ms, &finished), "autotune stage times");
             const gpp::StageTimer::Slot &t = ctx->timer.last();
             for (int i = 0; i < t.n; ++i) {
                 if (strncmp(t.name[i], "factored_gram", 13) == 0) g_ms = ms[i];
@@ -1012,6 +1030,40 @@ gpp_status gpp_ctx_autotune(gpp_ctx *ctx, gpp_form form)
     return GPP_OK;
 }
 
+}  // extern "C"
+
+namespace {
+
+// The last evaluation's times, after waiting for it alone: on a caller's stream
+// not for the work enqueued behind it (the context's own stream, idle then,
+// brings them), and nowhere for the null stream.
+gpp_status last_times(const gpp_ctx *ctx, double *total, double (&ms)[gpp::StageTimer::kMax])
+{
+    gpp_status st = set_device(ctx);
+    if (st) return st;
+    bool finished = false;
+    if (ctx->stream == ctx->own_stream) {
+        HIP_OR_FAIL(ctx->timer.read(0, ctx->own_stream, total, ms, &finished), "stage times");
+        return GPP_OK;
+    }
+    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+    HIP_OR_FAIL(hipStreamIsCapturing(ctx->stream, &capture), "hipStreamIsCapturing");
+    if (capture != hipStreamCaptureStatusNone)
+        return fail(GPP_ERR_LAUNCH, "the context's stream is being captured: no stage times yet");
+    for (;;) {
+        const hipError_t idle = hipStreamQuery(ctx->stream);
+        if (idle != hipSuccess && idle != hipErrorNotReady) return fail_hip(idle, "stage times");
+        HIP_OR_FAIL(ctx->timer.read(0, ctx->own_stream, total, ms, &finished), "stage times");
+        if (finished) return GPP_OK;
+        if (idle == hipSuccess) return fail(GPP_ERR_LAUNCH, "the last evaluation has not run");
+        usleep(20);
+    }
+}
+
+}  // namespace
+
+extern "C" {
+
 gpp_status gpp_ctx_last_timing(const gpp_ctx *ctx, double *total_ms, double *stage_ms, int max_stages,
                                int *nstages)
 {
@@ -1022,11 +1074,9 @@ gpp_status gpp_ctx_last_timing(const gpp_ctx *ctx, double *total_ms, double *sta
         if (nstages) *nstages = 0;
         return GPP_OK;
     }
-    gpp_status st = set_device(ctx);
-    if (st) return st;
-    HIP_OR_FAIL(hipStreamSynchronize(ctx->stream), "hipStreamSynchronize");
     double total = 0.0, ms[gpp::StageTimer::kMax];
-    HIP_OR_FAIL(ctx->timer.read(0, &total, ms), "stage times");
+    gpp_status st = last_times(ctx, &total, ms);
+    if (st) return st;
     if (total_ms) *total_ms = total;
     for (int i = 0; i < t.n && stage_ms && i < max_stages; ++i) stage_ms[i] = ms[i];
     if (nstages) *nstages = t.n;
@@ -1043,9 +1093,9 @@ gpp_status gpp_ctx_timing_summary(const gpp_ctx *ctx, int last_n, int *nevals, d
     if (avg_total_ms) *avg_total_ms = 0.0;
     if (nstages) *nstages = 0;
     if (!ctx->timed || L.n == 0) return GPP_OK;
-    gpp_status status = set_device(ctx);
+    double last_total = 0.0, last_ms[gpp::StageTimer::kMax];
+    gpp_status status = last_times(ctx, &last_total, last_ms);
     if (status) return status;
-    HIP_OR_FAIL(hipStreamSynchronize(ctx->stream), "hipStreamSynchronize");
     const int want = std::min(last_n, tm.filled);
     double tot = 0.0, st[gpp::StageTimer::kMax] = {};
     int m = 0;
@@ -1055,7 +1105,8 @@ gpp_status gpp_ctx_timing_summary(const gpp_ctx *ctx, int last_n, int *nevals, d
         for (int i = 0; same && i < L.n; ++i) same = S.name[i] && strcmp(S.name[i], L.name[i]) == 0;
         if (!same) break;  // an evaluation of another kind: stop at it
         double total = 0.0, ms[gpp::StageTimer::kMax];
-        HIP_OR_FAIL(tm.read(k, &total, ms), "stage times");
+        bool finished;  // before the last one
+        HIP_OR_FAIL(tm.read(k, ctx->own_stream, &total, ms, &finished), "stage times");
         tot += total;
         for (int i = 0; i < S.n; ++i) st[i] += ms[i];
         ++m;

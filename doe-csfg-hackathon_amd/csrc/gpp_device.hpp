@@ -187,15 +187,25 @@ __device__ __forceinline__ cplx block_sum(cplx v, cplx *scratch)
 }
 
 // Where a launch notes that its stage starts: the device's constant-rate clock,
-// written by the launch's first block.  clear: the later entries of the
-// evaluation to zero (the first stage's launch).  Stages run in stream order,
-// so the start of one is the end of the one before.  Events between the
-// launches took 6-10 us each (five stages: 33 of 65 us of an evaluation of
+// written by the launch's first block.  The first stage's launch also resets the
+// `clear` entries after its own: to zero, the last to `begin` (the count of
+// StampEnd).  Stages run in stream order, so the start of one is the end of the
+// one before.  Events between the launches took 6-10 us each (five stages: 33 of 65 us of an evaluation of
 // empty kernels).
 struct Stamp {
     unsigned long long *at = nullptr;
     int clear = 0;
+    unsigned long long begin = 0;
 };
+// Notes t0 (the launch's first thread).  The stores go past the L2: a host that
+// reads the times of a finished evaluation while the stream goes on copies from
+// memory, where a plain store may not be yet.
+__device__ __forceinline__ void stamp_store(const Stamp &st, unsigned long long t0)
+{
+    __hip_atomic_store(&st.at[0], t0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    for (int i = 1; i <= st.clear; ++i)
+        __hip_atomic_store(&st.at[i], i == st.clear ? st.begin : 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
 // Reads the clock at a kernel's start; store() goes after the kernel's loads.
 // `tie`, a wave-uniform value of the kernel, passes through the reading, which
 // thereby happens before the value's uses.  wall_clock64() counts as a memory
@@ -211,23 +221,28 @@ struct StampStart {
     }
     __device__ __forceinline__ void store() const
     {
-        if (st.at && threadIdx.x == 0 && blockIdx.x == 0 && blockIdx.y == 0 && blockIdx.z == 0) {
-            st.at[0] = t0;
-            for (int i = 1; i <= st.clear; ++i) st.at[i] = 0;
-        }
+        if (st.at && threadIdx.x == 0 && blockIdx.x == 0 && blockIdx.y == 0 && blockIdx.z == 0) stamp_store(st, t0);
     }
 };
 __device__ __forceinline__ void stamp_start(const Stamp &st)
 {
-    if (st.at && threadIdx.x == 0 && blockIdx.x == 0 && blockIdx.y == 0 && blockIdx.z == 0) {
-        st.at[0] = wall_clock64();
-        for (int i = 1; i <= st.clear; ++i) st.at[i] = 0;
-    }
+    if (st.at && threadIdx.x == 0 && blockIdx.x == 0 && blockIdx.y == 0 && blockIdx.z == 0)
+        stamp_store(st, wall_clock64());
 }
-// The end of the evaluation: the latest block of its last launch.
-__device__ __forceinline__ void stamp_end(unsigned long long *at)
+// The end of the evaluation: the latest block of its last launch.  count: on a
+// caller's stream the blocks that have noted theirs are counted, after their
+// times have arrived, so that a host can tell the evaluation's end from that of
+// later work on the stream.
+struct StampEnd {
+    unsigned long long *at = nullptr, *count = nullptr;
+};
+__device__ __forceinline__ void stamp_end(const StampEnd &e)
 {
-    if (at && threadIdx.x == 0) atomicMax(at, wall_clock64());
+    if (!e.at || threadIdx.x != 0) return;
+    atomicMax(e.at, wall_clock64());
+    if (!e.count) return;
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    atomicAdd(e.count, 1ull);
 }
 
 constexpr double kTo1 = 1e-6;    // to1, gppComplex.cpp:20, :241

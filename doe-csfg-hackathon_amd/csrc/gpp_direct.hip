@@ -64,7 +64,7 @@ struct DirectArgs {
     cplx *bg;         // optional gathered rows of aqsm (factored forms), else null
     const int32_t *perm;  // achstemp launch: row r of bg and part_achs is band perm[r] (null: r)
     Stamp stamp;      // the launch's stage start
-    unsigned long long *end;  // the evaluation's end (last launch)
+    StampEnd end;     // the evaluation's end (last launch)
 };
 
 struct WorkLayout {
@@ -136,7 +136,7 @@ DirectArgs make_args(const DevProblem &p, void *work)
     a.band_asx = reinterpret_cast<cplx *>(w + L.band_asx);
     a.bg = nullptr;
     a.perm = nullptr;
-    a.end = nullptr;
+    a.end = StampEnd{};
     return a;
 }
 
@@ -671,7 +671,7 @@ hipError_t launch_reduce(const DirectArgs &a, cplx *out, const CompatOut &co, in
     f.stamp = Stamp{};
     if (pairs > 0) {
         DirectArgs b = a;
-        b.end = nullptr;
+        b.end = StampEnd{};
         hipLaunchKernelGGL(k_reduce_bands, grid_rows((unsigned)((pairs + 3) / 4)), dim3(kReduceThreads), 0, s, b,
                            n1_begin, n1_end);
     }
@@ -699,7 +699,7 @@ hipError_t run_direct(const DevProblem &p, bool strict, void *work, const DevRes
     stage(p.nb == p.nv ? "direct_occupied" : strict ? "direct_unoccupied_strict" : "direct_unoccupied");
     GPP_TRY(launch_direct(a, strict, true, true, true, s));
     stage("direct_reduce");
-    if (timer) a.end = timer->end();
+    if (timer) a.end = timer->end(p.nfreq + 1);
     return launch_reduce(a, res.base, CompatOut{}, 0, p.nb, 1, s);
 }
 

@@ -309,7 +309,7 @@ __global__ __launch_bounds__(kRedThreads, (FC <= 3 && !P2 && !NEG) ? 4 : FC > 8 
 __global__ __launch_bounds__(kRedThreads) void k_fact_final(const cplx *col_ach, const cplx *col_asx,
                                                             const cplx *part_achs, long long ncols, int nfreq, int nb,
                                                             int nv, cplx *out, bool nan_acht, Stamp stamp,
-                                                            unsigned long long *end)
+                                                            StampEnd end)
 {
     stamp_start(stamp);
     __shared__ cplx scratch[kRedThreads / kWave];
@@ -372,7 +372,7 @@ constexpr int kAchtFinalBands = 16;
 __global__ __launch_bounds__(256) void k_acht_final(const cplx *__restrict__ part, int nparts,
                                                     const cplx *__restrict__ part_occ, int nparts_occ, int nb,
                                                     int nv, const int32_t *__restrict__ perm,
-                                                    cplx *__restrict__ out, Stamp stamp, unsigned long long *end)
+                                                    cplx *__restrict__ out, Stamp stamp, StampEnd end)
 {
     stamp_start(stamp);  // where no launch of the stage came before
     __shared__ cplx grp[256 / kAchtFinalBands][kAchtFinalBands];
@@ -633,10 +633,15 @@ hipError_t run_gram_pole(const DevProblem &p, const cplx *bg, cplx *tile_ach, cp
     return hipGetLastError();
 }
 
+unsigned acht_final_blocks(const DevProblem &p)
+{
+    return (p.nb + kAchtFinalBands - 1) / kAchtFinalBands + p.nv;
+}
+
 // Stages 5 and 6: acht_n1_loc of the problem's bands, row n1 to
 // out[perm ? perm[n1] : n1].  st: for the first launch.
 hipError_t run_acht(const DevProblem &p, const AchtSplit &as, int occ_chunk, int occ_nsplit, const AchtBufs &ab,
-                    const cplx *bg, const int32_t *perm, cplx *out, Stamp st, unsigned long long *end, hipStream_t s)
+                    const cplx *bg, const int32_t *perm, cplx *out, Stamp st, StampEnd end, hipStream_t s)
 {
     if (p.nb > p.nv) {
         if (as.narrow)
@@ -654,7 +659,7 @@ hipError_t run_acht(const DevProblem &p, const AchtSplit &as, int occ_chunk, int
         GPP_TRY(hipGetLastError());
         st = Stamp{};
     }
-    hipLaunchKernelGGL(k_acht_final, dim3((p.nb + kAchtFinalBands - 1) / kAchtFinalBands + p.nv), dim3(256), 0, s,
+    hipLaunchKernelGGL(k_acht_final, dim3(acht_final_blocks(p)), dim3(256), 0, s,
                        ab.part, as.jtiles * as.nks, ab.part_occ, p.ngpown * occ_nsplit, p.nb, p.nv, perm, out, st, end);
     return hipGetLastError();
 }
@@ -674,7 +679,7 @@ hipError_t run_factored(const DevProblem &p, GramKind kind, void *work, const De
     cplx *part_achs = reinterpret_cast<cplx *>(w + L.part_achs);
 
     const auto stage = [&](const char *nm) { return timer ? timer->stage(nm) : Stamp{}; };
-    const auto end = [&]() { return timer ? timer->end() : nullptr; };
+    const auto end = [&](unsigned blocks) { return timer ? timer->end(blocks) : StampEnd{}; };
     if (timer) timer->begin();
     // also gathers Bg
     GPP_TRY(launch_achstemp(p, part_achs, bg, stage("factored_gather_achstemp"), s));
@@ -684,7 +689,7 @@ hipError_t run_factored(const DevProblem &p, GramKind kind, void *work, const De
         GPP_TRY(run_gram_pole(p, bg, col_ach, col_asx, L.nsplit, c2a, c2x, stage("factored_gram_pole"), timer, s));
         const Stamp st = stage("factored_final");
         hipLaunchKernelGGL(k_fact_final, dim3(p.nfreq + 1), dim3(kRedThreads), 0, s, c2a, c2x, part_achs, p.ngpown,
-                           p.nfreq, p.nb, p.nv, res.base, true, st, end());
+                           p.nfreq, p.nb, p.nv, res.base, true, st, end(p.nfreq + 1));
         return hipGetLastError();
     }
     if (kind.ozaki_slices) {
@@ -704,11 +709,12 @@ hipError_t run_factored(const DevProblem &p, GramKind kind, void *work, const De
     const Stamp st_final = stage("factored_final");
     hipLaunchKernelGGL(k_fact_final, dim3(p.nfreq + 1), dim3(kRedThreads), 0, s, col_ach, col_asx, part_achs,
                        p.ngpown * L.nsplit, p.nfreq, p.nb, p.nv, res.base, true, st_final,
-                       kind.acht ? nullptr : end());
+                       kind.acht ? StampEnd{} : end(p.nfreq + 1));
     GPP_TRY(hipGetLastError());
     if (!kind.acht) return hipSuccess;
     const Stamp st = stage("factored_acht");
-    return run_acht(p, L.as, L.occ_chunk, L.occ_nsplit, ab, bg, nullptr, res.acht_n1_loc(), st, end(), s);
+    return run_acht(p, L.as, L.occ_chunk, L.occ_nsplit, ab, bg, nullptr, res.acht_n1_loc(), st,
+                    end(acht_final_blocks(p)), s);
 }
 
 // ---------------------------------------------------------------------------
@@ -1012,7 +1018,7 @@ hipError_t run_factored_bucketed(const DevProblem &p, GramKind kind, const Bucke
                 const int chunk = acht_occ_chunk(q, kind.red_chunk);
                 const int nsplit = reduce_sums_acht_occ(q.nv, q.wx_neg) ? L.nsplit : (p.ncouls + chunk - 1) / chunk;
                 GPP_TRY(run_acht(q, acht_split(q), chunk, nsplit, ab, bgq, bp.dev_perm() + bp.start[b],
-                                 res.acht_n1_loc(), Stamp{}, nullptr, s));
+                                 res.acht_n1_loc(), Stamp{}, StampEnd{}, s));
             }
         }
         if (bare0 < s1) {
@@ -1033,7 +1039,7 @@ hipError_t run_factored_bucketed(const DevProblem &p, GramKind kind, const Bucke
     st = stage("bucket_combine");
     hipLaunchKernelGGL(k_fact_final, dim3(p.nfreq + 1), dim3(kRedThreads), 0, s, at(L.col_ach), at(L.col_asx),
                        part_achs, L.ncols, p.nfreq, p.nb, p.nv, res.base, !kind.acht, st,
-                       timer ? timer->end() : nullptr);
+                       timer ? timer->end(p.nfreq + 1) : StampEnd{});
     return hipGetLastError();
 }
 

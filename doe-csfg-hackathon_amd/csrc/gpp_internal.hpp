@@ -59,22 +59,29 @@ struct StageTimer {
     struct Slot {
         const char *name[kMax] = {};
         int n = 0;  // stages recorded
+        unsigned long long begin = 0, end = 0;  // the count before and after the last launch's blocks (0, 0: not counted)
     };
     Slot slot[kRing];
     int cur = 0;     // slot of the current (last) evaluation
     int filled = 0;  // evaluations recorded, at most kRing
-    unsigned long long *dev = nullptr;  // [kRing][kMax + 1]: stage starts, then the end
-    int khz = 100000;                   // rate of the device clock
-    hipError_t init(int device);
+    unsigned long long *dev = nullptr;  // [kRing][kRow]: stage starts, then the end; last the count of StampEnd
+    static constexpr int kRow = kMax + 2;
+    int khz = 100000;      // rate of the device clock
+    bool counted = false;  // the evaluation runs on a caller's stream: count its last launch's blocks
+    // Each counted evaluation counts from a number of its own, so that the count
+    // of an earlier one in its row is not taken for it.
+    unsigned long long evaluations = 0;
+    hipError_t init(int device, hipStream_t s);
     void destroy();
     void begin();                 // starts a slot
     Stamp stage(const char *nm);  // for the first launch of the next stage
-    unsigned long long *end() { return dev ? dev + cur * (kMax + 1) + slot[cur].n : nullptr; }  // for the last launch
+    StampEnd end(unsigned blocks);  // for the last launch, of that many blocks
     const Slot &last() const { return slot[cur]; }
     const Slot &back(int k) const { return slot[(cur - k + kRing) % kRing]; }  // k evaluations before the last
-    // Milliseconds of the evaluation k before the last, total and per stage
-    // (the stream must be idle).
-    hipError_t read(int k, double *total, double (&stage_ms)[kMax]) const;
+    // The evaluation k before the last, copied on stream `via`: milliseconds,
+    // total and per stage, and whether it has finished (said of every one whose
+    // blocks were not counted: its stream must be idle then).
+    hipError_t read(int k, hipStream_t via, double *total, double (&stage_ms)[kMax], bool *finished) const;
 };
 
 // 1 if some of the n frequencies is negative (NaN counts as negative, so an

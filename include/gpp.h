@@ -384,10 +384,11 @@ gpp_status gpp_ctx_get_option(const gpp_ctx *ctx, gpp_option option, int *value)
 
 /*
  * GPU time of the last gpp_sigma in milliseconds, from the device clock as the
- * stages' own launches note it (10 ns steps; waits for the context's enqueued
- * work): total, and per stage (stage_ms[i] for i <
- * *nstages, at most max_stages written; stage names via
- * gpp_ctx_stage_name).  Any pointer may be NULL.
+ * stages' own launches note it (10 ns steps): total, and per stage
+ * (stage_ms[i] for i < *nstages, at most max_stages written; stage names via
+ * gpp_ctx_stage_name).  Waits for that evaluation, on a caller's stream
+ * (gpp_ctx_set_stream) not for the work behind it; fails while that stream is
+ * being captured.  Any pointer may be NULL.
  */
 gpp_status gpp_ctx_last_timing(const gpp_ctx *ctx, double *total_ms, double *stage_ms,
                                int max_stages, int *nstages);
