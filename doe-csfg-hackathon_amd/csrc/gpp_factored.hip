@@ -1044,3 +1044,34 @@ hipError_t run_factored_bucketed(const DevProblem &p, GramKind kind, const Bucke
 }
 
 }  // namespace gpp
+
+// Not part of the interface: which kernels the size rules pick, for the tests
+// that run those kernels at their edges.
+extern "C" {
+
+static gpp::DevProblem sizes_only(int nb, int nv, int ncouls, int ngpown)
+{
+    gpp::DevProblem p;
+    p.nb = nb; p.nv = nv; p.ncouls = ncouls; p.ngpown = ngpown; p.nfreq = 3;
+    return p;
+}
+
+// The FP64 Gram tile of GPP_OPT_GRAM_TILE 0 for one product, or for `groups` of
+// them over `bands` unoccupied bands in all: 1000 x G' columns + G-vectors.
+int gpp_test_gram_tile(int nb, int nv, int ncouls, int ngpown, int groups, int bands)
+{
+    static const int tiles[] = {64128, 128064, 64064, 32064, 16016};  // of GramTile
+    static const int32_t some = 0;
+    gpp::GramSlots g;
+    if (groups > 0) g = gpp::GramSlots{&some, groups, bands};
+    return tiles[gpp::gram_tile_for(sizes_only(nb, nv, ncouls, ngpown), g)];
+}
+
+// The acht_n1_loc product: its tile likewise, 1000000 more with a short last one.
+int gpp_test_acht_tile(int nb, int nv, int ncouls, int ngpown)
+{
+    const gpp::AchtSplit as = gpp::acht_split(sizes_only(nb, nv, ncouls, ngpown));
+    return (as.cut ? 1000000 : 0) + (as.narrow ? 64064 : 64128);
+}
+
+}
