@@ -1427,7 +1427,7 @@ gpp_status gpp_batch_autotune(gpp_batch *b, gpp_form form)
     };
     gpp::GramKind k = kind, best_k = kind;
     double best = 1e300, ms = 0;
-    for (int tile = 0; tile < (kind.ozaki_slices ? 0 : gpp::kGramTiles); ++tile) {  // FP64 Gram tiles only
+    for (int tile = 1; tile < (kind.ozaki_slices ? 0 : gpp::kGramTiles); ++tile) {  // FP64 only; tile 0 runs as tile 1
         k.tile = tile;
         if ((st = timed(k, 2, &ms))) return st;
         if (ms < best) best = ms, best_k.tile = tile;

@@ -283,15 +283,16 @@ __global__ __launch_bounds__(256) void k_pole_cols(const cplx *col_ach, const cp
 
 // Grid (ngpown, nsplit, ceil(nfreq/FC)).  NV: occupied band count fixed at
 // compile time (0: any).  Three waves per SIMD: with the wave-uniform pole
-// inputs held in scalar registers the FC = 8 variants fit 168 VGPRs (the
-// 8-occupied-band one spills 10), and at 16 frequencies x 8 occupied bands
-// three waves run the reduce 12% faster than two.  Two for FC = 16 (its 64
-// accumulators; the plain variants fit 208-241 VGPRs).  Four for the plain
-// kernels of at most three frequencies: their waves wait on memory half of
-// the time, and a fourth hides more of it despite 17 spilled registers
-// (3 frequencies x 2 occupied bands: 0.510 -> 0.486 ms at 512/2/32768/1638);
-// the p2-storing and negative-frequency variants spill 30-72 and keep three
-// (the p2 one at four: 0.70 -> 1.28 ms at 512/2/32768/1638).
+// inputs held in scalar registers the FC = 8 kernels fit 168 VGPRs (142-165;
+// the p2-storing ones 154-168, of which at most 8 spill).  Two waves are slower
+// or no faster (reduce, us, three / two, 40/nv/16384/819 and 8 frequencies: 2
+// bands 198 / 204, 8 bands 234 / 237, with p2 6 bands 249 / 284).  Two for FC =
+// 16 (its 64 accumulators; 207-239 VGPRs).  Four for the plain kernels of at
+// most three frequencies: their waves wait on memory half of the time, and a
+// fourth hides more of it despite 8-21 spilled registers at three frequencies
+// (40/nv/16384/819, four / three: 1 band 121 / 130, 2 bands 126 / 138, from 3
+// bands up within 2%); the p2-storing and negative-frequency ones take up to
+// 159 and keep three (the p2 one at four: 0.70 -> 1.28 ms at 512/2/32768/1638).
 // The negative-frequency kernels of 8 frequencies per pass run two (their
 // cutoff code spilled 84-186 registers at three).
 template <int FC, int NV, bool P2, bool NEG = false>
@@ -449,14 +450,9 @@ void launch_reduce_p2(const ReduceArgs &a, dim3 grid, hipStream_t s)
     // together, conj(bg) in scalar registers), beyond it the general one.
     // Reduce, us, general / own: 300/nv/16384/819, nv = 3 and 3 frequencies 184
     // / 137, 7 and 3 233 / 177, 1 and 8 229 / 187, 5 and 13 562 / 376, 6 and 24
-    // 917 / 604; the p2-storing one of one band and at most 3 frequencies the
-    // other way, 186 / 194.
-    if constexpr (P2 && FC <= 3) {
-        if (a.nv == 1) {
-            hipLaunchKernelGGL((k_pole_reduce<FC, 0, P2>), grid, dim3(kRedThreads), 0, s, a);
-            return;
-        }
-    }
+    // 917 / 604; with p2 40/nv/16384/819, 1 and 8 267 / 220, 3 and 4 256 / 200,
+    // 5 and 16 666 / 489, 7 and 8 458 / 254; the p2-storing one of one band and
+    // at most 3 frequencies the other way, 186 / 194.
     switch (a.nv) {
     case 1: hipLaunchKernelGGL((k_pole_reduce<FC, (P2 && FC <= 3) ? 0 : 1, P2>), grid, dim3(kRedThreads), 0, s, a); break;
     case 2: hipLaunchKernelGGL((k_pole_reduce<FC, 2, P2>), grid, dim3(kRedThreads), 0, s, a); break;

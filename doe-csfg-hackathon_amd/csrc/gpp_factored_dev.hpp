@@ -20,7 +20,7 @@ namespace fact {
 
 typedef double v4d __attribute__((ext_vector_type(4)));
 
-constexpr int kWJ = 64, kWI = 32;  // wave tile of the fused Gram and the acht product: 64 rows x 32 columns
+constexpr int kWJ = 64, kWI = 32;  // wave tile of the fused Gram: 64 columns x 32 G-vectors
 constexpr int kRedThreads = 256;   // pole-reduce and final-reduce blocks
 
 // s_waitcnt vmcnt(N) lgkmcnt(0) (N < 64): at most N of the wave's loads from
@@ -1030,7 +1030,7 @@ template <int F> struct FuseLds {
 };
 
 // Epilogue of one 128 x 128 tile (G-vector tile `itile`) after
-// gram_f64_acc<TRANS>: the accumulators are folded into Mu at once (128
+// gram_f64_acc: the accumulators are folded into Mu at once (128
 // registers instead of 192), and the elements are evaluated in eight rounds
 // (s, t): 32 columns (sub-tile s of both 64-column halves) x 64 G-vectors
 // (sub-tile t of the four 32-G-vector quarters).  In a round all 512 threads
@@ -1433,7 +1433,7 @@ template <int F> __device__ __forceinline__ void pole_reduce_bare(const BareArgs
         double wti2[kBareE];
         size_t at[kBareE];
 #pragma unroll
-        for (int e = 0; e < kBareE; ++e) {  // elements past the end repeat the last one, with q = 0
+        for (int e = 0; e < kBareE; ++e) {  // elements past the end load the last one again and add nothing
             at[e] = row + min(ig0 + e * kRedThreads, ig_end - 1);
             wt[e] = a.wtilde[at[e]];
             q[e] = a.ieps[at[e]];

@@ -170,11 +170,10 @@ struct BucketPlan {
     std::vector<int> start, size, nocc, row;
     std::vector<int> neg;   // per bucket: its row has a negative frequency
     bool identity = false;  // perm leaves every band in place
-    // Buckets in the order they are worked on: the nslot_occ ones with
-    // occupied bands, then the others, each most unoccupied bands first (the
-    // longest Gram tiles start first).
+    // Buckets in the order they are worked on: those with occupied bands, then
+    // the others, each most unoccupied bands first (the longest Gram tiles
+    // start first).
     std::vector<int> slot;
-    int nslot_occ = 0;
     // Device copy of tables(): perm, then per slot (first, end) of its
     // unoccupied rows in permuted order and its frequency row.  The owner of
     // the plan uploads it.
