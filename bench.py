@@ -402,9 +402,10 @@ def main():
     def direct_roofline(form):
         kname = "direct_unoccupied_strict" if form == "direct-strict" else "direct_unoccupied"
         kms = forms[form]["gpu_stage_ms"][kname]
-        flop = (NB - NV) * NGPOWN * NCOULS * NFREQ * FLOP_UNOCC
+        # the stage's one launch (k_direct) evaluates the occupied bands and achstemp too
+        flop = NGPOWN * NCOULS * NFREQ * ((NB - NV) * FLOP_UNOCC + NV * FLOP_OCC)
         achieved = flop / (kms * 1e-3) / 1e12
-        tr = load_traffic("k_unocc") if (form == "direct" and args.workload == "c1") else None
+        tr = load_traffic("k_direct") if (form == "direct" and args.workload == "c1") else None
         return {"bound": "valu", "pipe": "FP64 VALU (FP64 vector peak = FP64 matrix peak on MI355X)",
                 "kernel": kname, "achieved": achieved, "peak": PEAK_FP64_TFLOPS, "unit": "TFLOP/s",
                 "frac": achieved / PEAK_FP64_TFLOPS,
