@@ -259,7 +259,7 @@ __device__ __forceinline__ void unocc_block(const DirectArgs &a, int ncouls, uns
     int c0, c1;
     range_chunks(a, ncouls, g, c0, c1);
     // the fast form loads aqsn of the next chunk while this one is evaluated
-    // (171 -> 161 us at 512/2/1600/80; the strict form has no registers for it)
+    // (the strict form has no registers for it)
     cplx an_next = czero();
     if (!STRICT) an_next = load_an(c0);
     load_chunk(c0);
@@ -268,6 +268,10 @@ __device__ __forceinline__ void unocc_block(const DirectArgs &a, int ncouls, uns
     for (int c = c0; c < c1; ++c) {
         const int buf = (c - c0) & 1;
         cplx an = an_next;
+        // taken before the next loads are issued: the compiler else put the wait
+        // for it after them, which waited for them too (us, with / without:
+        // 512/2/16384/819/3 12940 / 12090, 1536/8/65536/1638/4 405500 / 381700)
+        if (!STRICT) asm volatile("" : "+v"(an.re), "+v"(an.im));
         if (c + 1 < c1) {
             load_chunk(c + 1);
             if (!STRICT) an_next = load_an(c + 1);
