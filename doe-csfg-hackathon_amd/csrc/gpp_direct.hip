@@ -445,7 +445,10 @@ __device__ __forceinline__ unsigned block_of_rows() { return blockIdx.y * gridDi
 // bands'.  Each kind's frequency passes one after the other, not by turns: the
 // dispatcher deals blocks round robin to eight XCDs, and two passes of unequal
 // width by turns gave four of them all the wide ones (us, 200/3/3000/150: five
-// frequencies 511 by turns, 409 so).
+// frequencies 511 by turns, 409 so).  Passes of equal width take turns by column
+// tile, where all bands' blocks run one pass after the other and the tile's rows
+// and aqsn are still in the caches (ms, one after the other / by tile:
+// 512/2/8192/819/32 58.1 / 57.1, 1536/8/65536/3276/16 3065 / 3049).
 // A kernel for each pair of widths (W, the last pass R; 0: W): one with every
 // width took 4 registers more than it has, the strict one 29, and ran the
 // strict form in passes of three (us, 512/2/16384/819 strict 4 frequencies
@@ -470,8 +473,14 @@ __global__ __launch_bounds__(kNW *kWave) __attribute__((amdgpu_waves_per_eu(4)))
             if (threadIdx.x % kWave == 0) a.part_achs[item] = s;
         }
     } else {
-        const unsigned before = a.occ_blocks + a.ach_blocks, u = b - before, pass = (a.blocks - before) / (unsigned)a.nz;
-        direct_pass<W, R, STRICT, false>(a, ncouls, u % pass, u / pass, lds);
+        const unsigned before = a.occ_blocks + a.ach_blocks, u = b - before, nz = a.nz;
+        if constexpr (R == 0) {
+            const unsigned ngroups = (a.nb - a.nv + kNW - 1) / kNW, q = u / ngroups;
+            direct_pass<W, R, STRICT, false>(a, ncouls, q / nz * ngroups + u % ngroups, q % nz, lds);
+        } else {
+            const unsigned pass = (a.blocks - before) / nz;
+            direct_pass<W, R, STRICT, false>(a, ncouls, u % pass, u / pass, lds);
+        }
     }
     stamp.store();
 }
