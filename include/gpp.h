@@ -152,8 +152,8 @@ typedef enum {
      * requested: 1 = evaluate the pole factors in the epilogue of the Gram
      * product, so the G'xG product Mu (ngpown * ncouls * 16 bytes of
      * workspace) is never stored -- for problems whose Mu does not fit in
-     * device memory; slower where it fits (512/2/32768/1638: 3.58 against
-     * 3.19 ms); 0 = store Mu and run the pole reduce as its own stage
+     * device memory; slower where it fits (512/2/32768/1638: 3.57 against
+     * 3.00 ms); 0 = store Mu and run the pole reduce as its own stage
      * (default). */
     GPP_OPT_FUSED_REDUCE = 9
 } gpp_option;
