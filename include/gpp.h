@@ -270,7 +270,8 @@ gpp_status gpp_sigma(gpp_ctx *ctx, gpp_form form, const gpp_outputs *out);
  * bands by identical rows and factor each group (one group: exactly the
  * plain factored form on that row); with more than GPP_OPT_MAX_BUCKETS
  * groups they run GPP_FORM_DIRECT instead (gpp_ctx_last_form tells which).
- * The batched entry points take one wx_array per instance.
+ * The batched entry points take one wx_array per instance.  After a device
+ * error (no memory, a failed copy) the shared wx_array is in effect.
  */
 gpp_status gpp_set_band_frequencies(gpp_ctx *ctx, const double *wx_bands);
 
